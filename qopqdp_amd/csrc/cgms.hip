@@ -17,31 +17,59 @@ __device__ __forceinline__ double wsum(double v) {
   return v;
 }
 
-// Sum m partials in the same fixed order as finalize_kernel (256 threads).
-__device__ double block_sum256(const double *p, int m, double *sh) {
-  double s = 0;
-  for (int i = threadIdx.x; i < m; i += 256) s += p[i];
-  s = wsum(s);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+// Fixed-order sums of m partials of one or two arrays by one 1024-thread
+// block: four independent accumulators per thread and array keep the loads in
+// flight (with 256 threads and one accumulator the sums of 2 x 5184 partials
+// took 12.8 us, all of it load latency).
+constexpr int SUM_THREADS = 1024;
+template <int N>
+__device__ __forceinline__ void block_sums(const double *const (&p)[N], int m, double *sh, double (&out)[N]) {
+  double s[N][4];
+#pragma unroll
+  for (int k = 0; k < N; k++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) s[k][j] = 0;
+  int i = threadIdx.x;
+  for (; i + 3 * SUM_THREADS < m; i += 4 * SUM_THREADS)
+#pragma unroll
+    for (int k = 0; k < N; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) s[k][j] += p[k][i + j * SUM_THREADS];
+  for (; i < m; i += SUM_THREADS)
+#pragma unroll
+    for (int k = 0; k < N; k++) s[k][0] += p[k][i];
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const double t = wsum((s[k][0] + s[k][1]) + (s[k][2] + s[k][3]));
+    if ((threadIdx.x & 63) == 0) sh[k * (SUM_THREADS / 64) + (threadIdx.x >> 6)] = t;
+  }
   __syncthreads();
-  double r = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-  __syncthreads();
-  return r;
+#pragma unroll
+  for (int k = 0; k < N; k++) {  // only the first wave's result is used
+    const double t = threadIdx.x < SUM_THREADS / 64 ? sh[k * (SUM_THREADS / 64) + threadIdx.x] : 0.0;
+    out[k] = wsum(t);
+  }
 }
 
 // After linop: pkp, b[imin] and the zeta/beta recurrences (:203-238).
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(SUM_THREADS)
 cgms_scalarA(CgmsDev d, int nch) {
-  __shared__ double sh[4];
+  __shared__ double sh[2 * SUM_THREADS / 64];
   CgmsState *s = d.st;
-  if (s->status != 0) return;
-  double Ain2 = block_sum256(d.partA, nch, sh);
-  double in2 = block_sum256(d.partB, nch, sh);
+  if (s->status != 0) {
+    if (threadIdx.x == 0) s->xpend = 0;  // the x update of the stopping iteration is done
+    return;
+  }
+  const double *const parts[2] = {d.partA, d.partB};
+  double sums[2];
+  block_sums<2>(parts, nch, sh, sums);
   if (threadIdx.x != 0) return;
   s->oldrsq = s->rsq;
-  double pkp = Ain2 + s->m2 * in2;  // ddagd_norm2 return value
+  double pkp = sums[0] + s->m2 * sums[1];  // ddagd_norm2 return value
   s->pkp = pkp;
   s->iteration++;
+  s->total++;
+  s->xpend = 0;
   if (pkp <= 0) { s->status = 2; s->break_reason = 1; return; }
   const int imin = s->imin, ns = s->ns;
   s->b[imin] = s->rsq / pkp;
@@ -56,46 +84,6 @@ cgms_scalarA(CgmsDev d, int nch) {
     else { zn = 0; s->b[i] = 0; }
     s->zn[i] = zn;
   }
-}
-
-// r -= b[imin] Mp ; x_i += b_i p_i ; partial |r|^2   (:209-252)
-template <int P>
-__global__ void __launch_bounds__(256)
-cgms_update(CgmsDev d, int Vh, VecView r, VecView Mp, int ns) {
-  using R = typename QT<P>::R;
-  using S = typename QT<P>::S;
-  const CgmsState *s = d.st;
-  if (s->status != 0) return;
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = 0;
-  if (h < Vh) {
-    const R b0 = (R)s->b[s->imin];
-    S *rr = (S *)r.data;
-    const S *mp = (const S *)Mp.data;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      S a = rr[c * Vh + h], m = mp[c * Vh + h];
-      a.x = fma(-b0, m.x, a.x);
-      a.y = fma(-b0, m.y, a.y);
-      rr[c * Vh + h] = a;
-      acc += (double)a.x * a.x + (double)a.y * a.y;
-    }
-    for (int i = 0; i < ns; i++) {
-      const R bi = (R)s->b[i];
-      S *x = (S *)d.xs[i].data;
-      const S *pm = (const S *)d.pms[i].data;
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        S xv = x[c * Vh + h], pv = pm[c * Vh + h];
-        xv.x = fma(bi, pv.x, xv.x);
-        xv.y = fma(bi, pv.y, xv.y);
-        x[c * Vh + h] = xv;
-      }
-    }
-  }
-  const int nch = (Vh + 63) / 64;
-  acc = wsum(acc);
-  if ((threadIdx.x & 63) == 0 && (h >> 6) < nch) d.partC[h >> 6] = acc;
 }
 
 // Relative-residual reduction (only when relmin > 0): r vs out[irel].
@@ -124,16 +112,38 @@ cgms_relnorm(CgmsDev d, int Vh, VecView r, VecView x) {
 // After the update: rsq, stopping tests, then alpha and the shift-over of
 // zeta/beta (:254-275, 349-376).  Sets status 1 when the host must fold the
 // solution and check the true residual.
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(SUM_THREADS)
 cgms_scalarB(CgmsDev d, int nch, int with_rel, int Vh) {
-  __shared__ double sh[4];
+  __shared__ double sh[2 * SUM_THREADS / 64];
   CgmsState *s = d.st;
   if (s->status != 0) return;
-  double rsq = block_sum256(d.partC, nch, sh);
-  double rel = with_rel ? block_sum256(d.partD, nch, sh) : 0.0;
+  double rsq, rel = 0;
+  if (with_rel) {
+    const double *const parts[2] = {d.partC, d.partD};
+    double sums[2];
+    block_sums<2>(parts, nch, sh, sums);
+    rsq = sums[0];
+    rel = sums[1];
+  } else {
+    const double *const parts[1] = {d.partC};
+    double sums[1];
+    block_sums<1>(parts, nch, sh, sums);
+    rsq = sums[0];
+  }
   if (threadIdx.x != 0) return;
   s->rsq = rsq;
   const int it = s->iteration;
+  s->xpend = with_rel ? 0 : 1;  // read only once the status is raised
+  if (s->cg) {  // the restart / stopping test at the top of lib/invert_cg_p.c's loop
+    if (with_rel) s->relnorm2 = rel / (double)Vh;
+    if (it >= s->restart || s->total >= s->max_iter || rsq < s->rsqstop ||
+        (with_rel && s->relnorm2 < s->relstop)) {
+      s->status = 1;
+      return;
+    }
+    s->a[0] = rsq / s->oldrsq;
+    return;
+  }
   double rsqc = s->zn[s->irsq] * s->zn[s->irsq] * rsq;
   if (with_rel) s->relnorm2 = s->zn[s->irel] * s->zn[s->irel] * (rel / (double)Vh);
   if (it >= s->restart || it >= s->max_iter) { s->status = 2; s->break_reason = 2; return; }
@@ -154,49 +164,73 @@ cgms_scalarB(CgmsDev d, int nch, int with_rel, int Vh) {
   for (int i = 0; i < ns; i++) { s->bo[i] = s->b[i]; s->zo[i] = s->z[i]; s->z[i] = s->zn[i]; }
 }
 
-// p = r + a[imin] p ; p_i = zn_i r + a_i p_i   (:349-376); pms[imin] is p
+// The solution and search directions of all shifts in one pass
+// (:209-252, 349-376): x_i += b_i p_i with the directions of this iteration,
+// then p_i = zn_i r + a_i p_i (the base: p = r + a p) and the partials of the
+// base |p|^2 for the next iteration's <p, A p>.  pms[imin] is p.
+// Streaming, 4 vectors per shift (x and p read and written) + r: with x and p
+// updated in separate passes it was 5, and A p was stored and read back
+// besides.  In the iteration that raises the status only x is updated; after a
+// host check only p (what = CGMS_P).  FP32 vectors: sums formed in FP64 and
+// rounded once.
 template <int P>
 __global__ void __launch_bounds__(256)
-cgms_pupdate(CgmsDev d, int Vh, VecView r, int ns) {
+cgms_xp(CgmsDev d, int Vh, VecView r, int ns, int what) {
   using R = typename QT<P>::R;
   using S = typename QT<P>::S;
   const CgmsState *s = d.st;
-  if (s->status != 0) return;
+  if (s->status != 0) {
+    if (what != CGMS_XP || !s->xpend) return;
+    what = CGMS_X;
+  }
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= Vh) return;
-  S rv[3];
-  const S *rr = (const S *)r.data;
+  double acc = 0;
+  if (h < Vh) {
+    S rv[3];
+    if (what & CGMS_P) {
+      const S *rr = (const S *)r.data;
 #pragma unroll
-  for (int c = 0; c < 3; c++) rv[c] = rr[c * Vh + h];
-  for (int i = 0; i < ns; i++) {
-    const bool base = i == s->imin;
-    const R ai = (R)s->a[i], zi = (R)s->zn[i];
-    S *pm = (S *)d.pms[i].data;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      S pv = pm[c * Vh + h];
-      if (base) {
-        pv.x = fma(ai, pv.x, rv[c].x);
-        pv.y = fma(ai, pv.y, rv[c].y);
-      } else {
-        R tx = zi * rv[c].x, ty = zi * rv[c].y;
-        pv.x = fma(ai, pv.x, tx);
-        pv.y = fma(ai, pv.y, ty);
-      }
-      pm[c * Vh + h] = pv;
+      for (int c = 0; c < 3; c++) rv[c] = rr[c * Vh + h];
     }
+    for (int i = 0; i < ns; i++) {
+      const bool base = i == s->imin;
+      const double ai = s->a[i], zi = s->zn[i], bi = s->b[i];
+      S *pm = (S *)d.pms[i].data;
+      S *x = (S *)d.xs[i].data;
+      S pv[3];
+#pragma unroll
+      for (int c = 0; c < 3; c++) pv[c] = pm[c * Vh + h];
+      if (what & CGMS_X) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          S xv = x[c * Vh + h];
+          xv.x = (R)fma(bi, (double)pv[c].x, (double)xv.x);
+          xv.y = (R)fma(bi, (double)pv[c].y, (double)xv.y);
+          x[c * Vh + h] = xv;
+        }
+      }
+      if (what & CGMS_P) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          const double tx = base ? (double)rv[c].x : zi * (double)rv[c].x;
+          const double ty = base ? (double)rv[c].y : zi * (double)rv[c].y;
+          pv[c].x = (R)fma(ai, (double)pv[c].x, tx);
+          pv[c].y = (R)fma(ai, (double)pv[c].y, ty);
+          pm[c * Vh + h] = pv[c];
+          if (base) acc += (double)pv[c].x * pv[c].x + (double)pv[c].y * pv[c].y;
+        }
+      }
+    }
+  }
+  if (what & CGMS_P) {
+    const int nch = (Vh + 63) / 64;
+    acc = wsum(acc);
+    if ((threadIdx.x & 63) == 0 && (h >> 6) < nch) d.partB[h >> 6] = acc;
   }
 }
 
 void cgms_launch_scalarA(CgmsDev d, int nch, hipStream_t st) {
-  hipLaunchKernelGGL(cgms_scalarA, dim3(1), dim3(256), 0, st, d, nch);
-  QOP_CHECK_HIP(hipGetLastError());
-}
-void cgms_launch_update(CgmsDev d, int prec, int Vh, VecView r, VecView Mp, int ns,
-                        hipStream_t st) {
-  dim3 g((Vh + 255) / 256), b(256);
-  if (prec == P64) hipLaunchKernelGGL(cgms_update<P64>, g, b, 0, st, d, Vh, r, Mp, ns);
-  else hipLaunchKernelGGL(cgms_update<P32>, g, b, 0, st, d, Vh, r, Mp, ns);
+  hipLaunchKernelGGL(cgms_scalarA, dim3(1), dim3(SUM_THREADS), 0, st, d, nch);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void cgms_launch_relnorm(CgmsDev d, int prec, int Vh, VecView r, VecView x,
@@ -207,15 +241,13 @@ void cgms_launch_relnorm(CgmsDev d, int prec, int Vh, VecView r, VecView x,
   QOP_CHECK_HIP(hipGetLastError());
 }
 void cgms_launch_scalarB(CgmsDev d, int nch, int with_rel, int Vh, hipStream_t st) {
-  hipLaunchKernelGGL(cgms_scalarB, dim3(1), dim3(256), 0, st, d, nch, with_rel, Vh);
+  hipLaunchKernelGGL(cgms_scalarB, dim3(1), dim3(SUM_THREADS), 0, st, d, nch, with_rel, Vh);
   QOP_CHECK_HIP(hipGetLastError());
 }
-void cgms_launch_pupdate(CgmsDev d, int prec, int Vh, VecView p, VecView r, int ns,
-                         hipStream_t st) {
-  (void)p;
+void cgms_launch_xp(CgmsDev d, int prec, int Vh, VecView r, int ns, int what, hipStream_t st) {
   dim3 g((Vh + 255) / 256), b(256);
-  if (prec == P64) hipLaunchKernelGGL(cgms_pupdate<P64>, g, b, 0, st, d, Vh, r, ns);
-  else hipLaunchKernelGGL(cgms_pupdate<P32>, g, b, 0, st, d, Vh, r, ns);
+  if (prec == P64) hipLaunchKernelGGL(cgms_xp<P64>, g, b, 0, st, d, Vh, r, ns, what);
+  else hipLaunchKernelGGL(cgms_xp<P32>, g, b, 0, st, d, Vh, r, ns, what);
   QOP_CHECK_HIP(hipGetLastError());
 }
 

@@ -7,7 +7,9 @@ namespace qop {
 // Hop reductions per RHS (FP64): RED_OUT2 = |out|^2, RED_X2 = |x|^2.
 // RED_CG: fused CG update in the epilogue (dst = r is updated in place with
 // r -= alpha (beta x + alpha_hop hop), xs += alpha x, reduction |r|^2).
-enum { RED_NONE = 0, RED_OUT2 = 1, RED_X2 = 2, RED_CG = 3 };
+// RED_R: RED_CG without the solution update (FP64 and FP32 vectors, one RHS
+// per thread): the second hop of the reference solvers' iteration.
+enum { RED_NONE = 0, RED_OUT2 = 1, RED_X2 = 2, RED_CG = 3, RED_R = 4 };
 int hop_partial_blocks(const Lattice *lat);
 
 // Hop: dst[b] = alpha_b * sum_k W_k src[b](x+d_k) + beta_b * x[b], for the
@@ -43,7 +45,7 @@ struct HopArgs {
   int single = 0;
   const void *links_bck = nullptr;
   VecView xs{};                  // RED_CG: FP32 solution increments (stride dstride)
-  const double *cg_alpha = nullptr;  // RED_CG: alpha of slot b at cg_alpha[b*cg_stride]
+  const double *cg_alpha = nullptr;  // RED_CG / RED_R: alpha of slot b at cg_alpha[b*cg_stride]
   int cg_stride = 0;
   int ngroups = 1;               // set by launch_hop_args
   int buf = 1;                   // set by launch_hop_args: FP32 / FP16 buffer loads

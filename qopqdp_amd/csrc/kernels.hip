@@ -394,6 +394,17 @@ __device__ __forceinline__ void hop_epilogue(const HopArgs &a, int h, int Vh, co
       }
       continue;
     }
+    if constexpr (RED == RED_R) {
+      // o = A p (not stored, rounded to the vector precision as a stored one
+      // would be); r -= alpha o, the sum formed in FP64 and rounded once
+      const double alr = a.cg_alpha[(long)rb * a.cg_stride];
+      R rv[6];
+      vload<P>(dd, dn, h, Vh, rv);
+#pragma unroll
+      for (int i = 0; i < 6; i++) rv[i] = (R)fma(-alr, (double)o[i], (double)rv[i]);
+      red[b] = vstore_norm2<P>(dd, dn, h, Vh, rv);
+      continue;
+    }
     if constexpr (RED == RED_OUT2) {
       red[b] = vstore_norm2<P, NT>(dd, dn, h, Vh, o);
       continue;
@@ -748,6 +759,10 @@ static void hop_dispatch_red(const HopArgs &a, dim3 grid, dim3 block, int red,
   if (red == RED_NONE) { if (hasx) QOP_LAUNCH(RED_NONE, true); else QOP_LAUNCH(RED_NONE, false); }
   else if (red == RED_OUT2) { if (hasx) QOP_LAUNCH(RED_OUT2, true); else QOP_LAUNCH(RED_OUT2, false); }
   else if (red == RED_CG) { QOP_LAUNCH(RED_CG, true); }
+  else if (red == RED_R) {
+    if constexpr (NB == 1 && !STG && !NT && P != P16 && LP == P) QOP_LAUNCH(RED_R, true);
+    else fatal(__FILE__, __LINE__, "hop: RED_R takes one FP64 / FP32 RHS per thread");
+  }
   else { QOP_LAUNCH(RED_X2, true); }
 #undef QOP_LAUNCH
 }
@@ -841,6 +856,7 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
               "hop: block must be a multiple of 64, 64..256 (512 with LDS staging)");
   QOP_REQUIRE(red == RED_NONE || hasx || red == RED_OUT2, "hop: RED_X2 / RED_CG need x");
   QOP_REQUIRE(red != RED_CG || (a.cg_alpha && a.xs.data && prec != P64), "hop: RED_CG needs alpha and xs");
+  QOP_REQUIRE(red != RED_R || a.cg_alpha, "hop: RED_R needs alpha");
   QOP_REQUIRE(a.n >= 1, "hop: n >= 1");
   QOP_REQUIRE(!a.slots || (prec == P64 && !a.single && red == RED_NONE && nb <= 8),
               "hop: a compacted slot list is for FP64 double-stored hops without reductions, at "

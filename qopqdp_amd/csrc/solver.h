@@ -18,7 +18,9 @@ struct CgmsState {
   int restart, max_iter;
   int nextRsqCheck, nextRelCheck;
   int break_reason;  // 1 pkp<=0, 2 restart/max_iter
-  int pad;
+  int xpend;         // the iteration that raised the status has its x update still to do
+  int cg;            // plain CG (lib/invert_cg_p.c:1-128): stop on rsq / relnorm, restarts on the host
+  int total;         // plain CG: operator applications over all restarts
   double rsq, oldrsq, pkp, insq, rsqstop, relstop, trueRsqFac, trueRelFac, relnorm2;
   double m2;  // base mass squared of the linear operator
   double shifts[CGMS_MAXSHIFT], a[CGMS_MAXSHIFT], b[CGMS_MAXSHIFT],
@@ -33,11 +35,11 @@ struct CgmsDev {
 
 // Launchers (cgms.hip)
 void cgms_launch_scalarA(CgmsDev d, int nch, hipStream_t st);
-void cgms_launch_update(CgmsDev d, int prec, int Vh, VecView r, VecView Mp, int ns,
-                        hipStream_t st);
 void cgms_launch_scalarB(CgmsDev d, int nch, int with_rel, int Vh, hipStream_t st);
-void cgms_launch_pupdate(CgmsDev d, int prec, int Vh, VecView p, VecView r, int ns,
-                         hipStream_t st);
+// x_i += b_i p_i (CGMS_X) and p_i = zn_i r + a_i p_i with |p|^2 of the base
+// (CGMS_P), of all ns shifts in one pass.
+enum { CGMS_X = 1, CGMS_P = 2, CGMS_XP = 3 };
+void cgms_launch_xp(CgmsDev d, int prec, int Vh, VecView r, int ns, int what, hipStream_t st);
 void cgms_launch_relnorm(CgmsDev d, int prec, int Vh, VecView r, VecView x,
                          hipStream_t st);
 

@@ -88,15 +88,109 @@ struct CgmsBuffers {
   }
 };
 
+// The device side of one CG or multi-shift CG: an iteration is
+//   t = D p (|t|^2);  b = r^2 / (|t|^2 + m^2 |p|^2);
+//   r -= b (m^2 p - D t) in the second hop's epilogue (|r|^2);
+//   a = r'^2 / r^2 and the shift recurrences;  x_i += b_i p_i, p_i = zn_i r + a_i p_i (|p|^2),
+// five launches, captured as a chunk; kernels past a raised status do nothing.
+class CgmsRun {
+ public:
+  CgmsRun(Links &L, int prec, double mass, int eo, int ns, bool with_rel, int irel, DevVec *const *x,
+          DevVec *const *pm, DevVec &p, DevVec &tmp, DevVec &r)
+      : B(L.lat, ns), prec_(prec), Vh_((int)L.lat->Vh), nl_(L.nl), ns_(ns), with_rel_(with_rel) {
+    hipStream_t st = stream();
+    const Lattice *lat = L.lat;
+    const int opp = 1 - eo;
+    p_ = p.half(eo);
+    r_ = r.half(eo);
+    hx_.resize(2 * ns);
+    for (int i = 0; i < ns; i++) {
+      hx_[i] = x[i]->half(eo);
+      hx_[ns + i] = pm[i]->half(eo);
+    }
+    if (with_rel) xrel_ = x[irel]->half(eo);
+    QOP_CHECK_HIP(hipMemcpyAsync(B.d.xs, hx_.data(), 2 * ns * sizeof(VecView), hipMemcpyHostToDevice, st));
+    // link arguments of both hops: any link conversion is done here, before
+    // the iterations are captured into a graph
+    set_hop_links(a1_, L, prec, opp);
+    set_hop_links(a2_, L, prec, eo);
+    a1_.g = a2_.g = lat->g;
+    a1_.status = a2_.status = &B.d.st->status;
+    a1_.parity = opp;
+    a1_.src = p_;
+    a1_.dst = tmp.half(opp);
+    a1_.partial = B.d.partA;
+    a2_.parity = eo;
+    a2_.src = tmp.half(opp);
+    a2_.dst = r_;
+    a2_.x = p_;
+    a2_.alpha = -1.0;
+    a2_.beta = mass * mass;
+    a2_.partial = B.d.partC;
+  }
+  // the scalars in B.host go to the device; |p|^2 of the base direction is
+  // formed for the next iteration
+  void start(int imin) {
+    hipStream_t st = stream();
+    a2_.cg_alpha = &B.d.st->b[imin];
+    B.push(st);
+    DotArgs d;
+    d.Vh = Vh_;
+    d.u = p_;
+    d.partial = B.d.partB;
+    launch_dot(d, prec_, prec_, 0, st);
+  }
+  // the p update of an iteration whose x update and scalars the host did
+  void resume() {
+    hipStream_t st = stream();
+    B.push(st);
+    cgms_launch_xp(B.d, prec_, Vh_, r_, ns_, CGMS_P, st);
+  }
+  // iterations until the status is raised; the state is in B.host then
+  void run() {
+    hipStream_t st = stream();
+    const int chunk = options().chunk > 0 ? options().chunk : 16;
+    if (options().use_graph && !graph_) {
+      graph_.begin(st);
+      for (int c = 0; c < chunk; c++) iteration();
+      graph_.end(st);
+    }
+    do {
+      if (graph_) graph_.launch(st);
+      else for (int c = 0; c < chunk; c++) iteration();
+      B.pull(st);
+    } while (B.host->status == 0);
+  }
+  CgmsBuffers B;
+
+ private:
+  void iteration() {
+    hipStream_t st = stream();
+    launch_hop_args(a1_, prec_, nl_, 1, 256, RED_OUT2, false, st);
+    cgms_launch_scalarA(B.d, B.nch, st);
+    launch_hop_args(a2_, prec_, nl_, 1, 256, RED_R, true, st);
+    if (with_rel_) {  // the relative residual needs x first
+      cgms_launch_xp(B.d, prec_, Vh_, r_, ns_, CGMS_X, st);
+      cgms_launch_relnorm(B.d, prec_, Vh_, r_, xrel_, st);
+    }
+    cgms_launch_scalarB(B.d, B.nch, with_rel_, Vh_, st);
+    cgms_launch_xp(B.d, prec_, Vh_, r_, ns_, with_rel_ ? CGMS_P : CGMS_XP, st);
+  }
+  int prec_, Vh_, nl_, ns_;
+  int with_rel_;
+  VecView p_, r_, xrel_{};
+  std::vector<VecView> hx_;
+  HopArgs a1_, a2_;
+  CapturedGraph graph_;
+};
+
 }  // namespace
 
 void invert_cgms(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg **ra,
                  const double *shifts, int ns, DevVec **out, const DevVec &in) {
   Lattice *lat = L.lat;
-  hipStream_t st = stream();
   QOP_REQUIRE(ns >= 1 && ns <= CGMS_MAXSHIFT, "invert_cgms: 1..64 shifts");
   QOP_REQUIRE(eo == 0 || eo == 1, "invert_cgms: subset must be even or odd");
-  const int opp = 1 - eo;
   double insq = norm2(in, eo);
   if (insq == 0.) {  // :152-162
     for (int i = 0; i < ns; i++) {
@@ -126,14 +220,10 @@ void invert_cgms(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg **r
   }
   copy(ry.v, in, eo);
 
-  CgmsBuffers B(lat, ns);
-  std::vector<VecView> hx(ns), hp(ns);
-  for (int i = 0; i < ns; i++) {
-    hx[i] = out[i]->half(eo);
-    hp[i] = (i == imin ? p.v : pm[i]->v).half(eo);
-  }
-  QOP_CHECK_HIP(hipMemcpyAsync(B.d.xs, hx.data(), ns * sizeof(VecView), hipMemcpyHostToDevice, st));
-  QOP_CHECK_HIP(hipMemcpyAsync(B.d.pms, hp.data(), ns * sizeof(VecView), hipMemcpyHostToDevice, st));
+  std::vector<DevVec *> pv(ns);
+  for (int i = 0; i < ns; i++) pv[i] = i == imin ? &p.v : &pm[i]->v;
+  CgmsRun run(L, prec, mass, eo, ns, relstop > 0, irel, out, pv.data(), p.v, tmp.v, r.v);
+  CgmsBuffers &B = run.B;
   CgmsState &S = *B.host;
   memset(&S, 0, sizeof S);
   S.status = 0;
@@ -149,53 +239,14 @@ void invert_cgms(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg **r
     S.zo[i] = S.z[i] = 1; S.zn[i] = 1;
     S.bo[i] = -1; S.a[i] = 0; S.b[i] = 0;
   }
-  B.push(st);
-
-  const int Vh = (int)lat->Vh;
-  const int nl = L.nl;
-  const int with_rel = relstop > 0;
-  // link arguments of both hops, resolved (and any link conversion done)
-  // before the iterations are captured into a graph
-  HopArgs l_opp, l_eo;
-  set_hop_links(l_opp, L, prec, opp);
-  set_hop_links(l_eo, L, prec, eo);
-  auto enqueue_iteration = [&]() {
-    // linop: tmp = D p (|tmp|^2), Mp = m^2 p - D tmp (|p|^2)
-    HopArgs a1 = l_opp;
-    a1.g = lat->g; a1.parity = opp;
-    a1.src = p.v.half(eo); a1.dst = tmp.v.half(opp);
-    a1.partial = B.d.partA; a1.status = &B.d.st->status;
-    launch_hop_args(a1, prec, nl, 1, 256, RED_OUT2, false, st);
-    HopArgs a2 = l_eo;
-    a2.g = lat->g; a2.parity = eo;
-    a2.src = tmp.v.half(opp); a2.dst = Mp.v.half(eo);
-    a2.x = p.v.half(eo); a2.alpha = -1.0; a2.beta = mass * mass;
-    a2.partial = B.d.partB; a2.status = &B.d.st->status;
-    launch_hop_args(a2, prec, nl, 1, 256, RED_X2, true, st);
-    cgms_launch_scalarA(B.d, B.nch, st);
-    cgms_launch_update(B.d, prec, Vh, r.v.half(eo), Mp.v.half(eo), ns, st);
-    if (with_rel) cgms_launch_relnorm(B.d, prec, Vh, r.v.half(eo), out[irel]->half(eo), st);
-    cgms_launch_scalarB(B.d, B.nch, with_rel, Vh, st);
-    cgms_launch_pupdate(B.d, prec, Vh, p.v.half(eo), r.v.half(eo), ns, st);
-  };
-
-  const int chunk = options().chunk > 0 ? options().chunk : 16;
-  CapturedGraph gexec;
-  if (options().use_graph) {
-    gexec.begin(st);
-    for (int c = 0; c < chunk; c++) enqueue_iteration();
-    gexec.end(st);
-  }
+  run.start(imin);
 
   double yAy = 0;
   auto linop = [&](DevVec &o, const DevVec &i) { return ddagd_norm2(L, prec, mass, o, i, eo, tmp.v); };
   DevVec &xmin = *out[imin];
   while (true) {
-    if (gexec) gexec.launch(st);
-    else for (int c = 0; c < chunk; c++) enqueue_iteration();
-    B.pull(st);
+    run.run();
     if (S.status == 2) break;
-    if (S.status == 0) continue;
     // status 1: fold the base solution into y and check the true residual
     // (:277-346), on the host with device vector operations.
     bool stop = false;
@@ -256,10 +307,9 @@ void invert_cgms(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg **r
     }
     for (int i = 0; i < ns; i++) { S.bo[i] = S.b[i]; S.zo[i] = S.z[i]; S.z[i] = S.zn[i]; }
     S.status = 0;
-    B.push(st);
-    cgms_launch_pupdate(B.d, prec, Vh, p.v.half(eo), r.v.half(eo), ns, st);
+    S.xpend = 0;
+    run.resume();
   }
-  gexec.reset();
   copy(xmin, y.v, eo);  // :378
   sync();
   for (int i = 0; i < ns; i++) {
@@ -272,50 +322,55 @@ void invert_cgms(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg **r
 }
 
 // ---------------------------------------------------------------------------
-// regular CG (lib/invert_cg_p.c:1-128), linop = ddagd
+// regular CG (lib/invert_cg_p.c:1-128), linop = ddagd.  The host runs the
+// (re)starts, where the residual is recomputed; the iterations between them run
+// on the device with the multi-shift CG's kernels at one shift, where they
+// took twelve launches and three host synchronisations each.  <p, A p> is
+// |D p|^2 + m^2 |p|^2, the value linop returns.
 void invert_cg(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg *ra,
                DevVec &out, const DevVec &in) {
   Lattice *lat = L.lat;
-  double a, b, rsq, oldrsq, pkp, relnorm = 1.0, insq, rsqstop;
-  int iteration = 0, total = 0, nrestart = -1;
-  int restart = ia->restart, max_iter = ia->max_iter, max_restarts = ia->max_restarts;
+  double rsq, relnorm = 1.0, insq, rsqstop;
+  int total = 0, nrestart = -1;
+  int max_iter = ia->max_iter, max_restarts = ia->max_restarts;
   if (max_restarts < 0) max_restarts = 5;
   ra->final_rsq = 0; ra->final_rel = 0; ra->final_iter = 0; ra->final_restart = 0;
   insq = norm2(in, eo);
   if (insq == 0.) { zero(out, eo); return; }
   TmpVec r(lat, prec), Mp(lat, prec), p(lat, prec), tmp(lat, prec);
-  auto linop = [&](DevVec &o, const DevVec &i) { ddagd_norm2(L, prec, mass, o, i, eo, tmp.v); };
   rsqstop = ra->rsqmin * insq;
-  rsq = 0; oldrsq = rsq;
-  while (true) {
-    if (total == 0 || iteration >= restart || total >= max_iter || rsq < rsqstop ||
-        relnorm < ra->relmin) {
-      if (total >= max_iter || nrestart >= max_restarts) break;
-      nrestart++;
-      copy(p.v, out, eo);
-      linop(Mp.v, p.v);
-      iteration = 1;
-      total++;
-      axpy(r.v, -1.0, Mp.v, in, eo);
-      rsq = norm2(r.v, eo);
-      if (ra->relmin > 0) relnorm = relnorm2(r.v, out, eo);
-      if (rsq < rsqstop || relnorm < ra->relmin || total >= max_iter) break;
-      copy(p.v, r.v, eo);
-    } else {
-      b = rsq / oldrsq;
-      axpy(p.v, b, p.v, r.v, eo);
-    }
-    oldrsq = rsq;
-    linop(Mp.v, p.v);
-    iteration++;
+  rsq = 0;
+  DevVec *xv[1] = {&out}, *pv[1] = {&p.v};
+  CgmsRun run(L, prec, mass, eo, 1, ra->relmin > 0, 0, xv, pv, p.v, tmp.v, r.v);
+  CgmsState &S = *run.B.host;
+  memset(&S, 0, sizeof S);
+  S.ns = 1;
+  S.cg = 1;
+  S.restart = ia->restart; S.max_iter = max_iter;
+  S.insq = insq; S.rsqstop = rsqstop; S.relstop = ra->relmin;
+  S.m2 = mass * mass;
+  S.zn[0] = 1;
+  while (total < max_iter && nrestart < max_restarts) {
+    nrestart++;
+    copy(p.v, out, eo);
+    ddagd_norm2(L, prec, mass, Mp.v, p.v, eo, tmp.v);
     total++;
-    pkp = redot(p.v, Mp.v, eo);
-    if (pkp <= 0) break;
-    a = rsq / pkp;
-    axpy(out, a, p.v, out, eo);
-    axpy(r.v, -a, Mp.v, r.v, eo);
+    axpy(r.v, -1.0, Mp.v, in, eo);
     rsq = norm2(r.v, eo);
     if (ra->relmin > 0) relnorm = relnorm2(r.v, out, eo);
+    if (rsq < rsqstop || relnorm < ra->relmin || total >= max_iter) break;
+    copy(p.v, r.v, eo);
+    S.status = 0;
+    S.xpend = 0;
+    S.iteration = 1;
+    S.total = total;
+    S.rsq = rsq;
+    run.start(0);
+    run.run();
+    total = S.total;
+    rsq = S.rsq;
+    if (S.status == 2) break;  // <p, A p> <= 0
+    if (ra->relmin > 0) relnorm = S.relnorm2;
   }
   ra->final_rsq = rsq / insq;
   ra->final_rel = relnorm;
