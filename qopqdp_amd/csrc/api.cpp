@@ -165,7 +165,7 @@ void links_from_gauge64(Links &L, double *const U_host[4], const QOP_asqtad_coef
   rephase_dev(L.lat, U, r0, bc, sign, 1, 1, nullptr, 0);
   fatten(L, L.lat, U, U, c, nullptr);
   sync();
-  for (int mu = 0; mu < 4; mu++) QOP_CHECK_HIP(hipFree(U[mu]));
+  for (int mu = 0; mu < 4; mu++) dev_free(U[mu]);
 }
 
 }  // namespace qop
@@ -194,6 +194,7 @@ QOP_status_t QOP_init(QOP_layout_t *layout) {
 QOP_status_t QOP_finalize(void) {
   CHECK_INIT;
   QOP_CHECK_HIP(hipDeviceSynchronize());
+  cache_trim();
   G.inited = 0;
   return QOP_SUCCESS;
 }
@@ -404,12 +405,12 @@ void QOP_F3_extract_G_to_raw(QOP_F_Real *dest[], QOP_F3_GaugeField *src, QOP_eve
 }
 void QOP_D3_destroy_G(QOP_D3_GaugeField *g) {
   if (!g) return;
-  for (int i = 0; i < 4; i++) if (g->U[i]) QOP_CHECK_HIP(hipFree(g->U[i]));
+  for (int i = 0; i < 4; i++) if (g->U[i]) dev_free(g->U[i]);
   delete g;
 }
 void QOP_F3_destroy_G(QOP_F3_GaugeField *g) {
   if (!g) return;
-  for (int i = 0; i < 4; i++) if (g->U[i]) QOP_CHECK_HIP(hipFree(g->U[i]));
+  for (int i = 0; i < 4; i++) if (g->U[i]) dev_free(g->U[i]);
   delete g;
 }
 // common_p.c:199-208, 244-257: the field keeps the caller's arrays; to_raw
@@ -469,7 +470,7 @@ FT *create_force(T *raw[], int eo, const char *fn) {
   if (!guard_oom(fn, nullptr, [&] {
         for (int i = 0; i < 4; i++) f->F[i] = upload_mat(G.lat, raw[i], eo);
       })) {
-    for (int i = 0; i < 4; i++) if (f->F[i]) QOP_CHECK_HIP(hipFree(f->F[i]));
+    for (int i = 0; i < 4; i++) if (f->F[i]) dev_free(f->F[i]);
     delete f;
     return nullptr;
   }
@@ -479,7 +480,7 @@ template <class FT>
 void destroy_force(FT *f) {
   if (!f) return;
   sync();
-  for (int i = 0; i < 4; i++) if (f->F[i]) QOP_CHECK_HIP(hipFree(f->F[i]));
+  for (int i = 0; i < 4; i++) if (f->F[i]) dev_free(f->F[i]);
   delete f;
 }
 

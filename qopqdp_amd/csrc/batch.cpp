@@ -171,7 +171,7 @@ HopShape tune_hop(Links &L, int prec, int nrhs, const DevBatch &src, DevBatch &d
   QOP_CHECK_HIP(hipEventDestroy(e1));
   if (scratch) {
     QOP_CHECK_HIP(hipStreamSynchronize(st));
-    QOP_CHECK_HIP(hipFree(scratch));
+    dev_free(scratch);
   }
   if (options().verbose)
     printf("TUNE: prec %d nrhs %d -> nb %d block %d remap %d nt %d inner %d tile %d stage %d "
@@ -202,25 +202,25 @@ BatchSolver::BatchSolver(Links &L, int eo, int capacity, int sloppy_prec, double
     devbatch_alloc(ts_, lat_, sp_, cap_);
     devbatch_alloc(xs_, lat_, P32, cap_);
     dev_alloc(&rhs_, cap_ * sizeof(BsRhs));
-    QOP_CHECK_HIP(hipHostMalloc(&rhs_h_, cap_ * sizeof(BsRhs), hipHostMallocDefault));
+    host_alloc(&rhs_h_, cap_ * sizeof(BsRhs));
     dev_alloc(&active_, 2 * cap_ * sizeof(int));
     sel_ = active_ + cap_;
-    QOP_CHECK_HIP(hipHostMalloc(&active_h_, 2 * cap_ * sizeof(int), hipHostMallocDefault));
+    host_alloc(&active_h_, 2 * cap_ * sizeof(int));
     sel_h_ = active_h_ + cap_;
     dev_alloc(&ru_, (3 * cap_ + 1) * sizeof(int));
     ru_cont_ = ru_ + cap_;
     slots_ = ru_ + 2 * cap_;
     QOP_CHECK_HIP(hipMemsetAsync(ru_, 0, (3 * cap_ + 1) * sizeof(int), st_));
     dev_alloc(&glob_, sizeof(BsGlobal));
-    QOP_CHECK_HIP(hipHostMalloc(&glob_h_, sizeof(BsGlobal), hipHostMallocDefault));
+    host_alloc(&glob_h_, sizeof(BsGlobal));
     dev_alloc(&partA_, 3 * (size_t)cap_ * nch_ * sizeof(double));
     partB_ = partA_ + (size_t)cap_ * nch_;
     partC_ = partB_ + (size_t)cap_ * nch_;
     dev_alloc(&coef_, (2 + 6) * (size_t)cap_ * sizeof(double));
     lcoef_ = coef_ + 2 * cap_;
     dev_alloc(&sums_, 2 * (size_t)cap_ * sizeof(double));
-    QOP_CHECK_HIP(hipHostMalloc(&sums_h_, 2 * (size_t)cap_ * sizeof(double), hipHostMallocDefault));
-    QOP_CHECK_HIP(hipHostMalloc(&hc_h_, 2 * (size_t)cap_ * sizeof(double), hipHostMallocDefault));
+    host_alloc(&sums_h_, 2 * (size_t)cap_ * sizeof(double));
+    host_alloc(&hc_h_, 2 * (size_t)cap_ * sizeof(double));
     memset(rhs_h_, 0, cap_ * sizeof(BsRhs));
     memset(active_h_, 0, 2 * cap_ * sizeof(int));
     glob_h_->status = 0;
@@ -257,18 +257,18 @@ void BatchSolver::release() {
   if (ev_) (void)hipEventDestroy(ev_);
   graph_.reset();
   for (DevBatch *b : {&x64_, &r64_, &b64_, &ax64_, &t64_, &rs_, &ps_, &ts_, &xs_}) devbatch_free(*b);
-  (void)hipFree(rhs_);
-  (void)hipHostFree(rhs_h_);
-  (void)hipFree(active_);
-  (void)hipFree(ru_);
-  (void)hipHostFree(active_h_);
-  (void)hipFree(glob_);
-  (void)hipHostFree(glob_h_);
-  (void)hipFree(partA_);
-  (void)hipFree(coef_);
-  (void)hipFree(sums_);
-  (void)hipHostFree(sums_h_);
-  (void)hipHostFree(hc_h_);
+  dev_free(rhs_);
+  host_free(rhs_h_);
+  dev_free(active_);
+  dev_free(ru_);
+  host_free(active_h_);
+  dev_free(glob_);
+  host_free(glob_h_);
+  dev_free(partA_);
+  dev_free(coef_);
+  dev_free(sums_);
+  host_free(sums_h_);
+  host_free(hc_h_);
 }
 
 int BatchSolver::free_slot() const {

@@ -54,6 +54,18 @@ template <class T>
 inline void dev_alloc(T **p, size_t bytes) {
   dev_alloc_bytes((void **)p, bytes);
 }
+// Gives memory of dev_alloc back (to the block cache of runtime.cpp: work
+// enqueued before the call may still use it).
+void dev_free(void *p);
+// Page-locked host memory of the solvers' status words and staging.
+void host_alloc_bytes(void **p, size_t bytes);
+template <class T>
+inline void host_alloc(T **p, size_t bytes) {
+  host_alloc_bytes((void **)p, bytes);
+}
+void host_free(void *p);
+void cache_trim();         // kept blocks go back to the driver
+size_t dev_cache_bytes();  // device memory held in kept blocks
 // Owning device buffer for temporaries: freed when it goes out of scope,
 // also while a DeviceOutOfMemory unwinds.
 template <class T>
@@ -62,7 +74,7 @@ struct DevBuf {
   DevBuf() = default;
   explicit DevBuf(size_t bytes) { dev_alloc(&p, bytes); }
   ~DevBuf() {
-    if (p) (void)hipFree(p);
+    if (p) dev_free(p);
   }
   DevBuf(const DevBuf &) = delete;
   DevBuf &operator=(const DevBuf &) = delete;
@@ -161,6 +173,7 @@ struct LinkSet {
   int nl = 0;            // 16 with Naik, 8 without
   void *data = nullptr;  // [2][nl][9][Vh] complex
   float *scale = nullptr;  // FP16: [2][nl][Vh]
+  long sites = 0;          // Vh of the array, set by build_links64
   const void *parity_data(const Lattice *lat, int p) const {
     return (const char *)data + (size_t)p * nl * 9 * lat->Vh * prec_cbytes(prec);
   }

@@ -23,7 +23,7 @@ using zd = std::complex<double>;
 EigcgState::~EigcgState() {
   if (store) {
     sync();
-    QOP_CHECK_HIP(hipFree(store));
+    dev_free(store);
   }
 }
 

@@ -18,6 +18,7 @@
 // field is copied into the site-innermost layout once per call.
 #include <cstring>
 #include <stdexcept>
+#include <vector>
 
 #include "common.h"
 
@@ -201,9 +202,35 @@ __device__ __forceinline__ M3 ld(const Lin &f, long V, unsigned s) {
   return m;
 }
 
-// Four field pointers passed by value (one per direction).
+// Four field pointers passed by value (one per direction), and the mids.
 struct Ptr4 {
   const double2 *p[4];
+};
+struct MidPtr {
+  double2 *p[8];
+};
+
+// Site-innermost fields of one call, allocated one by one (fields of the size
+// the block cache of dev_alloc keeps from call to call).
+class Fields {
+ public:
+  explicit Fields(long V) : bytes_((size_t)9 * V * sizeof(double2)) {}
+  Fields(const Fields &) = delete;
+  Fields &operator=(const Fields &) = delete;
+  ~Fields() {
+    for (double2 *f : f_) dev_free(f);
+  }
+  double2 *take() {
+    f_.reserve(f_.size() + 1);
+    double2 *f = nullptr;
+    dev_alloc(&f, bytes_);
+    f_.push_back(f);
+    return f;
+  }
+
+ private:
+  size_t bytes_;
+  std::vector<double2 *> f_;
 };
 
 // raw [V][18] -> site-innermost [9][V].  A block's TPB sites are one
@@ -254,7 +281,7 @@ __global__ __launch_bounds__(TPB) void lincomb_kernel(double2 *o, double co, dou
 template <typename T2>
 __global__ __launch_bounds__(TPB) void mid_kernel(Geom g, Sched q, long V, const T2 *const *xs,
                                                   const double *eps, int n, int nmid, double scale,
-                                                  double2 *mid) {
+                                                  MidPtr mid) {
   const int s0 = site_index(q, g.Vh);
   if (s0 < 0) return;
   const unsigned s = (unsigned)s0;
@@ -303,7 +330,7 @@ __global__ __launch_bounds__(TPB) void mid_kernel(Geom g, Sched q, long V, const
       }
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++) st_nt(mid + (long)mi[k] * 9 * V, V, s, acc[k]);
+    for (int k = 0; k < 4; k++) st_nt(mid.p[mi[k]], V, s, acc[k]);
   }
 }
 
@@ -741,22 +768,19 @@ constexpr double SIDE_FORCE_FLOPS = 7 * 198 + 3 * 216 + 3 * 18;
 namespace {
 
 // One force evaluation: launch geometry, site-innermost workspace and the
-// device table of vector pointers and eps.  nfields: fields besides the
-// derivative scratch (stpl3[4], mid5[4], stpl5, mid3).
+// device table of vector pointers and eps.
 class ForceRun {
  public:
-  ForceRun(const Lattice *lat, int nfields, const double *eps, const DevVec *const *xs, int n,
+  ForceRun(const Lattice *lat, const double *eps, const DevVec *const *xs, int n,
            hipStream_t st)
       : g_(lat->g), V_(lat->V), n9_(9 * lat->V), st_(st), sq_(make_sched(lat)),
-        b_(TPB), gs_(grid(lat->V)), ge_(grid(9 * lat->V)), gx_(8 * sq_.per) {
+        b_(TPB), gs_(grid(lat->V)), ge_(grid(9 * lat->V)), gx_(8 * sq_.per), buf_(lat->V) {
     if (V_ >= (1L << 27))
       throw std::runtime_error("fermion force: lattice volume of 2^27 sites or more (32-bit offsets)");
     prec_ = n > 0 ? xs[0]->prec : P64;
     for (int t = 0; t < n; t++)
       if (xs[t]->prec != prec_ || xs[t]->lat != lat || (prec_ != P64 && prec_ != P32))
         throw std::runtime_error("fermion force: vectors must share the lattice and be FP64 or FP32");
-    dev_alloc(&buf_.p, (size_t)(nfields + 10) * n9_ * sizeof(double2));
-    next_ = buf_.p;
     for (auto &q : stpl3_) q = take();
     for (auto &q : mid5_) q = take();
     stpl5_ = take();
@@ -772,11 +796,7 @@ class ForceRun {
     QOP_CHECK_HIP(hipMemcpy(tab_.p, h.data(), ntab * sizeof(double), hipMemcpyHostToDevice));
     n_ = n;
   }
-  double2 *take() {
-    double2 *r = next_;
-    next_ += n9_;
-    return r;
-  }
+  double2 *take() { return buf_.take(); }
   double flops_per_site = 0;
 
   void to_soa(const double *raw, double2 *f) {
@@ -787,7 +807,9 @@ class ForceRun {
     hipLaunchKernelGGL(lincomb_kernel, ge_, b_, 0, st_, o, co, ca, A, cb, B, n9_);
   }
   // mid fields of terms [t0, t0 + cnt): nmid = 4 (one-hop) or 8 (and three-hop)
-  void mids(int t0, int cnt, int nmid, double scale, double2 *mid) {
+  void mids(int t0, int cnt, int nmid, double scale, double2 *const *mids) {
+    MidPtr mid{};
+    for (int i = 0; i < nmid; i++) mid.p[i] = mids[i];
     const double *tab = tab_.p;
     if (prec_ == P64)
       hipLaunchKernelGGL(mid_kernel<double2>, gx_, b_, 0, st_, g_, sq_, V_,
@@ -877,9 +899,8 @@ class ForceRun {
   Sched sq_;
   dim3 b_, gs_, ge_, gx_;
   int prec_ = P64, n_ = 0;
-  DevBuf<double2> buf_;
+  Fields buf_;
   DevBuf<double> tab_;
-  double2 *next_ = nullptr;
   double2 *stpl3_[4] = {}, *mid5_[4] = {}, *stpl5_ = nullptr, *mid3_ = nullptr;
 };
 
@@ -992,7 +1013,7 @@ void asqtad_force_dev(const Lattice *lat, double *const U_raw[4], double *F_raw[
                       double *flops, hipStream_t st) {
   const bool naik = coef[5] != 0;
   const int nmid = naik ? 8 : 4;
-  ForceRun r(lat, 4 + nmid + 4, eps, xs, n, st);
+  ForceRun r(lat, eps, xs, n, st);
   double2 *U[4], *mid[8] = {}, *D[4];
   for (auto &u : U) u = r.take();
   for (int i = 0; i < nmid; i++) mid[i] = r.take();
@@ -1001,7 +1022,7 @@ void asqtad_force_dev(const Lattice *lat, double *const U_raw[4], double *F_raw[
     r.to_soa(U_raw[mu], U[mu]);
     r.lincomb(D[mu], 0.0, 0.0, nullptr, 0.0, nullptr);
   }
-  r.mids(0, n, nmid, -1.0, mid[0]);
+  r.mids(0, n, nmid, -1.0, mid);
   r.deriv(U, D, coef, mid, naik ? mid + 4 : nullptr);
   r.final(F_raw, U, D, -2.0);
   r.finish();
@@ -1016,7 +1037,7 @@ void hisq_force_dev(const Lattice *lat, double *const U_raw[4], double *const V_
                     double *flops, int *nfilt, hipStream_t st) {
   int nterms = 0;
   for (int k = 0; k < n_naiks; k++) nterms += n_orders[k];
-  ForceRun r(lat, 4 + 4 + 8 + 4 + 4, eps, xs, nterms, st);
+  ForceRun r(lat, eps, xs, nterms, st);
   double2 *U[4], *W[4], *mid[8], *F1[4], *F2[4];
   for (auto &u : U) u = r.take();
   for (auto &w : W) w = r.take();
@@ -1036,7 +1057,7 @@ void hisq_force_dev(const Lattice *lat, double *const U_raw[4], double *const V_
   int shift = 0;
   for (int k = 0; k < n_naiks; k++) {
     const int c = k == 0 ? nterms : n_orders[k];
-    r.mids(shift, c, 8, 1.0, mid[0]);
+    r.mids(shift, c, 8, 1.0, mid);
     for (int mu = 0; mu < 4; mu++) r.lincomb(F1[mu], 0.0, 0.0, nullptr, 0.0, nullptr);
     r.deriv(W, F1, k == 0 ? lev2 : diff, mid, mid + 4);
     const double cm = k == 0 ? 1.0 : eps_naik[k];
@@ -1074,11 +1095,8 @@ void fatten_dev(const Lattice *lat, const double *const gf[4], const double *con
   const bool have3 = coef3 != 0 || have5;
   const bool naik = lng_raw != nullptr;
   const bool sep_long = naik && (gl[0] != gf[0] || gl[1] != gf[1] || gl[2] != gf[2] || gl[3] != gf[3]);
-  const int nf = 4 + 1 + (have3 ? 2 : 0) + (naik ? 1 : 0) + (sep_long ? 4 : 0);
-  DevBuf<double2> buf;
-  dev_alloc(&buf.p, (size_t)nf * n9 * sizeof(double2));
-  double2 *p = buf.p;
-  auto take = [&] { double2 *r = p; p += n9; return r; };
+  Fields buf(V);
+  auto take = [&] { return buf.take(); };
   double2 *U[4], *UL[4], *F = take(), *S3 = nullptr, *S5 = nullptr, *Lk = nullptr;
   for (auto &u : U) u = take();
   if (have3) {

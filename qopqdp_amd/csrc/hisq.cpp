@@ -63,7 +63,7 @@ struct Raw4 {
   }
   void free() {
     for (int i = 0; i < 4; i++)
-      if (m[i]) QOP_CHECK_HIP(hipFree(m[i]));
+      if (m[i]) dev_free(m[i]);
     for (int i = 0; i < 4; i++) m[i] = nullptr;
   }
 };
@@ -161,7 +161,7 @@ HisqT *hisq_create(QOP_info_t *info, QOP_hisq_coeffs_t *c, GaugeT *gauge) {
     std::vector<int> cnt(2 * nw);
     QOP_CHECK_HIP(hipMemcpyAsync(cnt.data(), u.counts, 2 * nw * sizeof(int), hipMemcpyDeviceToHost, st));
     sync();
-    QOP_CHECK_HIP(hipFree(u.counts));
+    dev_free(u.counts);
     long bad = 0;
     for (long i = 0; i < nw; i++) {
       nsvd += cnt[2 * i];
@@ -183,7 +183,7 @@ HisqT *hisq_create(QOP_info_t *info, QOP_hisq_coeffs_t *c, GaugeT *gauge) {
       if (h->fn_deps) { h->fn_deps->L.free_all(); delete h->fn_deps; }
       for (auto &a : h->aux)
         for (auto *p : a)
-          if (p) QOP_CHECK_HIP(hipFree(p));
+          if (p) dev_free(p);
       delete h;
     }
   } owner{h};
@@ -264,7 +264,7 @@ void hisq_destroy(HisqT *h, DestroyL destroy) {
   sync();
   for (auto &a : h->aux)
     for (auto *p : a)
-      if (p) QOP_CHECK_HIP(hipFree(p));
+      if (p) dev_free(p);
   delete h;
 }
 

@@ -53,13 +53,15 @@ void build_links64(Links &L, const double *fat_dev[4], const double *lng_dev[4],
   const Lattice *lat = L.lat;
   L.nl = lng_dev ? 16 : 8;
   LinkSet &s = L.l64;
-  linkset_free(s);
+  // a reloaded object of the same lattice keeps its array
+  if (s.nl != L.nl || s.sites != lat->Vh) linkset_free(s);
   L.drop_derived();
   DevBuf<const double *> pbuf(8 * sizeof(double *));
   const double **ptrs = pbuf.p;
-  dev_alloc(&s.data, (size_t)2 * L.nl * 9 * lat->Vh * sizeof(double2));
+  if (!s.data) dev_alloc(&s.data, (size_t)2 * L.nl * 9 * lat->Vh * sizeof(double2));
   s.prec = P64;
   s.nl = L.nl;
+  s.sites = lat->Vh;
   const double *hp[8];
   for (int i = 0; i < 4; i++) { hp[i] = fat_dev[i]; hp[4 + i] = lng_dev ? lng_dev[i] : nullptr; }
   QOP_CHECK_HIP(hipMemcpyAsync(ptrs, hp, sizeof hp, hipMemcpyHostToDevice, st));

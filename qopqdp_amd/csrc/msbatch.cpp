@@ -37,10 +37,10 @@ MultiShiftBatch::MultiShiftBatch(Links &L, int eo, int capacity, int sloppy_prec
     dev_alloc(&ru_, cap_ * sizeof(int));
     QOP_CHECK_HIP(hipMemset(ru_, 0, cap_ * sizeof(int)));
     dev_alloc(&slot_, cap_ * sizeof(MsSlot));
-    QOP_CHECK_HIP(hipHostMalloc(&slot_h_, cap_ * sizeof(MsSlot), hipHostMallocDefault));
+    host_alloc(&slot_h_, cap_ * sizeof(MsSlot));
     dev_alloc(&active_, 2 * cap_ * sizeof(int));
     sel_ = active_ + cap_;
-    QOP_CHECK_HIP(hipHostMalloc(&active_h_, cap_ * sizeof(int), hipHostMallocDefault));
+    host_alloc(&active_h_, cap_ * sizeof(int));
     dev_alloc(&partA_, 3 * (size_t)cap_ * nch_ * sizeof(double));
     partB_ = partA_ + (size_t)cap_ * nch_;
     partC_ = partB_ + (size_t)cap_ * nch_;
@@ -72,15 +72,15 @@ void MultiShiftBatch::release() {
   sync();
   graph_.reset();
   for (DevBatch *b : {&b64_, &rs_, &ps_, &ts_, &pm_, &xm_, &x64_, &t64_, &ax64_}) devbatch_free(*b);
-  (void)hipFree(ru_);
-  (void)hipFree(slot_);
-  (void)hipHostFree(slot_h_);
-  (void)hipFree(active_);
-  (void)hipHostFree(active_h_);
-  (void)hipFree(partA_);
-  (void)hipFree(coef_);
-  (void)hipFree(sums_);
-  (void)hipFree(zero_status_);
+  dev_free(ru_);
+  dev_free(slot_);
+  host_free(slot_h_);
+  dev_free(active_);
+  host_free(active_h_);
+  dev_free(partA_);
+  dev_free(coef_);
+  dev_free(sums_);
+  dev_free(zero_status_);
 }
 
 void MultiShiftBatch::load(int slot, const DevVec &src, double ms_tol, int max_iter) {

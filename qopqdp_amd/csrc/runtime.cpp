@@ -14,16 +14,170 @@ namespace qop {
   abort();
 }
 
+// ---------------------------------------------------------------------------
+// Block cache of dev_alloc / dev_free and host_alloc / host_free.
+//
+// Solves, link construction and forces take their workspaces at every call;
+// hipMalloc and hipFree of a few GB take tens of milliseconds (one asqtad link
+// construction at 24^3x48: 8.5 ms of kernels in a 69 ms call), so freed blocks
+// are kept and handed out again.
+//  * A freed block may still be in use by work enqueued on any stream.  It is
+//    pending until a device synchronisation after its free (hipFree waits for
+//    the device too) and only then handed out, so a block never passes from
+//    one stream or thread to another with work in flight.
+//  * Bounded: blocks above CACHE_BLOCK bytes go back to the driver at once
+//    (calls that use them run long enough that their allocation does not show:
+//    one 32^3x64 link-matrix field, 302 MB, is still kept), and the kept blocks
+//    of a device total at most CACHE_TOTAL bytes.
+//  * Given back: at QOP_finalize, when a request server ends, and when
+//    an allocation fails (it is tried again then, and if it still fails the
+//    blocks freed while the failure unwinds are not kept).
+namespace {
+constexpr size_t CACHE_BLOCK = (size_t)384 << 20, CACHE_TOTAL = (size_t)8 << 30;
+constexpr size_t CACHE_HOST_BLOCK = (size_t)1 << 20, CACHE_HOST_TOTAL = (size_t)64 << 20;
+
+class BlockCache {
+ public:
+  BlockCache(bool host, size_t block, size_t total) : host_(host), block_(block), total_(total) {}
+  void *alloc(size_t bytes) {
+    int dev = 0;
+    QOP_CHECK_HIP(hipGetDevice(&dev));
+    const size_t want = bytes <= block_ ? round(bytes) : bytes;
+    std::lock_guard<std::mutex> lk(mu_);
+    void *p = nullptr;
+    if (want <= block_) {
+      p = take(ready_, dev, want);
+      if (!p && fits(pending_, dev, want)) {
+        QOP_CHECK_HIP(hipDeviceSynchronize());
+        settle(dev);
+        p = take(ready_, dev, want);
+      }
+    }
+    if (!p) {
+      hipError_t e = raw_alloc(&p, want);
+      if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // clear the error state of this thread
+        trim_locked();
+        e = raw_alloc(&p, want);
+      }
+      if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        failed_ = true;
+        throw DeviceOutOfMemory{bytes};
+      }
+      if (e != hipSuccess) fatal(__FILE__, __LINE__, hipGetErrorString(e));
+      if (want <= block_) live_[p] = Block{want, dev};
+    }
+    failed_ = false;
+    return p;
+  }
+  void free(void *p) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(mu_);
+    auto it = live_.find(p);
+    if (it == live_.end() || failed_ || kept_ + it->second.bytes > total_) {
+      if (it != live_.end()) live_.erase(it);
+      raw_free(p);
+      return;
+    }
+    kept_ += it->second.bytes;
+    pending_.emplace(it->second.bytes, std::make_pair(p, it->second.dev));
+    live_.erase(it);
+  }
+  void trim() {
+    std::lock_guard<std::mutex> lk(mu_);
+    trim_locked();
+  }
+  size_t kept() {
+    std::lock_guard<std::mutex> lk(mu_);
+    return kept_;
+  }
+
+ private:
+  struct Block {
+    size_t bytes;
+    int dev;
+  };
+  using Kept = std::multimap<size_t, std::pair<void *, int>>;
+  // whole 512-byte units, and 1/16 of the size for large blocks, so nearby
+  // sizes share blocks
+  static size_t round(size_t bytes) {
+    size_t unit = 512;
+    while (unit * 16 < bytes) unit *= 2;
+    return bytes ? (bytes + unit - 1) / unit * unit : unit;
+  }
+  // a kept block of at least `want` bytes and at most 1/8 more
+  static Kept::iterator find(Kept &k, int dev, size_t want) {
+    for (auto it = k.lower_bound(want); it != k.end() && it->first <= want + want / 8; ++it)
+      if (it->second.second == dev) return it;
+    return k.end();
+  }
+  static bool fits(Kept &k, int dev, size_t want) { return find(k, dev, want) != k.end(); }
+  void *take(Kept &k, int dev, size_t want) {
+    auto it = find(k, dev, want);
+    if (it == k.end()) return nullptr;
+    void *p = it->second.first;
+    live_[p] = Block{it->first, dev};
+    kept_ -= it->first;
+    k.erase(it);
+    return p;
+  }
+  // the pending blocks of a device that has been synchronised
+  void settle(int dev) {
+    for (auto it = pending_.begin(); it != pending_.end();) {
+      if (it->second.second == dev) {
+        ready_.insert(*it);
+        it = pending_.erase(it);
+      } else {
+        ++it;
+      }
+    }
+  }
+  hipError_t raw_alloc(void **p, size_t n) const {
+    return host_ ? hipHostMalloc(p, n, hipHostMallocDefault) : hipMalloc(p, n);
+  }
+  void raw_free(void *p) const {
+    if (host_) QOP_CHECK_HIP(hipHostFree(p));
+    else QOP_CHECK_HIP(hipFree(p));  // waits for the work that uses it
+  }
+  void trim_locked() {
+    for (Kept *k : {&ready_, &pending_}) {
+      for (auto &b : *k) raw_free(b.second.first);
+      k->clear();
+    }
+    kept_ = 0;
+  }
+  const bool host_;
+  const size_t block_, total_;
+  std::mutex mu_;
+  Kept ready_, pending_;
+  std::map<void *, Block> live_;
+  size_t kept_ = 0;
+  bool failed_ = false;  // the last allocation failed: its frees are not kept
+};
+// never destroyed: owners with static lifetime may free after main
+BlockCache &dev_cache() {
+  static BlockCache *c = new BlockCache(false, CACHE_BLOCK, CACHE_TOTAL);
+  return *c;
+}
+BlockCache &host_cache() {
+  static BlockCache *c = new BlockCache(true, CACHE_HOST_BLOCK, CACHE_HOST_TOTAL);
+  return *c;
+}
+}  // namespace
+
 void dev_alloc_bytes(void **p, size_t bytes) {
   *p = nullptr;
-  const hipError_t e = hipMalloc(p, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();  // clear the error state of this thread
-    *p = nullptr;
-    throw DeviceOutOfMemory{bytes};
-  }
-  if (e != hipSuccess) fatal(__FILE__, __LINE__, hipGetErrorString(e));
+  *p = dev_cache().alloc(bytes);
 }
+void dev_free(void *p) { dev_cache().free(p); }
+void host_alloc_bytes(void **p, size_t bytes) { *p = host_cache().alloc(bytes); }
+void host_free(void *p) { host_cache().free(p); }
+void cache_trim() {
+  dev_cache().trim();
+  host_cache().trim();
+}
+size_t dev_cache_bytes() { return dev_cache().kept(); }
 
 static std::mutex g_mu;
 
@@ -70,8 +224,8 @@ void devvec_alloc(DevVec &v, Lattice *lat, int prec) {
 }
 
 void devvec_free(DevVec &v) {
-  if (v.data) QOP_CHECK_HIP(hipFree(v.data));
-  if (v.norm) QOP_CHECK_HIP(hipFree(v.norm));
+  if (v.data) dev_free(v.data);
+  if (v.norm) dev_free(v.norm);
   v.data = nullptr;
   v.norm = nullptr;
 }
@@ -96,18 +250,19 @@ void devbatch_alloc(DevBatch &v, Lattice *lat, int prec, int n) {
 }
 
 void devbatch_free(DevBatch &v) {
-  if (v.data) QOP_CHECK_HIP(hipFree(v.data));
-  if (v.norm) QOP_CHECK_HIP(hipFree(v.norm));
+  if (v.data) dev_free(v.data);
+  if (v.norm) dev_free(v.norm);
   v.data = nullptr;
   v.norm = nullptr;
   v.n = 0;
 }
 
 void linkset_free(LinkSet &l) {
-  if (l.data) QOP_CHECK_HIP(hipFree(l.data));
-  if (l.scale) QOP_CHECK_HIP(hipFree(l.scale));
+  if (l.data) dev_free(l.data);
+  if (l.scale) dev_free(l.scale);
   l.data = nullptr;
   l.scale = nullptr;
+  l.sites = 0;
   l.prec = -1;
 }
 
@@ -179,7 +334,7 @@ struct Scratch {
     if (bytes <= n) return p;
     if (p) {
       QOP_CHECK_HIP(hipStreamSynchronize(stream()));
-      if (host) QOP_CHECK_HIP(hipHostFree(p)); else QOP_CHECK_HIP(hipFree(p));
+      if (host) QOP_CHECK_HIP(hipHostFree(p)); else dev_free(p);
     }
     p = nullptr;
     n = 0;

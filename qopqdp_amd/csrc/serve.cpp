@@ -100,6 +100,7 @@ class Server {
   Server(int capacity, int prec, size_t budget) : cap_(capacity), prec_(prec), budget_(budget) {
     size_t fr = 0, tot = 0;
     QOP_CHECK_HIP(hipMemGetInfo(&fr, &tot));
+    fr += dev_cache_bytes();  // given back when an allocation needs it
     reserve_ = std::min<size_t>((size_t)2 << 30, tot / 32);
     if (!budget_) budget_ = fr > reserve_ ? fr - reserve_ : 0;
     worker_ = std::thread([this] { run(); });
@@ -295,7 +296,7 @@ class Server {
   void drop_engine(Engine &e) {
     e.bs.reset();
     devvec_free(e.stage);
-    if (e.raw) QOP_CHECK_HIP(hipFree(e.raw));
+    if (e.raw) dev_free(e.raw);
     e.raw = nullptr;
     if (e.st && e.own_stream) QOP_CHECK_HIP(hipStreamDestroy(e.st));
     e.st = nullptr;
@@ -315,6 +316,7 @@ class Server {
       }
       size_t fr = 0, tot = 0;
       QOP_CHECK_HIP(hipMemGetInfo(&fr, &tot));
+      fr += dev_cache_bytes();
       if (used + need <= budget_ && fr >= need + reserve_) break;
       // evict the least recently used idle engine
       int victim = -1;
@@ -556,6 +558,7 @@ void QOPX_serve_destroy(QOPX_Server *s) {
   if (!s) return;
   delete s->s;
   delete s;
+  qop::cache_trim();
 }
 
 }  // extern "C"

@@ -66,14 +66,14 @@ struct CgmsBuffers {
       release();
       throw;
     }
-    QOP_CHECK_HIP(hipHostMalloc(&host, sizeof(CgmsState), hipHostMallocDefault));
+    host_alloc(&host, sizeof(CgmsState));
   }
   ~CgmsBuffers() { release(); }
   void release() {
-    if (d.st) (void)hipFree(d.st);
-    if (d.partA) (void)hipFree(d.partA);
-    if (d.xs) (void)hipFree(d.xs);
-    if (host) (void)hipHostFree(host);
+    if (d.st) dev_free(d.st);
+    if (d.partA) dev_free(d.partA);
+    if (d.xs) dev_free(d.xs);
+    if (host) host_free(host);
     d.st = nullptr;
     d.partA = nullptr;
     d.xs = nullptr;
