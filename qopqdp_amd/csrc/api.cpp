@@ -108,23 +108,10 @@ void build_links_from_raw(Links &L, T *fat[], T *lng[], int eo) {
 void fatten(Links &L, Lattice *lat, const double *const gf[4], const double *const gl[4],
             const QOP_asqtad_coeffs_t *c, QOP_info_t *info) {
   double coef[6] = {c->one_link, c->three_staple, c->five_staple, c->seven_staple, c->lepage, c->naik};
-  bool naik = c->naik != 0;
-  DevBuf<double> fbuf[4], lbuf[4];
-  double *fat[4], *lng[4];
-  size_t n = (size_t)lat->V * 18 * sizeof(double);
-  for (int i = 0; i < 4; i++) {
-    dev_alloc(&fbuf[i].p, n);
-    if (naik) dev_alloc(&lbuf[i].p, n);
-    fat[i] = fbuf[i].p;
-    lng[i] = lbuf[i].p;
-  }
-  const double *g[4] = {gf[0], gf[1], gf[2], gf[3]}, *gL[4] = {gl[0], gl[1], gl[2], gl[3]};
+  const bool naik = c->naik != 0;
   double t0 = wall_time();
-  launch_fatten(lat, g, gL, coef, fat, naik ? lng : nullptr, stream());
+  fatten_links64(lat, L, gf, gl, coef, stream());
   double dt = wall_time() - t0;
-  L.lat = lat;
-  const double *fc[4] = {fat[0], fat[1], fat[2], fat[3]}, *lc[4] = {lng[0], lng[1], lng[2], lng[3]};
-  build_links64(L, fc, naik ? lc : nullptr, stream());
   bool have3 = c->three_staple != 0 || c->five_staple != 0 || c->seven_staple != 0 || c->lepage != 0;
   if (info) {  // asqtad_dslash_p.c:536, 624-626
     info->final_sec = dt;

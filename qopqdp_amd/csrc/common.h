@@ -211,6 +211,8 @@ double *red_result(size_t ndoubles);   // device
 double *red_host(size_t ndoubles);     // pinned host
 
 // Link preparation (links.hip)
+// the FP64 array of nl links per site for L.lat (kept when it already fits)
+void links64_alloc(Links &L, int nl);
 void build_links64(Links &L, const double *fat_dev[4], const double *lng_dev[4],
                    hipStream_t st);
 void convert_links(const Lattice *lat, const LinkSet &src, LinkSet &dst,
@@ -236,6 +238,11 @@ void asqtad_force_dev(const Lattice *lat, double *const U_raw[4], double *F_raw[
 // lng (optional) = naik gl gl gl; coef as for asqtad_force_dev.
 void fatten_dev(const Lattice *lat, const double *const gf[4], const double *const gl[4],
                 const double coef[6], double *fat[4], double *lng[4], hipStream_t st);
+
+// The same smearing written straight into the double-stored FP64 links of L
+// (Naik links when c[5] != 0).
+void fatten_links64(const Lattice *lat, Links &L, const double *const gf[4],
+                    const double *const gl[4], const double coef[6], hipStream_t st);
 
 // HISQ fermion force (force.hip): F[mu] += TA(U_mu deriv_mu^+) with deriv
 // through level 2 (W, lev2 or the difference set diff per epsilon-Naik group),

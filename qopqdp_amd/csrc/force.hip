@@ -28,24 +28,25 @@ namespace {
 constexpr int TPB = 256;
 
 // Site order of the gathering kernels (x0-tiled, XCD-aware).  A slab is the
-// S = Vh / L0 sites of one x0 and parity; it is cut into tiles of T sites.
-// Logical blocks run tile by tile, and inside a tile over x0 and the two
-// parities, so the x0 +-1 neighbours a block gathers belong to blocks about
-// 2 T / TPB positions away, still in L2, and the x1..x3 neighbours mostly to
-// the same or the partner block.  The hardware dispatches block b to XCD
-// b % 8; XCD k runs the logical blocks [k per, (k+1) per), a contiguous part
-// of that order.  -1 marks padding threads.
+// S = Vh / L0 sites of one x0 and parity; it is cut into equal tiles of at most
+// 2048 sites.  A block takes 128 positions of a slab in both parities (its waves
+// alternate), so the parity-flipping neighbours of a site are in its own or a
+// nearby block.  Logical blocks run tile by tile and inside a tile over x0, so
+// the x0 +-1 neighbours a block gathers belong to blocks T / 128 positions
+// away.  The hardware dispatches block b to XCD b % 8; XCD k runs the logical
+// blocks [k per, (k+1) per), a contiguous part of that order.  -1 marks padding
+// threads.  Asqtad force at 24^3x48: 16.7 ms with 4096-site tiles of one parity
+// after the other; with both in a block 16.1 / 15.6 / 15.3 / 17.2 ms at tiles of
+// 512 / 1024 / 2048 / 4096.
 struct Sched {
   int S, T, nt, L0, bpt, per;  // slab, tile, tiles per slab, extent 0, blocks per tile, blocks per XCD
 };
 __device__ __forceinline__ int site_index(const Sched &q, int Vh) {
   const int w = (int)(blockIdx.x & 7) * q.per + (int)(blockIdx.x >> 3);
-  const int sub = w % q.bpt;
-  int r = w / q.bpt;
-  const int par = r & 1;
-  r >>= 1;
+  const int sub = w % q.bpt, r = w / q.bpt;
+  const int par = (int)(threadIdx.x >> 6) & 1;
   const int x0 = r % q.L0, tile = r / q.L0;
-  const int hs = tile * q.T + sub * TPB + (int)threadIdx.x;
+  const int hs = tile * q.T + sub * (TPB / 2) + (int)((threadIdx.x >> 7) * 64 + (threadIdx.x & 63));
   if (tile >= q.nt || hs >= q.S) return -1;
   return par * Vh + x0 * q.S + hs;
 }
@@ -340,18 +341,21 @@ __global__ __launch_bounds__(TPB) void mid_kernel(Geom g, Sched q, long V, const
 // I is the field along mu, K the link along nu.  TWO computes the two
 // 7-staples of a (sig, rho) pair in one pass, in the order in which the
 // reference accumulates them (:252-262).
+// The six matrices are loaded together before any product (__launch_bounds__
+// of one wave per SIMD in the kernels that use it): the kernels are bound by
+// L2 misses, and loads of one field at neighbouring sites find each other's
+// lines only when they are issued close together.  At 24^3x48 the link
+// construction took 4.58 ms with the loads spread between the products (three
+// waves per SIMD), 4.19 ms this way.
 __device__ __forceinline__ void add_staple(M3 &r, double sc, const double2 *I, const double2 *K, long V,
                                            const Geom &g, const Site &x, unsigned s, int mu, int nu) {
   const unsigned xpnu = nbr(g, x, nu, 1, mu, 0), xpmu = nbr(g, x, mu, 1, nu, 0);
   const unsigned xmnu = nbr(g, x, nu, -1, mu, 0), xmnupmu = nbr(g, x, nu, -1, mu, 1);
-  {
-    const M3 t = mm<false, true>(ld(I, V, xpnu), ld(K, V, xpmu));
-    axpy<false>(r, sc, mm<false, false>(ld(K, V, s), t));
-  }
-  {
-    const M3 t = mm<true, false>(ld(K, V, xmnu), ld(I, V, xmnu));
-    axpy<false>(r, sc, mm<false, false>(t, ld(K, V, xmnupmu)));
-  }
+  const M3 ip = ld(I, V, xpnu), im = ld(I, V, xmnu);
+  const M3 kp = ld(K, V, xpmu), km = ld(K, V, xmnu), k0 = ld(K, V, s), kmp = ld(K, V, xmnupmu);
+  __builtin_amdgcn_sched_barrier(0);
+  axpy<false>(r, sc, mm<false, false>(k0, mm<false, true>(ip, kp)));
+  axpy<false>(r, sc, mm<false, false>(mm<true, false>(km, im), kmp));
 }
 template <bool ACC, bool HASE, bool TWO = false>
 __global__ __launch_bounds__(TPB) void staple_kernel(Geom g, Sched q, long V, double2 *out, double sc, const double2 *I,
@@ -575,29 +579,135 @@ __global__ __launch_bounds__(TPB) void force_kernel(long V, double2 *F, const do
 
 // ---------------------------------------------------------------------------
 // Asqtad fattening (lib/asqtad_dslash_p.c:391-633, compute_gen_staple /
-// make_imp_links) on the same site-innermost fields and site order: each
-// generalised staple S(x) = K(x) I(x+nu) K(x+mu)^+ + K(x-nu)^+ I(x-nu) K(x-nu+mu)
-// (I the field along mu, K the link along nu) is one kernel that adds c S
-// to the fat link and, when the next smearing level needs it, stores S.
-template <bool STORE>
-__global__ __launch_bounds__(TPB) void fat_staple_kernel(Geom g, Sched q, long V, double2 *out, double2 *fat,
-                                                         double c, const double2 *I, const double2 *K,
-                                                         int mu, int nu) {
+// make_imp_links) on the same site-innermost fields and site order.  With
+// st_nu(I) = K(x) I(x+nu) K(x+mu)^+ + K(x-nu)^+ I(x-nu) K(x-nu+mu), K = U_nu,
+// linear in I, the sum over all paths is taken from the innermost staple out:
+//   T_tau = c5 U_mu + c7 st_tau(U_mu)
+//   R_nu  = c3 U_mu + cL st_nu(U_mu) + sum_{rho != mu,nu} st_rho(T_tau), tau the fourth direction
+//   F     = c1 U_mu + sum_nu st_nu(R_nu)
+// (the reference builds the outermost staple last, one path at a time): 15
+// staples per direction instead of 18, and three launches, each a pass over
+// the fields it needs once, instead of 18 that read and write the fat link.
+// Bytes per site and direction: (4 + 3) + (7 + 3) + (7 + 1) fields of 144 B
+// against 96; HBM-bound (3 flops per byte).
+// Measured per direction at 24^3x48: inner 209, middle 407, outer 198 us (L2 misses
+// at 6 TB/s), against nine staple passes of 117 us and nine of 99 us.
+template <bool HASE>
+__global__ __launch_bounds__(TPB, 1) void fat_inner_kernel(Geom g, Sched q, long V, Ptr4 U, MidPtr T, double c5, double c7,
+                                                        int mu) {
   const int s0 = site_index(q, g.Vh);
   if (s0 < 0) return;
   const unsigned s = (unsigned)s0;
   const Site x = site_of(g, s);
-  const unsigned xpnu = nbr(g, x, nu, 1, mu, 0), xpmu = nbr(g, x, mu, 1, nu, 0);
-  const unsigned xmnu = nbr(g, x, nu, -1, mu, 0), xmnupmu = nbr(g, x, nu, -1, mu, 1);
-  M3 r = mm<false, false>(ld(K, V, s), mm<false, true>(ld(I, V, xpnu), ld(K, V, xpmu)));
-  {
-    const M3 t = mm<true, false>(ld(K, V, xmnu), ld(I, V, xmnu));
-    axpy<false>(r, 1.0, mm<false, false>(t, ld(K, V, xmnupmu)));
+#pragma unroll 1
+  for (int tau = 0; tau < 4; tau++) {
+    if (tau == mu) continue;
+    M3 r = zero3();
+    add_staple(r, c7, U.p[mu], U.p[tau], V, g, x, s, mu, tau);
+    if constexpr (HASE) axpy<false>(r, c5, ld(U.p[mu], V, s));
+    st(T.p[tau], V, s, r);
   }
-  if constexpr (STORE) st_nt(out, V, s, r);
-  M3 f = ld_nt(fat, V, s);
-  axpy<false>(f, c, r);
-  st_nt(fat, V, s, f);
+}
+
+// One direction rho of fat_middle_kernel: staples along rho of A (into ra), B
+// (into rb) and, with the Lepage term, U_mu (into rl); the four links along
+// rho are loaded once for the three.
+template <bool HAS5, bool HASL>
+__device__ __forceinline__ void add_staples3(M3 &ra, M3 &rb, M3 &rl, double c, double cl, const double2 *A,
+                                             const double2 *B, const double2 *Um, const double2 *K, long V,
+                                             const Geom &g, const Site &x, unsigned s, int mu, int rho) {
+#define SB() __builtin_amdgcn_sched_barrier(0)
+  {
+    const unsigned xp = nbr(g, x, rho, 1, mu, 0);
+    const M3 k0 = ld(K, V, s), kp = ld(K, V, nbr(g, x, mu, 1, rho, 0));
+    if constexpr (HAS5) {
+      axpy<false>(ra, c, mm<false, false>(k0, mm<false, true>(ld(A, V, xp), kp)));
+      SB();
+      axpy<false>(rb, c, mm<false, false>(k0, mm<false, true>(ld(B, V, xp), kp)));
+      SB();
+    }
+    if constexpr (HASL) axpy<false>(rl, cl, mm<false, false>(k0, mm<false, true>(ld(Um, V, xp), kp)));
+  }
+  SB();
+  {
+    const unsigned xm = nbr(g, x, rho, -1, mu, 0);
+    const M3 km = ld(K, V, xm), kmp = ld(K, V, nbr(g, x, rho, -1, mu, 1));
+    if constexpr (HAS5) {
+      axpy<false>(ra, c, mm<false, false>(mm<true, false>(km, ld(A, V, xm)), kmp));
+      SB();
+      axpy<false>(rb, c, mm<false, false>(mm<true, false>(km, ld(B, V, xm)), kmp));
+      SB();
+    }
+    if constexpr (HASL) axpy<false>(rl, cl, mm<false, false>(mm<true, false>(km, ld(Um, V, xm)), kmp));
+  }
+  SB();
+#undef SB
+}
+
+// R of the three directions d0, d1, d2 other than mu in one pass.  T.p[d]: the
+// field whose staple along rho enters R of the third direction (U_mu itself,
+// scaled by c = c5, when there are no 7-link paths).  Three accumulators are
+// live (two waves per SIMD); with one launch per direction each T and U would
+// be read twice.
+template <bool HAS5, bool HASL>
+__global__ __launch_bounds__(TPB, 2) void fat_middle_kernel(Geom g, Sched q, long V, Ptr4 U, Ptr4 T, MidPtr R, double c3,
+                                                            double c, double cl, int mu, int d0, int d1, int d2) {
+  const int s0 = site_index(q, g.Vh);
+  if (s0 < 0) return;
+  const unsigned s = (unsigned)s0;
+  const Site x = site_of(g, s);
+  M3 r0 = zero3();
+  axpy<false>(r0, c3, ld(U.p[mu], V, s));
+  M3 r1 = r0, r2 = r0;
+  add_staples3<HAS5, HASL>(r1, r2, r0, c, cl, T.p[d2], T.p[d1], U.p[mu], U.p[d0], V, g, x, s, mu, d0);
+  add_staples3<HAS5, HASL>(r0, r2, r1, c, cl, T.p[d2], T.p[d0], U.p[mu], U.p[d1], V, g, x, s, mu, d1);
+  add_staples3<HAS5, HASL>(r0, r1, r2, c, cl, T.p[d1], T.p[d0], U.p[mu], U.p[d2], V, g, x, s, mu, d2);
+  st(R.p[d0], V, s, r0);
+  st(R.p[d1], V, s, r1);
+  st(R.p[d2], V, s, r2);
+}
+
+// F = c1 U_mu + c sum_nu st_nu(R_nu)
+__global__ __launch_bounds__(TPB, 1) void fat_outer_kernel(Geom g, Sched q, long V, double2 *F, Ptr4 U, Ptr4 R, double c1,
+                                                        double c, int mu) {
+  const int s0 = site_index(q, g.Vh);
+  if (s0 < 0) return;
+  const unsigned s = (unsigned)s0;
+  const Site x = site_of(g, s);
+  M3 r = zero3();
+  axpy<false>(r, c1, ld(U.p[mu], V, s));
+#pragma unroll 1
+  for (int nu = 0; nu < 4; nu++)
+    if (nu != mu) add_staple(r, c, R.p[nu], U.p[nu], V, g, x, s, mu, nu);
+  st(F, V, s, r);
+}
+
+// One direction of the double-stored links (layout of LinkSet) from a
+// site-innermost field f along mu, hops of d sites: block kf holds f(x) / 2,
+// block kb -f(x - d mu)^+ / 2.  A copy kernel: 144 B read (the shifted read
+// mostly from L2) and 288 B written per site, all runs contiguous; from the
+// raw layout the same took 1.2 ms at 24^3x48 for the eight link fields, now
+// 0.53 ms.
+__global__ __launch_bounds__(TPB) void store_links_kernel(Geom g, Sched q, long V, const double2 *f, double2 *out, int nl,
+                                                          int kf, int kb, int mu, int d) {
+  const int s0 = site_index(q, g.Vh);
+  if (s0 < 0) return;
+  const unsigned s = (unsigned)s0;
+  const Site x = site_of(g, s);
+  const long Vh = g.Vh;
+  const int p = s >= (unsigned)Vh;
+  const unsigned h = s - (p ? (unsigned)Vh : 0u);
+  M3 a = ld(f, V, s);
+#pragma unroll
+  for (int e = 0; e < 9; e++) a.e[e] = make_double2(0.5 * a.e[e].x, 0.5 * a.e[e].y);
+  st_nt(out + ((long)p * nl + kf) * 9 * Vh, Vh, h, a);
+  const M3 b = ld(f, V, nbr(g, x, mu, -d, 0, 0));
+  M3 o;
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) o.e[3 * i + j] = make_double2(-(0.5 * b.e[3 * j + i].x), 0.5 * b.e[3 * j + i].y);
+  st_nt(out + ((long)p * nl + kb) * 9 * Vh, Vh, h, o);
 }
 
 // Naik link L(x) = c U(x) U(x+mu) U(x+2mu) (lib/asqtad_dslash_p.c:600-620)
@@ -745,16 +855,17 @@ __global__ __launch_bounds__(TPB) void u3_deriv_kernel(long V, const double2 *Vr
 }
 
 inline dim3 grid(long n) { return dim3((unsigned)((n + TPB - 1) / TPB)); }
-// The schedule for a lattice: tiles of up to 4096 sites (whole blocks).
+// The schedule for a lattice: equal tiles of whole 128-position blocks (unequal
+// ones cost 12% at 12x18x20x28, where 2048 does not divide the slab of 5040).
 inline Sched make_sched(const Lattice *lat) {
   Sched q;
   q.L0 = lat->L[0];
   q.S = (int)(lat->Vh / q.L0);
-  const int Sb = (q.S + TPB - 1) / TPB * TPB;
-  q.T = Sb < 4096 ? Sb : 4096;
-  q.nt = (q.S + q.T - 1) / q.T;
-  q.bpt = q.T / TPB;
-  const long W = (long)q.nt * q.L0 * 2 * q.bpt;
+  const int H = TPB / 2;
+  q.nt = (q.S + 2047) / 2048;
+  q.T = ((q.S + q.nt - 1) / q.nt + H - 1) / H * H;
+  q.bpt = q.T / H;
+  const long W = (long)q.nt * q.L0 * q.bpt;
   q.per = (int)((W + 7) / 8);
   return q;
 }
@@ -1083,66 +1194,101 @@ void hisq_force_dev(const Lattice *lat, double *const U_raw[4], double *const V_
 
 // Asqtad fattening (lib/asqtad_dslash_p.c:391-633) of raw FP64 device links:
 // fat = coef1' U + sum of staples (coef1' = coef1 - 6 lepage, :531), lng =
-// naik U U U from gl; the order of accumulation is the reference's.
-void fatten_dev(const Lattice *lat, const double *const gf[4], const double *const gl[4],
-                const double c[6], double *fat_raw[4], double *lng_raw[4], hipStream_t st) {
+// naik U U U from gl, written raw (fat_raw, lng_raw) or, with dst given, as
+// its double-stored set.  dst changes only once every workspace is allocated.
+static void fatten_run(const Lattice *lat, const double *const gf[4], const double *const gl[4], const double c[6],
+                       double *const *fat_raw, double *const *lng_raw, Links *dst, hipStream_t st) {
   const long V = lat->V, n9 = 9 * V;
   if (V >= (1L << 27))
     throw std::runtime_error("fattening: lattice volume of 2^27 sites or more (32-bit offsets)");
   const Geom &g = lat->g;
   const double coef1 = c[0] - 6 * c[4], coef3 = c[1], coef5 = c[2], coef7 = c[3], coefL = c[4];
-  const bool have5 = coef5 != 0 || coef7 != 0 || coefL != 0;
-  const bool have3 = coef3 != 0 || have5;
-  const bool naik = lng_raw != nullptr;
+  const bool has5 = coef5 != 0 || coef7 != 0;
+  const bool hasR = has5 || coefL != 0;  // else F needs only the 3-staples of U
+  const bool have3 = coef3 != 0 || hasR;
+  const bool naik = dst ? c[5] != 0 : lng_raw != nullptr;
+  const int nl = naik ? 16 : 8, per = nl / 4;
   const bool sep_long = naik && (gl[0] != gf[0] || gl[1] != gf[1] || gl[2] != gf[2] || gl[3] != gf[3]);
   Fields buf(V);
-  auto take = [&] { return buf.take(); };
-  double2 *U[4], *UL[4], *F = take(), *S3 = nullptr, *S5 = nullptr, *Lk = nullptr;
-  for (auto &u : U) u = take();
-  if (have3) {
-    S3 = take();
-    S5 = take();
-  }
-  if (naik) Lk = take();
-  for (int i = 0; i < 4; i++) UL[i] = sep_long ? take() : U[i];
+  Ptr4 U{}, UL{}, T{}, R{};
+  MidPtr Tw{}, Rw{};
+  double2 *F = buf.take(), *Lk = naik ? buf.take() : nullptr;
   const Sched sq = make_sched(lat);
   const dim3 b(TPB), gs = grid(V), ge = grid(n9), gx(8 * sq.per);
+  double2 *uf[4], *ul[4];
   for (int mu = 0; mu < 4; mu++) {
-    hipLaunchKernelGGL(to_soa_kernel, gs, b, 0, st, (const double2 *)gf[mu], U[mu], V);
-    if (sep_long) hipLaunchKernelGGL(to_soa_kernel, gs, b, 0, st, (const double2 *)gl[mu], UL[mu], V);
+    uf[mu] = buf.take();
+    ul[mu] = sep_long ? buf.take() : uf[mu];
+    U.p[mu] = uf[mu];
+    UL.p[mu] = ul[mu];
   }
-  auto add = [&](bool store, double2 *out, double cc, const double2 *I, const double2 *K, int mu, int nu) {
-    if (store)
-      hipLaunchKernelGGL(fat_staple_kernel<true>, gx, b, 0, st, g, sq, V, out, F, cc, I, K, mu, nu);
-    else
-      hipLaunchKernelGGL(fat_staple_kernel<false>, gx, b, 0, st, g, sq, V, out, F, cc, I, K, mu, nu);
-  };
-  for (int dir = 0; dir < 4; dir++) {
-    hipLaunchKernelGGL(lincomb_kernel, ge, b, 0, st, F, 0.0, coef1, (const double2 *)U[dir], 0.0,
-                       (const double2 *)nullptr, n9);
-    if (have3) {
-      for (int nu = 0; nu < 4; nu++) {
-        if (nu == dir) continue;
-        add(true, S3, coef3, U[dir], U[nu], dir, nu);
-        if (coefL != 0) add(false, nullptr, coefL, S3, U[nu], dir, nu);
-        if (coef5 != 0 || coef7 != 0)
-          for (int rho = 0; rho < 4; rho++) {
-            if (rho == dir || rho == nu) continue;
-            add(coef7 != 0, S5, coef5, S3, U[rho], dir, rho);
-            if (coef7 != 0)
-              for (int sig = 0; sig < 4; sig++)
-                if (sig != dir && sig != nu && sig != rho) add(false, nullptr, coef7, S5, U[sig], dir, sig);
-          }
+  // three T and three R fields, placed by direction below
+  double2 *t3[3] = {}, *r3[3] = {};
+  for (int i = 0; i < 3; i++) {
+    if (coef7 != 0) t3[i] = buf.take();
+    if (hasR) r3[i] = buf.take();
+  }
+  double2 *links = nullptr;
+  if (dst) {
+    dst->lat = const_cast<Lattice *>(lat);
+    links64_alloc(*dst, nl);
+    links = (double2 *)dst->l64.data;
+  }
+  for (int mu = 0; mu < 4; mu++) {
+    hipLaunchKernelGGL(to_soa_kernel, gs, b, 0, st, (const double2 *)gf[mu], uf[mu], V);
+    if (sep_long) hipLaunchKernelGGL(to_soa_kernel, gs, b, 0, st, (const double2 *)gl[mu], ul[mu], V);
+  }
+  for (int mu = 0; mu < 4; mu++) {
+    int d[3], nd = 0;
+    for (int nu = 0; nu < 4; nu++)
+      if (nu != mu) {
+        T.p[nu] = coef7 != 0 ? t3[nd] : U.p[mu];
+        R.p[nu] = hasR ? r3[nd] : U.p[mu];
+        Tw.p[nu] = t3[nd];
+        Rw.p[nu] = r3[nd];
+        d[nd++] = nu;
       }
+    if (!have3) {
+      hipLaunchKernelGGL(lincomb_kernel, ge, b, 0, st, F, 0.0, coef1, U.p[mu], 0.0, (const double2 *)nullptr, n9);
+    } else {
+      if (coef7 != 0) {
+        if (coef5 != 0) hipLaunchKernelGGL(fat_inner_kernel<true>, gx, b, 0, st, g, sq, V, U, Tw, coef5, coef7, mu);
+        else hipLaunchKernelGGL(fat_inner_kernel<false>, gx, b, 0, st, g, sq, V, U, Tw, coef5, coef7, mu);
+      }
+      const double c5 = coef7 != 0 ? 1.0 : coef5;
+      if (has5 && coefL != 0)
+        hipLaunchKernelGGL((fat_middle_kernel<true, true>), gx, b, 0, st, g, sq, V, U, T, Rw, coef3, c5, coefL, mu, d[0], d[1], d[2]);
+      else if (has5)
+        hipLaunchKernelGGL((fat_middle_kernel<true, false>), gx, b, 0, st, g, sq, V, U, T, Rw, coef3, c5, coefL, mu, d[0], d[1], d[2]);
+      else if (hasR)
+        hipLaunchKernelGGL((fat_middle_kernel<false, true>), gx, b, 0, st, g, sq, V, U, T, Rw, coef3, c5, coefL, mu, d[0], d[1], d[2]);
+      hipLaunchKernelGGL(fat_outer_kernel, gx, b, 0, st, g, sq, V, F, U, R, coef1, hasR ? 1.0 : coef3, mu);
     }
-    hipLaunchKernelGGL(from_soa_kernel, gs, b, 0, st, (const double2 *)F, (double2 *)fat_raw[dir], V);
-    if (naik) {
-      hipLaunchKernelGGL(naik_link_kernel, gx, b, 0, st, g, sq, V, Lk, (const double2 *)UL[dir], c[5], dir);
-      hipLaunchKernelGGL(from_soa_kernel, gs, b, 0, st, (const double2 *)Lk, (double2 *)lng_raw[dir], V);
+    if (naik)
+      hipLaunchKernelGGL(naik_link_kernel, gx, b, 0, st, g, sq, V, Lk, UL.p[mu], c[5], mu);
+    if (links) {
+      hipLaunchKernelGGL(store_links_kernel, gx, b, 0, st, g, sq, V, (const double2 *)F, links, nl, per * mu,
+                         per * mu + per / 2, mu, 1);
+      if (naik)
+        hipLaunchKernelGGL(store_links_kernel, gx, b, 0, st, g, sq, V, (const double2 *)Lk, links, nl, per * mu + 1,
+                           per * mu + 3, mu, 3);
+    } else {
+      hipLaunchKernelGGL(from_soa_kernel, gs, b, 0, st, (const double2 *)F, (double2 *)fat_raw[mu], V);
+      if (naik) hipLaunchKernelGGL(from_soa_kernel, gs, b, 0, st, (const double2 *)Lk, (double2 *)lng_raw[mu], V);
     }
   }
   QOP_CHECK_HIP(hipGetLastError());
   QOP_CHECK_HIP(hipStreamSynchronize(st));
+}
+
+void fatten_dev(const Lattice *lat, const double *const gf[4], const double *const gl[4], const double c[6],
+                double *fat_raw[4], double *lng_raw[4], hipStream_t st) {
+  fatten_run(lat, gf, gl, c, fat_raw, lng_raw, nullptr, st);
+}
+
+void fatten_links64(const Lattice *lat, Links &L, const double *const gf[4], const double *const gl[4],
+                    const double c[6], hipStream_t st) {
+  fatten_run(lat, gf, gl, c, nullptr, nullptr, &L, st);
 }
 
 }  // namespace qop

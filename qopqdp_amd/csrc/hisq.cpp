@@ -191,17 +191,19 @@ HisqT *hisq_create(QOP_info_t *info, QOP_hisq_coeffs_t *c, GaugeT *gauge) {
   h->n_naiks = n_naiks;
   h->fn.assign(n_naiks, nullptr);
   const double *w[4] = {W.m[0], W.m[1], W.m[2], W.m[3]};
+  const bool naik2 = a2.naik != 0, naik_sets = n_naiks > 1 || g_hisq.want_deps;
+  double k2[6];
+  coef6(a2, k2);
+  flops += smear_flops(a2, lat);
   Raw4 fat2, lng2;
-  fat2.alloc(lat);
-  const bool naik2 = a2.naik != 0;
-  if (naik2) lng2.alloc(lat);
-  {
-    double k[6];
-    coef6(a2, k);
-    launch_fatten(lat, w, w, k, fat2.m, naik2 ? lng2.m : nullptr, st);
-    flops += smear_flops(a2, lat);
-  }
-  if (n_naiks > 1 || g_hisq.want_deps) {
+  if (!naik_sets) {
+    // the only set: smeared straight into its link object (owner frees it)
+    h->fn[0] = new LinksT;
+    fatten_links64(lat, h->fn[0]->L, w, w, k2, st);
+  } else {
+    fat2.alloc(lat);
+    if (naik2) lng2.alloc(lat);
+    launch_fatten(lat, w, w, k2, fat2.m, naik2 ? lng2.m : nullptr, st);
     // the "difference" set (hisq_links_p.c:195-221, 241-247)
     Raw4 fat3, lng3;
     fat3.alloc(lat);
@@ -231,10 +233,10 @@ HisqT *hisq_create(QOP_info_t *info, QOP_hisq_coeffs_t *c, GaugeT *gauge) {
     li.free();
     fat3.free();
     lng3.free();
+    h->fn[0] = links_from_raw_dev<LinksT>(lat, fat2, naik2 ? &lng2 : nullptr);
+    fat2.free();
+    lng2.free();
   }
-  h->fn[0] = links_from_raw_dev<LinksT>(lat, fat2, naik2 ? &lng2 : nullptr);
-  fat2.free();
-  lng2.free();
   if (aux) {
     for (int i = 0; i < 4; i++) {
       h->aux[0][i] = Uc.m[i];

@@ -48,20 +48,26 @@ __global__ void dblstore_kernel(Geom g, const double *const *fat,
   }
 }
 
+void links64_alloc(Links &L, int nl) {
+  const Lattice *lat = L.lat;
+  LinkSet &s = L.l64;
+  L.nl = nl;
+  // a reloaded object of the same lattice keeps its array
+  if (s.nl != nl || s.sites != lat->Vh) linkset_free(s);
+  L.drop_derived();
+  if (!s.data) dev_alloc(&s.data, (size_t)2 * nl * 9 * lat->Vh * sizeof(double2));
+  s.prec = P64;
+  s.nl = nl;
+  s.sites = lat->Vh;
+}
+
 void build_links64(Links &L, const double *fat_dev[4], const double *lng_dev[4],
                    hipStream_t st) {
   const Lattice *lat = L.lat;
-  L.nl = lng_dev ? 16 : 8;
+  links64_alloc(L, lng_dev ? 16 : 8);
   LinkSet &s = L.l64;
-  // a reloaded object of the same lattice keeps its array
-  if (s.nl != L.nl || s.sites != lat->Vh) linkset_free(s);
-  L.drop_derived();
   DevBuf<const double *> pbuf(8 * sizeof(double *));
   const double **ptrs = pbuf.p;
-  if (!s.data) dev_alloc(&s.data, (size_t)2 * L.nl * 9 * lat->Vh * sizeof(double2));
-  s.prec = P64;
-  s.nl = L.nl;
-  s.sites = lat->Vh;
   const double *hp[8];
   for (int i = 0; i < 4; i++) { hp[i] = fat_dev[i]; hp[4 + i] = lng_dev ? lng_dev[i] : nullptr; }
   QOP_CHECK_HIP(hipMemcpyAsync(ptrs, hp, sizeof hp, hipMemcpyHostToDevice, st));
