@@ -396,7 +396,7 @@ struct Mix {
   int m5acc;
 };
 template <bool ACC, bool HASB, int EPI = EPI_STORE>
-__global__ __launch_bounds__(TPB) void side_force_kernel(Geom g, Sched q, long V, double2 *force, double2 *stpl,
+__global__ __launch_bounds__(TPB, 1) void side_force_kernel(Geom g, Sched q, long V, double2 *force, double2 *stpl,
                                                          Lin bot, const double2 *side,
                                                          const double2 *top, int mu, int nu, Mix mx) {
   const int s0 = site_index(q, g.Vh);
@@ -404,34 +404,34 @@ __global__ __launch_bounds__(TPB) void side_force_kernel(Geom g, Sched q, long V
   const unsigned s = (unsigned)s0;
   const Site x = site_of(g, s);
   const unsigned xpmu = nbr(g, x, mu, 1, nu, 0), xpnu = nbr(g, x, nu, 1, mu, 0);
-  // SB() keeps the scheduler from hoisting every matrix load to the top:
-  // with all 14 in flight a thread needs ~500 registers (one wave per SIMD).
+  // The matrices of a group of terms (+mu, -mu, the lower staple) are loaded
+  // together before its products, with one wave per SIMD: the kernel is bound
+  // by L2 misses, and the loads of one field at x and a neighbour share lines
+  // only when they are issued close together.  Fewer loads in flight (SB()
+  // between all of them, two waves per SIMD, 216 registers) took 15.2 ms per
+  // asqtad force of 8 terms at 24^3x48, this 13.7; all 14 at once spill.  A
+  // variant that walks along mu and carries the -mu terms halves the loads but
+  // serialises their latency: 14.2 ms there, and slower on small lattices.
   // B(x+nu) S(x+mu)^+ and S(x+mu) are loaded once and serve both the force
   // terms at +mu and the staple; the staple is formed last, after the force
   // is stored, so its epilogue (EPI) has the registers of the force terms.
 #define SB() __builtin_amdgcn_sched_barrier(0)
   M3 f, bs;
   {
-    const M3 Smu = ld(side, V, xpmu);
-    bs = mm<false, true>(ld<HASB>(bot, V, xpnu), Smu);  // B(x+nu) S(x+mu)^+
+    const M3 Bn = ld<HASB>(bot, V, xpnu), Sp = ld(side, V, xpmu);
+    const M3 T = ld(top, V, s), Tn = ld(top, V, xpnu), B = ld<HASB>(bot, V, s);
     SB();
-    f = mm<false, true>(ld(top, V, s), bs);  // T S(x+mu) B(x+nu)^+
-    SB();
-    const M3 b2 = mm<false, false>(ld<HASB>(bot, V, s), Smu);  // B(x) S(x+mu)
-    SB();
-    axpy<false>(f, 1.0, mm<false, true>(b2, ld(top, V, xpnu)));
+    bs = mm<false, true>(Bn, Sp);  // B(x+nu) S(x+mu)^+
+    f = mm<false, true>(T, bs);    // T S(x+mu) B(x+nu)^+
+    axpy<false>(f, 1.0, mm<false, true>(mm<false, false>(B, Sp), Tn));
   }
-  SB();
   {
     const unsigned xmmu = nbr(g, x, mu, -1, nu, 0), xmmupnu = nbr(g, x, mu, -1, nu, 1);
-    const M3 Sm = ld(side, V, xmmu);
-    const M3 t1 = mm<true, false>(ld<HASB>(bot, V, xmmu), Sm);  // B(x-mu)^+ S(x-mu)
+    const M3 Bm = ld<HASB>(bot, V, xmmu), Bmn = ld<HASB>(bot, V, xmmupnu);
+    const M3 Tm = ld(top, V, xmmu), Tmn = ld(top, V, xmmupnu), Sm = ld(side, V, xmmu);
     SB();
-    axpy<false>(f, 1.0, mm<false, false>(t1, ld(top, V, xmmupnu)));
-    SB();
-    const M3 t2 = mm<true, false>(ld(top, V, xmmu), Sm);  // T(x-mu)^+ S(x-mu)
-    SB();
-    axpy<false>(f, 1.0, mm<false, false>(t2, ld<HASB>(bot, V, xmmupnu)));
+    axpy<false>(f, 1.0, mm<false, false>(mm<true, false>(Bm, Sm), Tmn));  // B(x-mu)^+ S(x-mu) T
+    axpy<false>(f, 1.0, mm<false, false>(mm<true, false>(Tm, Sm), Bmn));  // T(x-mu)^+ S(x-mu) B
   }
   SB();
   axpy<false>(f, 1.0, ld_nt(force, V, s));
@@ -439,11 +439,11 @@ __global__ __launch_bounds__(TPB) void side_force_kernel(Geom g, Sched q, long V
   SB();
   {
     const unsigned xmnu = nbr(g, x, nu, -1, mu, 0), xmnupmu = nbr(g, x, nu, -1, mu, 1);
-    M3 sp = mm<false, false>(ld(side, V, s), bs);
+    const M3 S0 = ld(side, V, s), Sd = ld(side, V, xmnu), Sdp = ld(side, V, xmnupmu);
+    const M3 Bd = ld<HASB>(bot, V, xmnu);
     SB();
-    const M3 t = mm<true, false>(ld(side, V, xmnu), ld<HASB>(bot, V, xmnu));
-    SB();
-    axpy<false>(sp, 1.0, mm<false, false>(t, ld(side, V, xmnupmu)));
+    M3 sp = mm<false, false>(S0, bs);
+    axpy<false>(sp, 1.0, mm<false, false>(mm<true, false>(Sd, Bd), Sdp));
     if constexpr (ACC) axpy<false>(sp, 1.0, ld_nt(stpl, V, s));
     if constexpr (EPI == EPI_FIN) {
       SB();
@@ -503,23 +503,31 @@ __global__ __launch_bounds__(TPB) void naik_deriv_kernel(Geom g, Sched q, long V
 }
 
 // Lepage fix-up (lib/asqtad_force_fnmat_p.c:317-339), first half:
-// acc(x) = sum_{nu != mu} [q_nu(x) + q_nu(x)^+], q_nu(x) = m_nu(x) U_nu(x)^+ - m_nu(x-nu)^+ U_nu(x-nu)
-__global__ __launch_bounds__(TPB) void lepage_acc_kernel(Geom g, Sched q, long V, double2 *acc, Ptr4 U,
-                                                         Ptr4 m, int mu) {
+// acc_mu(x) = sum_{nu != mu} [q_nu(x) + q_nu(x)^+], q_nu(x) = m_nu(x) U_nu(x)^+ - m_nu(x-nu)^+ U_nu(x-nu),
+// all four mu in one pass (each q_nu is formed once instead of three times:
+// 20 matrices per site instead of 52).
+__global__ __launch_bounds__(TPB, 1) void lepage_acc_kernel(Geom g, Sched q, long V, MidPtr acc, Ptr4 U, Ptr4 m) {
   const int s0 = site_index(q, g.Vh);
   if (s0 < 0) return;
   const unsigned s = (unsigned)s0;
   const Site x = site_of(g, s);
-  M3 r = zero3();
+  M3 r[4];
+#pragma unroll
+  for (int mu = 0; mu < 4; mu++) r[mu] = zero3();
+#pragma unroll
   for (int nu = 0; nu < 4; nu++) {
-    if (nu == mu) continue;
     const unsigned b = nbr(g, x, nu, -1, 0, 0);
     M3 t = mm<false, true>(ld(m.p[nu], V, s), ld(U.p[nu], V, s));
     axpy<false>(t, -1.0, mm<true, false>(ld(m.p[nu], V, b), ld(U.p[nu], V, b)));
-    axpy<false>(r, 1.0, t);
-    axpy<true>(r, 1.0, t);
+    M3 h = t;
+    axpy<true>(h, 1.0, t);
+#pragma unroll
+    for (int mu = 0; mu < 4; mu++)
+      if (mu != nu) axpy<false>(r[mu], 1.0, h);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  st(acc, V, s, r);
+#pragma unroll
+  for (int mu = 0; mu < 4; mu++) st_nt(acc.p[mu], V, s, r[mu]);
 }
 
 // second half: D(x) += cf [acc(x) U(x) - U(x) acc(x+mu)]
@@ -1101,11 +1109,11 @@ void ForceRun::deriv(double2 *const U[4], double2 *D[4], const double coef[6], d
   if (coefL != 0) {
     // Lepage fix-up (:317-339)
     const Ptr4 Up = {{U[0], U[1], U[2], U[3]}}, Mp = {{mid[0], mid[1], mid[2], mid[3]}};
-    for (int mu = 0; mu < 4; mu++) {
-      hipLaunchKernelGGL(lepage_acc_kernel, gx_, b_, 0, st_, g_, sq_, V_, mid3, Up, Mp, mu);
+    const MidPtr acc = {{stpl3[0], stpl3[1], stpl3[2], stpl3[3]}};  // free by now
+    hipLaunchKernelGGL(lepage_acc_kernel, gx_, b_, 0, st_, g_, sq_, V_, acc, Up, Mp);
+    for (int mu = 0; mu < 4; mu++)
       hipLaunchKernelGGL(lepage_apply_kernel, gx_, b_, 0, st_, g_, sq_, V_, D[mu], (const double2 *)U[mu],
-                         (const double2 *)mid3, -coefL, mu);
-    }
+                         (const double2 *)acc.p[mu], -coefL, mu);
     nfl += 4 * (3 * (2 * 198 + 3 * 18) + 198 + 216 + 36);
   }
   // Naik part (lib/asqtad_force_fnmat_p.c:395-445)
