@@ -54,6 +54,11 @@ struct HopArgs {
 };
 void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
                      bool hasx, hipStream_t st);
+// One-RHS hop of the reference path (FP64 / FP32 vectors, no batch masks):
+// launches the four-wave kernel or the one-thread-per-site kernel, whichever
+// suits the lattice; with b, the hop onto the other parity in the same launch.
+void launch_hop_one(const HopArgs &a, const HopArgs *b, int prec, int nl, int red, bool hasx,
+                    hipStream_t st);
 
 // out[b] = sum_i c_i v_i[b] (complex c_i; coef device [n][3][2] or host cr/ci)
 struct LincombArgs {

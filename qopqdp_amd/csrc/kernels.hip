@@ -731,6 +731,37 @@ hop_kernel(const HopArgs a) {
   }
 }
 
+// What changes in the arguments of a one-RHS hop for the other parity
+// (blockIdx.y = 1): byte offsets of its pointers.  Added to a copy in scalar
+// registers; choosing between two argument blocks by reference would put them
+// in scratch memory.
+struct PairOffs {
+  long links, bck, src, dst, x;
+};
+__device__ __forceinline__ void hop_other_parity(HopArgs &a, const PairOffs &o) {
+  if (blockIdx.y == 0) return;
+  a.parity ^= 1;
+  a.links = (const char *)a.links + o.links;
+  a.links_bck = (const char *)a.links_bck + o.bck;
+  a.src.data = (char *)a.src.data + o.src;
+  a.dst.data = (char *)a.dst.data + o.dst;
+  a.x.data = (char *)a.x.data + o.x;
+}
+static PairOffs pair_offs(const HopArgs &a, const HopArgs &b) {
+  auto d = [](const void *p, const void *q) { return (long)((intptr_t)q - (intptr_t)p); };
+  return {d(a.links, b.links), d(a.links_bck, b.links_bck), d(a.src.data, b.src.data), d(a.dst.data, b.dst.data),
+          d(a.x.data, b.x.data)};
+}
+
+// The hops onto both parities (mass term, no reduction) in one launch.
+template <int P, int NL, bool SGL, bool BUF>
+__global__ void __launch_bounds__(256)
+hop_pair_kernel(const HopArgs a0, const PairOffs o) {
+  HopArgs a = a0;
+  hop_other_parity(a, o);
+  hop_group<P, NL, 1, RED_NONE, true, false, SGL, false, P, BUF>(a, 0, -1);
+}
+
 int hop_partial_blocks(const Lattice *lat) { return (int)((lat->Vh + 63) / 64); }
 
 // LDS bytes of a staged block: NB RHS x blockDim sites x (3 stored complex
@@ -849,6 +880,17 @@ static void hop_dispatch_nb(const HopArgs &a, int nb, dim3 grid, dim3 block,
   }
 }
 
+// buffer loads (FP32 / FP16, double-stored links) where every byte offset
+// from the RHS group's first vector / norm and from a direction's first
+// link stays below 2^31
+static bool hop_buf_fits(const HopArgs &a, int prec, int nb) {
+  const long lim = 1L << 31, Vh = a.g.Vh;
+  const long esz = prec == P16 ? 4 : 8;   // stored vector element
+  const long lesz = prec == P32 ? 8 : 4;  // stored link element (P32H: FP16 links)
+  return prec != P64 && !a.single && !a.plain && ((long)(nb - 1) * a.sstride + 3 * Vh) * esz < lim &&
+         ((long)(nb - 1) * a.nstride + Vh) * 4 < lim && 9 * Vh * lesz < lim;
+}
+
 void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
                      bool hasx, hipStream_t st) {
   QOP_REQUIRE(nb == 1 || nb == 2 || nb == 4 || nb == 8 || nb == 16, "hop: rhs per thread must be 1,2,4,8,16");
@@ -878,22 +920,13 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
     const int slab = a.g.Vh / a.g.L[0];
     QOP_REQUIRE(a.tile % block == 0 && slab % a.tile == 0, "hop: tile must divide the x0 slab");
   }
-  // buffer loads (FP32 / FP16, double-stored links) where every byte offset
-  // from the RHS group's first vector / norm and from a direction's first
-  // link stays below 2^31; otherwise (or when a.plain asks for it) one RHS
-  // per thread with plain loads
-  {
-    const long lim = 1L << 31, Vh = a.g.Vh;
-    const long esz = prec == P16 ? 4 : 8;   // stored vector element
-    const long lesz = prec == P32 ? 8 : 4;  // stored link element (P32H: FP16 links)
-    a.buf = prec != P64 && !a.single && !a.plain && ((long)(nb - 1) * a.sstride + 3 * Vh) * esz < lim &&
-            ((long)(nb - 1) * a.nstride + Vh) * 4 < lim && 9 * Vh * lesz < lim;
-    if (prec != P64 && !a.single && !a.buf) {
-      nb = 1;
-      a.stage = 0;
-      a.nt = 0;
-      if (block > 256) block = 256;
-    }
+  // otherwise (or when a.plain asks for it) one RHS per thread with plain loads
+  a.buf = hop_buf_fits(a, prec, nb);
+  if (prec != P64 && !a.single && !a.buf) {
+    nb = 1;
+    a.stage = 0;
+    a.nt = 0;
+    if (block > 256) block = 256;
   }
   int nblk = (a.g.Vh + block - 1) / block;
   a.ngroups = (a.n + nb - 1) / nb;
@@ -921,6 +954,181 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
     if (nl == 16) hop_dispatch_nb<P16, 16>(a, nb, grid, blk, red, hasx, st);
     else hop_dispatch_nb<P16, 8>(a, nb, grid, blk, red, hasx, st);
   }
+  QOP_CHECK_HIP(hipGetLastError());
+}
+
+// ---------------------------------------------------------------------------
+// One-RHS hop with four waves per 64 sites: wave mu forms the terms of
+// direction mu, the four partial sums meet in LDS and waves 0..2 finish colour
+// 0..2 (epilogue and reduction as hop_epilogue, chunk sums in the same 64-site
+// chunks).  For lattices that cannot fill the chip with one thread per site:
+// a wave loads 4 of a site's 16 links, all at once, instead of walking all 16,
+// and there are four times as many waves.  Where one wave per SIMD of the
+// one-thread-per-site kernel already reaches the memory rate it gains nothing.
+template <int P, int NL, int RED, bool HASX, bool SGL>
+__global__ void __launch_bounds__(256)
+hop_split_kernel(const HopArgs a0, const PairOffs o2) {
+  using R = typename PT<P>::R;
+  using S = typename PT<P>::S;
+  __shared__ R part[4][6][64];
+  __shared__ double rsum[3];
+  HopArgs a = a0;
+  hop_other_parity(a, o2);
+  if (a.status && *a.status != 0) return;
+  const Geom g = a.g;
+  const int Vh = g.Vh;
+  const int mu = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+  const int chunk = logical_block(a.remap), h = chunk * 64 + lane;
+  R acc[6];
+#pragma unroll
+  for (int i = 0; i < 6; i++) acc[i] = 0;
+  if (h < Vh) {
+    constexpr int PER = NL / 4, HP = PER / 2;
+    int x[4], lex;
+    site_coords(g, h, a.parity, x, lex);
+    // element planes are uniform, the site a 32-bit byte offset
+    auto at = [&](const void *base, long plane, int site) {
+      return *(const S *)((const char *)base + plane * Vh * (long)sizeof(S) + (unsigned)site * (unsigned)sizeof(S));
+    };
+    // this wave's direction, selected (an index into x or g.L would put them
+    // in scratch memory)
+    const int Lm = mu == 0 ? g.L[0] : mu == 1 ? g.L[1] : mu == 2 ? g.L[2] : g.L[3];
+    const int sm = mu == 0 ? g.stride[0] : mu == 1 ? g.stride[1] : mu == 2 ? g.stride[2] : g.stride[3];
+    const int xm = mu == 0 ? x[0] : mu == 1 ? x[1] : mu == 2 ? x[2] : x[3];
+    S u_[PER][9], v_[PER][3];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const int d = PER == 4 ? (j == 0 ? 1 : j == 1 ? 3 : j == 2 ? -1 : -3) : (j == 0 ? 1 : -1);
+      const int y = xm + d;
+      const int nb = (lex + (y >= Lm ? d - Lm : y < 0 ? d + Lm : d) * sm) >> 1;
+      const bool fwd = !SGL || j < HP;
+      const long k = SGL ? HP * mu + (fwd ? j : j - HP) : PER * mu + j;
+#pragma unroll
+      for (int e = 0; e < 9; e++) u_[j][e] = at(fwd ? a.links : a.links_bck, 9 * k + e, fwd ? h : nb);
+#pragma unroll
+      for (int c = 0; c < 3; c++) v_[j][c] = at(a.src.data, c, nb);
+    }
+    // all loads of the direction in flight before the first product
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const bool fwd = !SGL || j < HP;
+      const S(&u)[9] = u_[j];
+      const S(&v)[3] = v_[j];
+#pragma unroll
+      for (int r = 0; r < 3; r++) {
+        R re = acc[2 * r], im = acc[2 * r + 1];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          // single-stored backward term: -U(x-d)^dagger
+          const R wr = fwd ? u[3 * r + c].x : -u[3 * c + r].x, wi = fwd ? u[3 * r + c].y : u[3 * c + r].y;
+          re = fma(wr, v[c].x, re);
+          re = fma(-wi, v[c].y, re);
+          im = fma(wr, v[c].y, im);
+          im = fma(wi, v[c].x, im);
+        }
+        acc[2 * r] = re;
+        acc[2 * r + 1] = im;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 6; i++) part[mu][i][lane] = acc[i];
+  __syncthreads();
+  if (mu < 3) {
+    double red = 0;
+    if (h < Vh) {
+      const int c = mu;
+      const R al = (R)a.alpha, be = (R)a.beta;
+      R o[2], xv[2] = {0, 0};
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int k = 2 * c + i;
+        o[i] = al * (((part[0][k][lane] + part[1][k][lane]) + part[2][k][lane]) + part[3][k][lane]);
+      }
+      const long own = (long)c * Vh + h;
+      if constexpr (HASX) {
+        const S t = ((const S *)a.x.data)[own];
+        xv[0] = t.x;
+        xv[1] = t.y;
+        o[0] = fma(be, xv[0], o[0]);
+        o[1] = fma(be, xv[1], o[1]);
+      }
+      S *dst = (S *)a.dst.data;
+      if constexpr (RED == RED_R) {
+        const double alr = *a.cg_alpha;
+        const S t = dst[own];
+        o[0] = (R)fma(-alr, (double)o[0], (double)t.x);
+        o[1] = (R)fma(-alr, (double)o[1], (double)t.y);
+      }
+      S t;
+      t.x = o[0];
+      t.y = o[1];
+      dst[own] = t;
+      if constexpr (RED == RED_X2) red = (double)xv[0] * (double)xv[0] + (double)xv[1] * (double)xv[1];
+      else red = (double)o[0] * (double)o[0] + (double)o[1] * (double)o[1];
+    }
+    if constexpr (RED != RED_NONE) {
+      const double s = wave_sum(red);
+      if (lane == 0) rsum[mu] = s;
+    }
+  }
+  if constexpr (RED != RED_NONE) {
+    __syncthreads();
+    if (threadIdx.x == 0 && (long)chunk * 64 < Vh) a.partial[chunk] = (rsum[0] + rsum[1]) + rsum[2];
+  }
+}
+
+template <int P, int NL, bool SGL>
+static void hop_split_launch(const HopArgs &a, const PairOffs &b, dim3 grid, int red, bool hasx, hipStream_t st) {
+#define QOP_LAUNCH(RD, HX) hipLaunchKernelGGL((hop_split_kernel<P, NL, RD, HX, SGL>), grid, dim3(256), 0, st, a, b)
+  if (red == RED_NONE) { if (hasx) QOP_LAUNCH(RED_NONE, true); else QOP_LAUNCH(RED_NONE, false); }
+  else if (red == RED_OUT2) QOP_LAUNCH(RED_OUT2, false);
+  else if (red == RED_R) QOP_LAUNCH(RED_R, true);
+  else QOP_LAUNCH(RED_X2, true);
+#undef QOP_LAUNCH
+}
+
+static void launch_hop_pair(const HopArgs &a0, const HopArgs &b0, int prec, int nl, hipStream_t st) {
+  HopArgs a = a0;
+  a.buf = hop_buf_fits(a, prec, 1);
+  a.ngroups = 1;
+  const PairOffs b = pair_offs(a0, b0);
+  const int nblk = ((a.g.Vh + 255) / 256 + 7) / 8 * 8;
+  const dim3 grid(nblk, 2), blk(256);
+#define QOP_PAIR(P_, NL_)                                                                                     \
+  do {                                                                                                        \
+    if (a.single) hipLaunchKernelGGL((hop_pair_kernel<P_, NL_, true, false>), grid, blk, 0, st, a, b);        \
+    else if (a.buf) hipLaunchKernelGGL((hop_pair_kernel<P_, NL_, false, P_ != P64>), grid, blk, 0, st, a, b); \
+    else hipLaunchKernelGGL((hop_pair_kernel<P_, NL_, false, false>), grid, blk, 0, st, a, b);                \
+  } while (0)
+  if (prec == P64) { if (nl == 16) QOP_PAIR(P64, 16); else QOP_PAIR(P64, 8); }
+  else { if (nl == 16) QOP_PAIR(P32, 16); else QOP_PAIR(P32, 8); }
+#undef QOP_PAIR
+  QOP_CHECK_HIP(hipGetLastError());
+}
+
+void launch_hop_one(const HopArgs &a, const HopArgs *b, int prec, int nl, int red, bool hasx, hipStream_t st) {
+  QOP_REQUIRE(prec == P64 || prec == P32, "hop: the reference path has FP64 or FP32 vectors");
+  QOP_REQUIRE(a.n == 1 && !a.coef && !a.active && !a.slots && red != RED_CG, "hop: one unmasked RHS");
+  // Solves, one thread per site / four waves (ms): FP64 8^3x16 4.2 / 3.2,
+  // 12^3x24 6.0 / 5.4, 16^3x24 8.3 / 8.4, 16^3x32 13.0 / 13.3; FP32 8^3x16
+  // 2.5 / 1.9, 16^3x32 4.5 / 4.2, 16^2x20x32 5.1 / 5.1, 20^3x32 5.9 / 6.3
+  const int lim = prec == P64 ? 49152 : 81920;
+  if (a.g.Vh > lim || (red == RED_OUT2 && hasx)) {
+    if (b) launch_hop_pair(a, *b, prec, nl, st);
+    else launch_hop_args(a, prec, nl, 1, 256, red, hasx, st);
+    return;
+  }
+  const int nblk = (((a.g.Vh + 63) / 64) + 7) / 8 * 8;
+  dim3 grid(nblk, b ? 2 : 1);
+  const PairOffs b2 = pair_offs(a, b ? *b : a);
+#define QOP_SPLIT(P_, NL_) \
+  do { if (a.single) hop_split_launch<P_, NL_, true>(a, b2, grid, red, hasx, st); \
+       else hop_split_launch<P_, NL_, false>(a, b2, grid, red, hasx, st); } while (0)
+  if (prec == P64) { if (nl == 16) QOP_SPLIT(P64, 16); else QOP_SPLIT(P64, 8); }
+  else { if (nl == 16) QOP_SPLIT(P32, 16); else QOP_SPLIT(P32, 8); }
+#undef QOP_SPLIT
   QOP_CHECK_HIP(hipGetLastError());
 }
 

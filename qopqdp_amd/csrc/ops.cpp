@@ -34,9 +34,8 @@ void set_hop_links(HopArgs &a, Links &L, int prec, int out_parity) {
   }
 }
 
-void hop(Links &L, int prec, DevVec &dst, int out_parity, const DevVec &src,
-         double alpha, double beta, const DevVec *x, int red, double *dev_result,
-         hipStream_t st, const int *status) {
+static HopArgs hop_args(Links &L, int prec, DevVec &dst, int out_parity, const DevVec &src,
+                        double alpha, double beta, const DevVec *x) {
   Lattice *lat = L.lat;
   QOP_REQUIRE(dst.prec == prec && src.prec == prec && (!x || x->prec == prec),
               "hop: precision mismatch");
@@ -50,10 +49,17 @@ void hop(Links &L, int prec, DevVec &dst, int out_parity, const DevVec &src,
   a.n = 1;
   a.alpha = alpha;
   a.beta = beta;
+  return a;
+}
+
+void hop(Links &L, int prec, DevVec &dst, int out_parity, const DevVec &src,
+         double alpha, double beta, const DevVec *x, int red, double *dev_result,
+         hipStream_t st, const int *status) {
+  HopArgs a = hop_args(L, prec, dst, out_parity, src, alpha, beta, x);
   a.status = status;
-  int nch = hop_partial_blocks(lat);
+  int nch = hop_partial_blocks(L.lat);
   if (red != RED_NONE) a.partial = red_partial(nch);
-  launch_hop_args(a, prec, L.nl, 1, 256, red, x != nullptr, st);
+  launch_hop_one(a, nullptr, prec, L.nl, red, x != nullptr, st);
   if (red != RED_NONE) launch_finalize(a.partial, nch, 1, dev_result, st, status);
 }
 
@@ -78,7 +84,11 @@ void dslash(Links &L, double mass, DevVec &out, const DevVec &in, int eo_out, in
   auto hop_only = [&](int par) { hop(L, prec, out, par, *src, 1.0, 0.0, nullptr, RED_NONE, nullptr, st); };
   auto hop_mass = [&](int par) { hop(L, prec, out, par, *src, 1.0, mass, src, RED_NONE, nullptr, st); };
   if (eo_in == eo_out) {
-    if (eo_out == 2) { hop_mass(0); hop_mass(1); }
+    if (eo_out == 2) {  // both parities in one launch
+      const HopArgs a = hop_args(L, prec, out, 0, *src, 1.0, mass, src);
+      const HopArgs b = hop_args(L, prec, out, 1, *src, 1.0, mass, src);
+      launch_hop_one(a, &b, prec, L.nl, RED_NONE, true, st);
+    }
     else mass_only(eo_out);
   } else {
     if (eo_out == 0 || eo_out == 2) {

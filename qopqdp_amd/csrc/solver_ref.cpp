@@ -166,9 +166,9 @@ class CgmsRun {
  private:
   void iteration() {
     hipStream_t st = stream();
-    launch_hop_args(a1_, prec_, nl_, 1, 256, RED_OUT2, false, st);
+    launch_hop_one(a1_, nullptr, prec_, nl_, RED_OUT2, false, st);
     cgms_launch_scalarA(B.d, B.nch, st);
-    launch_hop_args(a2_, prec_, nl_, 1, 256, RED_R, true, st);
+    launch_hop_one(a2_, nullptr, prec_, nl_, RED_R, true, st);
     if (with_rel_) {  // the relative residual needs x first
       cgms_launch_xp(B.d, prec_, Vh_, r_, ns_, CGMS_X, st);
       cgms_launch_relnorm(B.d, prec_, Vh_, r_, xrel_, st);
