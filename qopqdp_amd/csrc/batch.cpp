@@ -207,10 +207,9 @@ BatchSolver::BatchSolver(Links &L, int eo, int capacity, int sloppy_prec, double
     sel_ = active_ + cap_;
     host_alloc(&active_h_, 2 * cap_ * sizeof(int));
     sel_h_ = active_h_ + cap_;
-    dev_alloc(&ru_, (3 * cap_ + 1) * sizeof(int));
+    dev_alloc(&ru_, 2 * cap_ * sizeof(int));
     ru_cont_ = ru_ + cap_;
-    slots_ = ru_ + 2 * cap_;
-    QOP_CHECK_HIP(hipMemsetAsync(ru_, 0, (3 * cap_ + 1) * sizeof(int), st_));
+    QOP_CHECK_HIP(hipMemsetAsync(ru_, 0, 2 * cap_ * sizeof(int), st_));
     dev_alloc(&glob_, sizeof(BsGlobal));
     host_alloc(&glob_h_, sizeof(BsGlobal));
     dev_alloc(&partA_, 3 * (size_t)cap_ * nch_ * sizeof(double));
@@ -306,11 +305,11 @@ static void batch_lincomb(Lattice *lat, int cap, const DevBatch &out, int nin, c
   launch_lincomb(a, out.prec, pin, nin, partial != nullptr, st);
 }
 
-void BatchSolver::apply_A64(const int *mask, bool listed) {
+void BatchSolver::apply_A64(const int *mask, bool update) {
   hipStream_t st = st_;
   LinkSet &ls = L_.get(P64);
   const int opp = 1 - eo_;
-  HopArgs a;
+  HopFlagArgs a;
   a.g = lat_->g;
   a.parity = opp;
   a.links = ls.parity_data(lat_, opp);
@@ -320,14 +319,20 @@ void BatchSolver::apply_A64(const int *mask, bool listed) {
   a.sstride = a.dstride = a.xstride = 3 * lat_->Vh;
   a.nstride = lat_->Vh;
   a.n = cap_;
-  // the flagged slots, compacted into consecutive RHS of the launch, so k of
-  // them take ceil(k / RHS per thread) link reads wherever they sit in the
-  // batch; the groups past them read nothing
-  if (!listed) bs_launch_compact(mask, cap_, slots_, st);
-  a.slots = slots_;
+  // the flagged slots are consecutive RHS of the launch, so k of them take
+  // ceil(k / RHS per thread) link reads wherever they sit in the batch; the
+  // groups past them read nothing
+  a.flags = mask;
+  // x + xs: formed in the first hop's gathers, which read the FP32 increments
+  // 16 times per site instead of once, or in a pass of its own, a launch more.
+  // Masked first hop and pass per iteration: 16^3x32, 24 slots 34 against
+  // 39 us; 24^3x48, 16 slots 67 against 60 us
+  const bool sadd = update && lat_->Vh <= 131072;
+  if (update && !sadd) bs_launch_ru_x(mask, cap_, (int)lat_->Vh, x64_.slot(0), xs_.slot(0), 3 * lat_->Vh, st);
+  a.src_add = xs_.data;
   ru_shape_.apply(a);
-  launch_hop_args(a, P64, ls.nl, ru_shape_.nb, ru_shape_.block, RED_NONE, false, st);
-  HopArgs b = a;
+  launch_hop_flagged(a, ls.nl, ru_shape_.nb, ru_shape_.block, sadd ? RED_SADD : RED_NONE, false, st);
+  HopFlagArgs b = a;
   b.parity = eo_;
   b.links = ls.parity_data(lat_, eo_);
   b.lscale = ls.parity_scale(lat_, eo_);
@@ -335,7 +340,17 @@ void BatchSolver::apply_A64(const int *mask, bool listed) {
   b.dst = ax64_.slot(0);
   b.x = x64_.slot(0);
   b.coef = coef_;
-  launch_hop_args(b, P64, ls.nl, ru_shape_.nb, ru_shape_.block, RED_NONE, true, st);
+  if (update) {
+    b.xs64 = sadd ? xs_.data : nullptr;
+    b.b64 = b64_.data;
+    b.rs = rs_.slot(0);
+    b.ps = ps_.slot(0);
+    b.r2 = partA_;
+    b.re = partB_;
+    b.im = partC_;
+  }
+  launch_hop_flagged(b, ls.nl, ru_shape_.nb, ru_shape_.block,
+                  !update ? RED_NONE : sp_ == P16 ? RED_RU16 : RED_RU32, true, st);
 }
 
 void BatchSolver::load(int slot, const DevVec &src, const DevVec *x0, double mass, double tol,
@@ -490,21 +505,12 @@ void BatchSolver::enqueue_iteration() {
   launch_hop_args(b, sp_, ls.nl, shape2_.nb, shape2_.block, RED_CG, true, st);
   bs_launch_scalar2(rhs_, active_, glob_, partC_, nch_, cap_, ru_, st);
   if (join_ > 0) bs_launch_ru_join(rhs_, active_, ru_, cap_, st);
-  bs_launch_pupdate(rhs_, active_, &glob_->status, sp_, (int)Vh, rs_.slot(0), ps_.slot(0), 3 * Vh, cap_, 1,
-                    partB_, st);
-  // reliable update of the flagged slots, all on the device, over their
-  // compacted list
-  const long stride = 3 * Vh;
-  bs_launch_compact(ru_, cap_, slots_, st);
-  bs_launch_ru(rhs_, active_, ru_, ru_cont_, slots_, lcoef_, sp_, (int)Vh, x64_.slot(0), xs_.slot(0), b64_.slot(0),
-               ax64_.slot(0), rs_.slot(0), ps_.slot(0), stride, partA_, partB_, partC_, nch_, cap_, 0, partB_, st);
+  // reliable update of the flagged slots, all on the device, then the search
+  // directions of all slots
   apply_A64(ru_, true);
-  bs_launch_ru(rhs_, active_, ru_, ru_cont_, slots_, lcoef_, sp_, (int)Vh, x64_.slot(0), xs_.slot(0), b64_.slot(0),
-               ax64_.slot(0), rs_.slot(0), ps_.slot(0), stride, partA_, partB_, partC_, nch_, cap_, 1, partB_, st);
-  bs_launch_ru(rhs_, active_, ru_, ru_cont_, slots_, lcoef_, sp_, (int)Vh, x64_.slot(0), xs_.slot(0), b64_.slot(0),
-               ax64_.slot(0), rs_.slot(0), ps_.slot(0), stride, partA_, partB_, partC_, nch_, cap_, 2, partB_, st);
-  bs_launch_ru(rhs_, active_, ru_, ru_cont_, slots_, lcoef_, sp_, (int)Vh, x64_.slot(0), xs_.slot(0), b64_.slot(0),
-               ax64_.slot(0), rs_.slot(0), ps_.slot(0), stride, partA_, partB_, partC_, nch_, cap_, 3, partB_, st);
+  bs_launch_ru_scalar(rhs_, active_, ru_, ru_cont_, lcoef_, partA_, partB_, partC_, nch_, cap_, st);
+  bs_launch_pnext(rhs_, active_, &glob_->status, ru_cont_, lcoef_, sp_, (int)Vh, rs_.slot(0), ps_.slot(0), 3 * Vh,
+                  cap_, partB_, st);
 }
 
 void BatchSolver::build_graph() {

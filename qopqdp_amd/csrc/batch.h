@@ -46,28 +46,22 @@ struct BsGlobal {
 void bs_launch_scalar1(BsRhs *rhs, const int *active, const int *status,
                        const double *partA, const double *partB, int nch, int n,
                        int *ru_cont, hipStream_t st);
-void bs_launch_update(BsRhs *rhs, const int *active, const int *status, int prec,
-                      int Vh, VecView rs, VecView Aps, VecView ps, VecView xs,
-                      long stride, double *partC, int n, hipStream_t st);
 void bs_launch_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob,
                        const double *partC, int nch, int n, int *ru, hipStream_t st);
-// Device reliable update, stage 0: x += xs; 1: residual, |r|^2 and <rs,ps>;
-// 2: per-slot decisions; 3: search-direction fix.
-// list: compacted flagged slots (bs_launch_compact of ru), read by the
-// vector steps 0, 1 and 3
-void bs_launch_ru(BsRhs *rhs, int *active, int *ru, int *ru_cont, const int *list, double *lcoef,
-                  int prec, int Vh, VecView x64, VecView xs, VecView b64, VecView ax64, VecView rs,
-                  VecView ps, long stride, double *pr2, double *pre, double *pim, int nch,
-                  int n, int stage, double *ppB, hipStream_t st);
+// x += xs, xs = 0 of the flagged slots, where it is a pass of its own.
+void bs_launch_ru_x(const int *ru, int n, int Vh, VecView x64, VecView xs, long stride, hipStream_t st);
+// Decisions of the reliable updates of the flagged slots, from the partials
+// |r|^2 and <rs, ps> of the second masked FP64 hop.
+void bs_launch_ru_scalar(BsRhs *rhs, int *active, int *ru, int *ru_cont, double *lcoef,
+                         const double *pr2, const double *pre, const double *pim, int nch, int n,
+                         hipStream_t st);
 // A slot whose residual has dropped to join2 * r2_rel joins the reliable
 // update of this iteration when another slot is flagged for one.
 void bs_launch_ru_join(BsRhs *rhs, const int *active, int *ru, int n, hipStream_t st);
-// out[0] = number k of nonzero flags[0..n), out[1..k] their indices (device)
-void bs_launch_compact(const int *flags, int n, int *out, hipStream_t st);
-void bs_launch_commit(BsGlobal *glob, hipStream_t st);
-void bs_launch_pupdate(const BsRhs *rhs, const int *active, const int *status,
-                       int prec, int Vh, VecView rs, VecView ps, long stride, int n,
-                       int skip_flagged, double *partB, hipStream_t st);
+// Search directions of the running slots, after any reliable updates.
+void bs_launch_pnext(const BsRhs *rhs, const int *active, const int *status, const int *ru_cont,
+                     const double *lcoef, int prec, int Vh, VecView rs, VecView ps, long stride,
+                     int n, double *partB, hipStream_t st);
 void bs_launch_sum(const double *part, int nch, int n, const int *sel,
                    double *out, hipStream_t st);
 
@@ -145,9 +139,9 @@ class BatchSolver {
  private:
   void enqueue_iteration();
   void build_graph();
-  // ax64 = A x64 on the slots set in mask (listed: slots_ already holds
-  // their compacted list)
-  void apply_A64(const int *mask, bool listed = false);
+  // ax64 = A x64 on the slots set in mask; with update (the reliable update
+  // of the iteration) x64 += xs first and the residual in place of ax64
+  void apply_A64(const int *mask, bool update = false);
 
   Links &L_;
   Lattice *lat_;
@@ -166,7 +160,6 @@ class BatchSolver {
   int *active_ = nullptr, *active_h_ = nullptr;
   int *sel_ = nullptr, *sel_h_ = nullptr;
   int *ru_ = nullptr, *ru_cont_ = nullptr;  // device reliable-update masks
-  int *slots_ = nullptr;  // device [1 + cap]: compacted slot list of the masked FP64 hops
   BsGlobal *glob_ = nullptr, *glob_h_ = nullptr;
   double *partA_ = nullptr, *partB_ = nullptr, *partC_ = nullptr;
   double *coef_ = nullptr;      // [cap][2] hop coefficients (-1, m2)

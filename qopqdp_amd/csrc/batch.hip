@@ -133,43 +133,6 @@ bs_scalar1(BsRhs *rhs, const int *active, const int *status, const double *partA
   R.alpha = pAp > 0 ? R.r2 / pAp : 0.0;
 }
 
-// rs -= alpha Aps ; xs += alpha ps ; partial |rs|^2
-template <int P>
-__global__ void __launch_bounds__(256)
-bs_update(const BsRhs *rhs, const int *active, const int *status, int Vh, VecView rs,
-          VecView Aps, VecView ps, VecView xs, long stride, double *partC) {
-  using R = typename BT<P>::R;
-  if (*status != 0) return;
-  const int b = blockIdx.y;
-  if (!active[b]) return;
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = 0;
-  if (h < Vh) {
-    const R al = (R)rhs[b].alpha;
-    const size_t off = (size_t)b * stride;
-    const long noff = (long)b * Vh;
-    const size_t cb = sizeof(typename BT<P>::S);
-    R r[6], a[6], p[6];
-    ld3<P>((const char *)rs.data + off * cb, rs.norm ? rs.norm + noff : nullptr, h, Vh, r);
-    ld3<P>((const char *)Aps.data + off * cb, Aps.norm ? Aps.norm + noff : nullptr, h, Vh, a);
-    ld3<P>((const char *)ps.data + off * cb, ps.norm ? ps.norm + noff : nullptr, h, Vh, p);
-#pragma unroll
-    for (int i = 0; i < 6; i++) r[i] = fma(-al, a[i], r[i]);
-    st3_q<P>((char *)rs.data + off * cb, rs.norm ? rs.norm + noff : nullptr, h, Vh, r);
-#pragma unroll
-    for (int i = 0; i < 6; i++) acc += (double)r[i] * (double)r[i];
-    // xs is FP32
-    float x[6];
-    ld3<P32>((const char *)xs.data + off * sizeof(float2), nullptr, h, Vh, x);
-#pragma unroll
-    for (int i = 0; i < 6; i++) x[i] = fmaf((float)al, (float)p[i], x[i]);
-    st3<P32>((char *)xs.data + off * sizeof(float2), nullptr, h, Vh, x);
-  }
-  const int nch = (Vh + 63) / 64;
-  acc = bsum(acc);
-  if ((threadIdx.x & 63) == 0 && (h >> 6) < nch) partC[(long)b * nch + (h >> 6)] = acc;
-}
-
 // new r2, reliable-update and stopping decisions, beta
 __global__ void __launch_bounds__(1024)
 bs_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, int nch, int *ru) {
@@ -194,59 +157,28 @@ bs_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, i
   }
 }
 
-// ps = rs + beta ps
-// ps = rs + beta ps ; partial |ps|^2 of the stored ps (the next iteration's
-// p.Ap needs it)
-template <int P>
-__global__ void __launch_bounds__(256)
-bs_pupdate(const BsRhs *rhs, const int *active, const int *status, int Vh, VecView rs,
-           VecView ps, long stride, int skip_flagged, double *partB) {
-  using R = typename BT<P>::R;
-  if (status && *status != 0) return;
-  const int b = blockIdx.y;
-  if (!active[b]) return;
-  if (skip_flagged && rhs[b].need_update) return;
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = 0;
-  if (h < Vh) {
-    const R be = (R)rhs[b].beta;
-    const size_t off = (size_t)b * stride;
-    const long noff = (long)b * Vh;
-    const size_t cb = sizeof(typename BT<P>::S);
-    R r[6], p[6];
-    float *pn = ps.norm ? ps.norm + noff : nullptr;
-    ld3<P>((const char *)rs.data + off * cb, rs.norm ? rs.norm + noff : nullptr, h, Vh, r);
-    ld3<P>((const char *)ps.data + off * cb, pn, h, Vh, p);
-#pragma unroll
-    for (int i = 0; i < 6; i++) p[i] = fma(be, p[i], r[i]);
-    st3_q<P>((char *)ps.data + off * cb, pn, h, Vh, p);
-#pragma unroll
-    for (int i = 0; i < 6; i++) acc += (double)p[i] * (double)p[i];
-  }
-  const int nch = (Vh + 63) / 64;
-  acc = bsum(acc);
-  if ((threadIdx.x & 63) == 0 && (h >> 6) < nch) partB[(long)b * nch + (h >> 6)] = acc;
-}
-
 // ---------------------------------------------------------------------------
 // Reliable update on the device, for the slots flagged by bs_scalar2 (ru[b]):
-//   x += xs, xs = 0                         (bs_ru_x)
-//   ax = A x in FP64                        (two masked FP64 hops)
-//   r = b - ax ; rs = r ; |r|^2, <rs, ps>   (bs_ru_resid)
-//   stop / continue, beta                   (bs_ru_scalar)
-//   ps = (1 - beta <rs,ps>/|r|^2) rs + beta ps  (bs_ru_pfix)
+//   t = D (x + xs) in FP64                       (masked hop, RED_SADD; on large
+//                                                 lattices bs_ru_x, then a plain hop)
+//   x += xs, xs = 0 ; r = b - (m^2 x - D t) ; rs = r ; |r|^2, <rs, ps>
+//                                                (masked hop, RED_RU16 / RED_RU32)
+//   stop / continue, beta                        (bs_ru_scalar)
+//   ps = (1 - beta <rs,ps>/|r|^2) rs + beta ps   (bs_pnext)
 // Unflagged slots skip every step, so a slot's arithmetic is the same
-// whatever the other slots do.  The vector steps run one block per 256 sites
-// over the compacted list of the flagged slots (list[0] = their number, then
-// the slots; bs_compact), so an iteration with no update costs one short
-// launch per step.
+// whatever the other slots do.  Every launch is in the captured iteration and
+// costs a few microseconds also when no slot is flagged, so the vector steps
+// are part of the hops, the hops find the flagged slots themselves and one
+// kernel updates the search directions of all slots: eight launches per
+// iteration where there were twelve.  Twelve requests at 8x12^2x16 through
+// the server 10.9 -> 8.1 ms, 24 refinements and 4 x 6 multi-shift at 16^3x32
+// 39.9 -> 36.0 ms, 16 FP16 solves at 24^3x48 unchanged within 1%.
+// x += xs, xs = 0 of the flagged slots
 __global__ void __launch_bounds__(256)
-bs_ru_x(const int *list, int Vh, VecView x64, VecView xs, long stride) {
-  const int k = list[0];
+bs_ru_x(const int *ru, int n, int Vh, VecView x64, VecView xs, long stride) {
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= Vh) return;
-  for (int j = 0; j < k; j++) {
-    const int b = list[1 + j];
+  for (int b = 0; b < n; b++) {
+    if (!ru[b] || h >= Vh) continue;
     const size_t off = (size_t)b * stride;
     double2 *x = (double2 *)x64.data + off;
     float2 *y = (float2 *)xs.data + off;
@@ -259,55 +191,6 @@ bs_ru_x(const int *list, int Vh, VecView x64, VecView xs, long stride) {
       x[c * Vh + h] = a;
       y[c * Vh + h] = make_float2(0.f, 0.f);
     }
-  }
-}
-
-template <int P>
-__global__ void __launch_bounds__(256)
-bs_ru_resid(const int *list, int Vh, VecView b64, VecView ax64, VecView rs, VecView ps, long stride,
-            double *part_r2, double *part_re, double *part_im) {
-  using R = typename BT<P>::R;
-  const int k = list[0];
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int j = 0; j < k; j++) {
-  const int b = list[1 + j];
-  double r2 = 0, dre = 0, dim = 0;
-  if (h < Vh) {
-    const size_t off = (size_t)b * stride;
-    const long noff = (long)b * Vh;
-    const size_t cb = sizeof(typename BT<P>::S);
-    const double2 *bb = (const double2 *)b64.data + off;
-    const double2 *aa = (const double2 *)ax64.data + off;
-    R rv[6];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      double2 u = bb[c * Vh + h], w = aa[c * Vh + h];
-      double xr = u.x - w.x, xi = u.y - w.y;
-      r2 += xr * xr + xi * xi;
-      rv[2 * c] = (R)xr;
-      rv[2 * c + 1] = (R)xi;
-    }
-    float *rn = rs.norm ? rs.norm + noff : nullptr;
-    st3_q<P>((char *)rs.data + off * cb, rn, h, Vh, rv);  // rv: the stored rs
-    R p[6];
-    const R *q = rv;
-    ld3<P>((const char *)ps.data + off * cb, ps.norm ? ps.norm + noff : nullptr, h, Vh, p);
-#pragma unroll
-    for (int c = 0; c < 3; c++) {  // <rs, ps> = sum conj(rs) ps
-      double qr = q[2 * c], qi = q[2 * c + 1], pr = p[2 * c], pi = p[2 * c + 1];
-      dre += qr * pr + qi * pi;
-      dim += qr * pi - qi * pr;
-    }
-  }
-  const int nch = (Vh + 63) / 64;
-  r2 = bsum(r2);
-  dre = bsum(dre);
-  dim = bsum(dim);
-  if ((threadIdx.x & 63) == 0 && (h >> 6) < nch) {
-    part_r2[(long)b * nch + (h >> 6)] = r2;
-    part_re[(long)b * nch + (h >> 6)] = dre;
-    part_im[(long)b * nch + (h >> 6)] = dim;
-  }
   }
 }
 
@@ -340,42 +223,50 @@ bs_ru_scalar(BsRhs *rhs, int *active, int *ru, int *ru_cont, double *lcoef,
   ru_cont[b] = 1;
 }
 
+// Search directions of all running slots: ps = rs + beta ps, or after a
+// reliable update that continues (ru_cont) the fixed combination of lcoef;
+// partial |ps|^2 of the stored ps (the next iteration's p.Ap needs it).
 template <int P>
 __global__ void __launch_bounds__(256)
-bs_ru_pfix(const int *list, const int *ru_cont, const double *lcoef, int Vh, VecView rs, VecView ps,
-           long stride, double *partB) {
+bs_pnext(const BsRhs *rhs, const int *active, const int *status, const int *ru_cont, const double *lcoef, int Vh,
+         VecView rs, VecView ps, long stride, double *partB) {
   using R = typename BT<P>::R;
-  const int k = list[0];
+  if (*status != 0) return;
+  const int b = blockIdx.y;
+  if (!active[b]) return;
+  const bool fix = ru_cont[b] != 0;
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int j = 0; j < k; j++) {
-  const int b = list[1 + j];
-  if (!ru_cont[b]) continue;  // the slot stopped at this update
   double acc = 0;
   if (h < Vh) {
-  const size_t off = (size_t)b * stride;
-  const long noff = (long)b * Vh;
-  const size_t cb = sizeof(typename BT<P>::S);
-  const double c0r = lcoef[6 * b], c0i = lcoef[6 * b + 1], c1 = lcoef[6 * b + 2];
-  R r[6], p[6];
-  ld3<P>((const char *)rs.data + off * cb, rs.norm ? rs.norm + noff : nullptr, h, Vh, r);
-  ld3<P>((const char *)ps.data + off * cb, ps.norm ? ps.norm + noff : nullptr, h, Vh, p);
+    const size_t off = (size_t)b * stride;
+    const long noff = (long)b * Vh;
+    const size_t cb = sizeof(typename BT<P>::S);
+    R r[6], p[6];
+    float *pn = ps.norm ? ps.norm + noff : nullptr;
+    ld3<P>((const char *)rs.data + off * cb, rs.norm ? rs.norm + noff : nullptr, h, Vh, r);
+    ld3<P>((const char *)ps.data + off * cb, pn, h, Vh, p);
+    if (!fix) {
+      const R be = (R)rhs[b].beta;
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    double rr = r[2 * c], ri = r[2 * c + 1];
-    double pr = fma(c0r, rr, fma(-c0i, ri, c1 * (double)p[2 * c]));
-    double pi = fma(c0r, ri, fma(c0i, rr, c1 * (double)p[2 * c + 1]));
-    p[2 * c] = (R)pr;
-    p[2 * c + 1] = (R)pi;
-  }
-  float *pn = ps.norm ? ps.norm + noff : nullptr;
-  st3_q<P>((char *)ps.data + off * cb, pn, h, Vh, p);
+      for (int i = 0; i < 6; i++) p[i] = fma(be, p[i], r[i]);
+    } else {
+      const double c0r = lcoef[6 * b], c0i = lcoef[6 * b + 1], c1 = lcoef[6 * b + 2];
 #pragma unroll
-  for (int i = 0; i < 6; i++) acc += (double)p[i] * (double)p[i];
+      for (int c = 0; c < 3; c++) {
+        double rr = r[2 * c], ri = r[2 * c + 1];
+        double pr = fma(c0r, rr, fma(-c0i, ri, c1 * (double)p[2 * c]));
+        double pi = fma(c0r, ri, fma(c0i, rr, c1 * (double)p[2 * c + 1]));
+        p[2 * c] = (R)pr;
+        p[2 * c + 1] = (R)pi;
+      }
+    }
+    st3_q<P>((char *)ps.data + off * cb, pn, h, Vh, p);
+#pragma unroll
+    for (int i = 0; i < 6; i++) acc += (double)p[i] * (double)p[i];
   }
   const int nch = (Vh + 63) / 64;
   acc = bsum(acc);
   if ((threadIdx.x & 63) == 0 && (h >> 6) < nch) partB[(long)b * nch + (h >> 6)] = acc;
-  }
 }
 
 // One thread: if any slot is flagged for a reliable update in this
@@ -395,12 +286,6 @@ __global__ void bs_ru_join(BsRhs *rhs, const int *active, int *ru, int n) {
   }
 }
 
-// Last kernel of an iteration: raise the status the host polls.  Kernels of
-// one iteration all see the same status because only this kernel changes it.
-__global__ void bs_commit(BsGlobal *glob) {
-  if (glob->status == 0 && glob->pending) glob->status = 1;
-}
-
 // out[b] = sum of slot b's partials (fixed order), for selected slots
 __global__ void __launch_bounds__(1024)
 bs_sum(const double *part, int nch, const int *sel, double *out) {
@@ -416,53 +301,21 @@ void bs_launch_scalar1(BsRhs *rhs, const int *active, const int *status, const d
   hipLaunchKernelGGL(bs_scalar1, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, status, partA, partB, nch, ru_cont);
   QOP_CHECK_HIP(hipGetLastError());
 }
-void bs_launch_update(BsRhs *rhs, const int *active, const int *status, int prec, int Vh,
-                      VecView rs, VecView Aps, VecView ps, VecView xs, long stride,
-                      double *partC, int n, hipStream_t st) {
-  dim3 g((Vh + 255) / 256, n), bl(256);
-  if (prec == P32) hipLaunchKernelGGL(bs_update<P32>, g, bl, 0, st, rhs, active, status, Vh, rs, Aps, ps, xs, stride, partC);
-  else if (prec == P16) hipLaunchKernelGGL(bs_update<P16>, g, bl, 0, st, rhs, active, status, Vh, rs, Aps, ps, xs, stride, partC);
-  else hipLaunchKernelGGL(bs_update<P64>, g, bl, 0, st, rhs, active, status, Vh, rs, Aps, ps, xs, stride, partC);
-  QOP_CHECK_HIP(hipGetLastError());
-}
 void bs_launch_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, int nch,
                        int n, int *ru, hipStream_t st) {
   hipLaunchKernelGGL(bs_scalar2, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, glob, partC, nch, ru);
-  QOP_CHECK_HIP(hipGetLastError());
-}
-// Compacted list of the flagged slots: out[0] = their number k, out[1..k]
-// their indices in increasing order (one wavefront, ballot and prefix count).
-__global__ void __launch_bounds__(64) bs_compact(const int *flags, int n, int *out) {
-  const int lane = (int)threadIdx.x;
-  int base = 0;
-  for (int i0 = 0; i0 < n; i0 += 64) {
-    const int i = i0 + lane;
-    const bool f = i < n && flags[i] != 0;
-    const unsigned long long m = __ballot(f);
-    if (f) out[1 + base + __popcll(m & ((1ull << lane) - 1ull))] = i;
-    base += __popcll(m);
-  }
-  if (lane == 0) out[0] = base;
-}
-void bs_launch_compact(const int *flags, int n, int *out, hipStream_t st) {
-  hipLaunchKernelGGL(bs_compact, dim3(1), dim3(64), 0, st, flags, n, out);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_ru_join(BsRhs *rhs, const int *active, int *ru, int n, hipStream_t st) {
   hipLaunchKernelGGL(bs_ru_join, dim3(1), dim3(64), 0, st, rhs, active, ru, n);
   QOP_CHECK_HIP(hipGetLastError());
 }
-void bs_launch_commit(BsGlobal *glob, hipStream_t st) {
-  hipLaunchKernelGGL(bs_commit, dim3(1), dim3(64), 0, st, glob);
-  QOP_CHECK_HIP(hipGetLastError());
-}
-void bs_launch_pupdate(const BsRhs *rhs, const int *active, const int *status, int prec, int Vh,
-                       VecView rs, VecView ps, long stride, int n, int skip_flagged, double *partB,
-                       hipStream_t st) {
+void bs_launch_pnext(const BsRhs *rhs, const int *active, const int *status, const int *ru_cont,
+                     const double *lcoef, int prec, int Vh, VecView rs, VecView ps, long stride, int n,
+                     double *partB, hipStream_t st) {
   dim3 g((Vh + 255) / 256, n), bl(256);
-  if (prec == P32) hipLaunchKernelGGL(bs_pupdate<P32>, g, bl, 0, st, rhs, active, status, Vh, rs, ps, stride, skip_flagged, partB);
-  else if (prec == P16) hipLaunchKernelGGL(bs_pupdate<P16>, g, bl, 0, st, rhs, active, status, Vh, rs, ps, stride, skip_flagged, partB);
-  else hipLaunchKernelGGL(bs_pupdate<P64>, g, bl, 0, st, rhs, active, status, Vh, rs, ps, stride, skip_flagged, partB);
+  if (prec == P32) hipLaunchKernelGGL(bs_pnext<P32>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
+  else hipLaunchKernelGGL(bs_pnext<P16>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_sum(const double *part, int nch, int n, const int *sel, double *out, hipStream_t st) {
@@ -470,28 +323,14 @@ void bs_launch_sum(const double *part, int nch, int n, const int *sel, double *o
   QOP_CHECK_HIP(hipGetLastError());
 }
 
-}  // namespace qop
-
-namespace qop {
-void bs_launch_ru(BsRhs *rhs, int *active, int *ru, int *ru_cont, const int *list, double *lcoef,
-                  int prec, int Vh, VecView x64, VecView xs, VecView b64, VecView ax64, VecView rs,
-                  VecView ps, long stride, double *pr2, double *pre, double *pim, int nch, int n,
-                  int stage, double *ppB, hipStream_t st) {
-  dim3 g((Vh + 255) / 256), bl(256);
-  if (stage == 0) {
-    hipLaunchKernelGGL(bs_ru_x, g, bl, 0, st, list, Vh, x64, xs, stride);
-  } else if (stage == 1) {
-    if (prec == P32) hipLaunchKernelGGL(bs_ru_resid<P32>, g, bl, 0, st, list, Vh, b64, ax64, rs, ps, stride, pr2, pre, pim);
-    else if (prec == P16) hipLaunchKernelGGL(bs_ru_resid<P16>, g, bl, 0, st, list, Vh, b64, ax64, rs, ps, stride, pr2, pre, pim);
-    else hipLaunchKernelGGL(bs_ru_resid<P64>, g, bl, 0, st, list, Vh, b64, ax64, rs, ps, stride, pr2, pre, pim);
-  } else if (stage == 2) {
-    hipLaunchKernelGGL(bs_ru_scalar, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, ru, ru_cont, lcoef,
-                       (const double *)pr2, (const double *)pre, (const double *)pim, nch);
-  } else {
-    if (prec == P32) hipLaunchKernelGGL(bs_ru_pfix<P32>, g, bl, 0, st, list, (const int *)ru_cont, (const double *)lcoef, Vh, rs, ps, stride, ppB);
-    else if (prec == P16) hipLaunchKernelGGL(bs_ru_pfix<P16>, g, bl, 0, st, list, (const int *)ru_cont, (const double *)lcoef, Vh, rs, ps, stride, ppB);
-    else hipLaunchKernelGGL(bs_ru_pfix<P64>, g, bl, 0, st, list, (const int *)ru_cont, (const double *)lcoef, Vh, rs, ps, stride, ppB);
-  }
+void bs_launch_ru_x(const int *ru, int n, int Vh, VecView x64, VecView xs, long stride, hipStream_t st) {
+  hipLaunchKernelGGL(bs_ru_x, dim3((Vh + 255) / 256), dim3(256), 0, st, ru, n, Vh, x64, xs, stride);
   QOP_CHECK_HIP(hipGetLastError());
 }
+void bs_launch_ru_scalar(BsRhs *rhs, int *active, int *ru, int *ru_cont, double *lcoef, const double *pr2,
+                         const double *pre, const double *pim, int nch, int n, hipStream_t st) {
+  hipLaunchKernelGGL(bs_ru_scalar, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, ru, ru_cont, lcoef, pr2, pre, pim, nch);
+  QOP_CHECK_HIP(hipGetLastError());
+}
+
 }  // namespace qop

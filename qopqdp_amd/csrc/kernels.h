@@ -9,7 +9,12 @@ namespace qop {
 // r -= alpha (beta x + alpha_hop hop), xs += alpha x, reduction |r|^2).
 // RED_R: RED_CG without the solution update (FP64 and FP32 vectors, one RHS
 // per thread): the second hop of the reference solvers' iteration.
-enum { RED_NONE = 0, RED_OUT2 = 1, RED_X2 = 2, RED_CG = 3, RED_R = 4 };
+// FP64 hops over flagged slots (launch_hop_flagged):
+// RED_SADD: src is src + src_add (FP32 increments), formed as it is read.
+// RED_RU32 / RED_RU16: the end of a reliable update in the epilogue, with the
+// sloppy vectors in FP32 / FP16 (RuArgs): x += xs, xs = 0; out = A x is not
+// stored; r = b - A x goes into the sloppy rs; |r|^2 and <rs, ps>.
+enum { RED_NONE = 0, RED_OUT2 = 1, RED_X2 = 2, RED_CG = 3, RED_R = 4, RED_SADD = 5, RED_RU32 = 6, RED_RU16 = 7 };
 int hop_partial_blocks(const Lattice *lat);
 
 // Hop: dst[b] = alpha_b * sum_k W_k src[b](x+d_k) + beta_b * x[b], for the
@@ -27,9 +32,10 @@ struct HopArgs {
   double alpha = 1.0, beta = 0.0;
   double *partial = nullptr;     // [n][nchunk]
   const int *active = nullptr;   // device [n] or null
-  const int *slots = nullptr;    // device [1 + n] or null: count k, then the slots that launch
-                                 // RHS 0..k-1 work on (FP64 masked hops: k flagged slots take
-                                 // ceil(k / RHS per thread) link reads)
+  const int *slots = nullptr;    // device [1 + n] or null: count k, then the slots that launch RHS
+                                 // 0..k-1 work on.  No caller passes one, but the test for it stays:
+                                 // without it the compiler schedules the one-RHS FP64 hop 1.6 times
+                                 // slower (28 against 45 us at 16^3x32)
   const int *status = nullptr;   // device flag: kernel is a no-op when nonzero
   int remap = 1;
   int nt = 0;                    // non-temporal link loads
@@ -54,6 +60,21 @@ struct HopArgs {
 };
 void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
                      bool hasx, hipStream_t st);
+// FP64 hop over the flagged slots, with the operands of RED_SADD and of
+// RED_RU32 / RED_RU16: all [slot] with the strides of the launch (vectors
+// sstride complex, norms nstride).  xs null: x holds the solution; ps null: no
+// <rs, ps>.  The partial arrays are [slot][nchunk].  (A type of its own: the
+// arguments of the other hops keep their size.)
+struct HopFlagArgs : HopArgs {
+  const int *flags = nullptr;  // device [n]: launch RHS j works on the j-th slot whose flag is set, so
+                               // k flagged slots take ceil(k / RHS per thread) link reads
+  const void *src_add = nullptr;
+  void *xs64 = nullptr;
+  const void *b64 = nullptr;
+  VecView rs{}, ps{};
+  double *r2 = nullptr, *re = nullptr, *im = nullptr;
+};
+void launch_hop_flagged(HopFlagArgs a, int nl, int nb, int block, int red, bool hasx, hipStream_t st);
 // One-RHS hop of the reference path (FP64 / FP32 vectors, no batch masks):
 // launches the four-wave kernel or the one-thread-per-site kernel, whichever
 // suits the lattice; with b, the hop onto the other parity in the same launch.

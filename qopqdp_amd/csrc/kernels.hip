@@ -343,12 +343,88 @@ __device__ __forceinline__ int site_of_block(const Geom &g, int sb, int tile) {
   return x0 * (g.Vh / g.L[0]) + j * tile + (rem - x0 * tb) * blockDim.x + threadIdx.x;
 }
 
+// The j-th slot whose flag is set, or -1 (all lanes of the wave call it; one
+// load and ballot per 64 slots, so the flagged slots need no list built by a
+// kernel of its own).
+__device__ __forceinline__ int nth_flag(const int *flags, int n, int j) {
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    const int i = i0 + (int)(threadIdx.x & 63);
+    unsigned long long m = __ballot(i < n && flags[i] != 0);
+    const int c = __popcll(m);
+    if (j < c) {
+      for (; j > 0; j--) m &= m - 1;
+      return i0 + __ffsll(m) - 1;
+    }
+    j -= c;
+  }
+  return -1;
+}
+
+// RED_SADD: the FP32 increment of a source word is added as it is read.
+template <class S>
+__device__ __forceinline__ void src_add(const HopFlagArgs &a, S &t, int slot, long at) {
+  const float2 d = ((const float2 *)a.src_add + (long)slot * a.sstride)[at];
+  t.x += (double)d.x;
+  t.y += (double)d.y;
+}
+
+// RED_RU32 / RED_RU16 (SP: the sloppy precision): the own-site x as it enters
+// A x, x + xs, stored, and xs cleared.
+__device__ __forceinline__ void ru_x(const HopFlagArgs &a, int h, int Vh, int slot, double xv[6]) {
+  if (!a.xs64) return;
+  float2 *xs = (float2 *)a.xs64 + (long)slot * a.sstride;
+  double2 *x64 = (double2 *)a.x.data + (long)slot * a.xstride;
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    const float2 d = xs[(long)c * Vh + h];
+    xv[2 * c] += (double)d.x;
+    xv[2 * c + 1] += (double)d.y;
+    x64[(long)c * Vh + h] = make_double2(xv[2 * c], xv[2 * c + 1]);
+    xs[(long)c * Vh + h] = make_float2(0.f, 0.f);
+  }
+}
+// o = A x: r = b - o into rs, |r|^2 and <rs, ps> of the stored rs.
+template <int SP>
+__device__ __forceinline__ void ru_resid(const HopFlagArgs &a, int h, int Vh, int slot, const double o[6],
+                                         double red[3]) {
+  using R = typename PT<SP>::R;
+  using S = typename PT<SP>::S;
+  const long off = (long)slot * a.sstride, noff = (long)slot * a.nstride;
+  const double2 *bb = (const double2 *)a.b64 + off;
+  R rv[6];
+  double r2 = 0, dre = 0, dim = 0;
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    double2 u = bb[(long)c * Vh + h];
+    double xr = u.x - o[2 * c], xi = u.y - o[2 * c + 1];
+    // explicit FMAs here and below: the sums must not depend on how each
+    // launch shape's instance is contracted
+    r2 = fma(xr, xr, fma(xi, xi, r2));
+    rv[2 * c] = (R)xr;
+    rv[2 * c + 1] = (R)xi;
+  }
+  vstore_q<SP>((S *)a.rs.data + off, a.rs.norm ? a.rs.norm + noff : nullptr, h, Vh, rv);  // rv: the stored rs
+  if (a.ps.data) {
+    R p[6];
+    vload<SP>((const S *)a.ps.data + off, a.ps.norm ? a.ps.norm + noff : nullptr, h, Vh, p);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {  // <rs, ps> = sum conj(rs) ps
+      double qr = rv[2 * c], qi = rv[2 * c + 1], pr = p[2 * c], pi = p[2 * c + 1];
+      dre = fma(qr, pr, fma(qi, pi, dre));
+      dim = fma(qr, pi, fma(-qi, pr, dim));
+    }
+  }
+  red[0] = r2;
+  red[1] = dre;
+  red[2] = dim;
+}
+
 // Output of one site for NB RHS: out = beta x + alpha acc (stored), or the
 // fused CG update; per-RHS reduction terms in red[].
-template <int P, int NB, int RED, bool HASX, bool NT>
-__device__ __forceinline__ void hop_epilogue(const HopArgs &a, int h, int Vh, const int sl[NB],
+template <int P, int NB, int RED, bool HASX, bool NT, class A>
+__device__ __forceinline__ void hop_epilogue(const A &a, int h, int Vh, const int sl[NB],
                                              const bool act[NB], typename PT<P>::R acc[NB][6],
-                                             double red[NB]) {
+                                             double red[NB], double ru[][3]) {
   using R = typename PT<P>::R;
 #pragma unroll
   for (int b = 0; b < NB; b++) {
@@ -364,11 +440,16 @@ __device__ __forceinline__ void hop_epilogue(const HopArgs &a, int h, int Vh, co
       // the fused CG update streams p, r and x (each read or written once
       // per iteration at its own site): non-temporal
       vload<P, RED == RED_CG>(xd, xn, h, Vh, xv);
+      if constexpr (RED == RED_RU32 || RED == RED_RU16) ru_x(a, h, Vh, rb, xv);
 #pragma unroll
       for (int i = 0; i < 6; i++) o[i] = fma((R)be, xv[i], (R)al * acc[b][i]);
     } else {
 #pragma unroll
       for (int i = 0; i < 6; i++) o[i] = (R)al * acc[b][i];
+    }
+    if constexpr (RED == RED_RU32 || RED == RED_RU16) {
+      ru_resid<RED == RED_RU16 ? P16 : P32>(a, h, Vh, rb, o, ru[b]);
+      continue;
     }
     char *dd = (char *)a.dst.data + (long)rb * a.dstride * sizeof(typename PT<P>::S);
     float *dn = a.dst.norm ? a.dst.norm + (long)rb * a.nstride : nullptr;
@@ -434,10 +515,11 @@ __device__ __forceinline__ void hop_epilogue(const HopArgs &a, int h, int Vh, co
 // links and per-link scales).
 // One RHS group of the hop for one site block: the group starting at launch
 // RHS b0_in and site block sb_in, or (negative) the ones the grid gives.
-template <int P, int NL, int NB, int RED, bool HASX, bool NT, bool SGL, bool STG, int LP, bool BUF>
-__device__ __forceinline__ void hop_group(const HopArgs &a, int b0_in, int sb_in) {
+template <int P, int NL, int NB, int RED, bool HASX, bool NT, bool SGL, bool STG, int LP, bool BUF, class A>
+__device__ __forceinline__ void hop_group(const A &a, int b0_in, int sb_in) {
   static_assert(!BUF || (P != P64 && !SGL), "buffer loads: FP32 / FP16, double-stored links");
   using R = typename PT<P>::R;
+  constexpr bool GL = std::is_same<A, HopFlagArgs>::value;
   const Geom g = a.g;
   const int Vh = g.Vh;
   const int lb = logical_block(a.remap);
@@ -453,16 +535,23 @@ __device__ __forceinline__ void hop_group(const HopArgs &a, int b0_in, int sb_in
   double red[NB];
 #pragma unroll
   for (int b = 0; b < NB; b++) red[b] = 0.0;
+  constexpr bool RU = RED == RED_RU32 || RED == RED_RU16;
+  double ru[RU ? NB : 1][3];
+#pragma unroll
+  for (int b = 0; b < (RU ? NB : 1); b++) ru[b][0] = ru[b][1] = ru[b][2] = 0.0;
 
   bool act[NB];
   int sl[NB];  // slot of each RHS of this thread
   bool any = false;
 #pragma unroll
   for (int b = 0; b < NB; b++) {
-    // the launch's RHS j = b0 + b is slot j, or with a compacted list
-    // (a.slots: count, then the slots) the j-th listed slot
+    // the launch's RHS j = b0 + b is slot j, or the j-th flagged or listed one
     const int j = b0 + b;
-    if (a.slots) {
+    if constexpr (GL) {
+      sl[b] = nth_flag(a.flags, a.n, j);
+      act[b] = sl[b] >= 0;
+      if (!act[b]) sl[b] = j;
+    } else if (a.slots) {
       act[b] = j < a.slots[0];
       sl[b] = act[b] ? a.slots[1 + j] : j;
     } else {
@@ -502,7 +591,11 @@ __device__ __forceinline__ void hop_group(const HopArgs &a, int b0_in, int sb_in
           tr[b * bs + threadIdx.x] = rec;
         } else {
 #pragma unroll
-          for (int c = 0; c < 3; c++) td[(b * 3 + c) * bs + threadIdx.x] = sd[(long)c * Vh + hs];
+          for (int c = 0; c < 3; c++) {
+            S t = sd[(long)c * Vh + hs];
+            if constexpr (RED == RED_SADD) src_add(a, t, sl[b], (long)c * Vh + hs);
+            td[(b * 3 + c) * bs + threadIdx.x] = t;
+          }
         }
       }
     }
@@ -604,7 +697,10 @@ __device__ __forceinline__ void hop_group(const HopArgs &a, int b0_in, int sb_in
             } else {
               const S *sd = (const S *)a.src.data + (long)sl[b] * a.sstride;
 #pragma unroll
-              for (int c = 0; c < 3; c++) gm[b][c] = sd[(long)c * Vh + nb];
+              for (int c = 0; c < 3; c++) {
+                gm[b][c] = sd[(long)c * Vh + nb];
+                if constexpr (RED == RED_SADD) src_add(a, gm[b][c], sl[b], (long)c * Vh + nb);
+              }
               if constexpr (P == P16) nm[b] = a.src.norm[(long)sl[b] * a.nstride + nb];
             }
           }
@@ -698,9 +794,25 @@ __device__ __forceinline__ void hop_group(const HopArgs &a, int b0_in, int sb_in
         }
       }
     }
-    hop_epilogue<P, NB, RED, HASX, NT>(a, h, Vh, sl, act, acc, red);
+    hop_epilogue<P, NB, RED, HASX, NT>(a, h, Vh, sl, act, acc, red, ru);
   }
-  if constexpr (RED != RED_NONE) {
+  if constexpr (RU) {
+    const long nchunk = (Vh + 63) / 64;
+    const int chunk = h >> 6;
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      if (!act[b]) continue;
+      const double r2 = wave_sum(ru[b][0]), re = wave_sum(ru[b][1]), im = wave_sum(ru[b][2]);
+      if ((threadIdx.x & 63) == 0 && chunk < nchunk) {
+        const long at = (long)sl[b] * nchunk + chunk;
+        a.r2[at] = r2;
+        if (a.ps.data) {
+          a.re[at] = re;
+          a.im[at] = im;
+        }
+      }
+    }
+  } else if constexpr (RED != RED_NONE && RED != RED_SADD) {
     const long nchunk = (Vh + 63) / 64;
     const int chunk = h >> 6;
 #pragma unroll
@@ -712,23 +824,25 @@ __device__ __forceinline__ void hop_group(const HopArgs &a, int b0_in, int sb_in
   }
 }
 
-// GL (FP64 launches with a compacted slot list): the RHS group is the
-// innermost logical block index (XCD-aware order), so the groups of one site
-// block run side by side and share its links in L2, and the blocks of groups
-// past the listed slots return before any load: an empty list costs a
-// launch of idle blocks.  Otherwise one group and site block per block.
 template <int P, int NL, int NB, int RED, bool HASX, bool NT, bool SGL, bool STG, int LP = P,
-          bool BUF = false, bool GL = false>
+          bool BUF = false>
 __global__ void __launch_bounds__(STG ? 512 : 256)
 hop_kernel(const HopArgs a) {
-  if constexpr (GL) {
-    const int lb = logical_block(a.remap);
-    const int b0 = (lb % a.ngroups) * NB, sb = lb / a.ngroups;
-    if (b0 >= a.slots[0] || sb * (int)blockDim.x >= a.g.Vh) return;
-    hop_group<P, NL, NB, RED, HASX, NT, SGL, STG, LP, BUF>(a, b0, sb);
-  } else {
-    hop_group<P, NL, NB, RED, HASX, NT, SGL, STG, LP, BUF>(a, -1, -1);
-  }
+  hop_group<P, NL, NB, RED, HASX, NT, SGL, STG, LP, BUF>(a, -1, -1);
+}
+
+// The FP64 hop over flagged slots: the RHS group is the innermost logical
+// block index (XCD-aware order), so the groups of one site block run side by
+// side and share its links in L2, and the blocks of groups past the flagged
+// slots return before any load: with no flag set a launch costs its idle
+// blocks.
+template <int NL, int NB, int RED, bool HASX, bool STG>
+__global__ void __launch_bounds__(STG ? 512 : 256)
+hop_flag_kernel(const HopFlagArgs a) {
+  const int lb = logical_block(a.remap);
+  const int b0 = (lb % a.ngroups) * NB, sb = lb / a.ngroups;
+  if (nth_flag(a.flags, a.n, b0) < 0 || sb * (int)blockDim.x >= a.g.Vh) return;
+  hop_group<P64, NL, NB, RED, HASX, false, false, STG, P64, false>(a, b0, sb);
 }
 
 // What changes in the arguments of a one-RHS hop for the other parity
@@ -774,17 +888,10 @@ static size_t stage_bytes(int prec, int nb, int block) {
 // BUF: buffer loads (FP32 / FP16 with double-stored links; launch_hop_args
 // routes lattices whose offsets do not fit to the plain-load instance).
 template <int P, int NL, int NB, bool NT, bool SGL = false, bool STG = false, int LP = P,
-          bool BUF = (P != P64 && !SGL), bool GL = false>
+          bool BUF = (P != P64 && !SGL)>
 static void hop_dispatch_red(const HopArgs &a, dim3 grid, dim3 block, int red,
                              bool hasx, hipStream_t st) {
   const size_t lds = STG ? stage_bytes(P, NB, (int)block.x) : 0;
-  if constexpr (GL) {
-    // compacted slot lists: FP64, no reduction
-    if (hasx) hipLaunchKernelGGL((hop_kernel<P, NL, NB, RED_NONE, true, NT, SGL, STG, LP, BUF, true>), grid, block, lds, st, a);
-    else hipLaunchKernelGGL((hop_kernel<P, NL, NB, RED_NONE, false, NT, SGL, STG, LP, BUF, true>), grid, block, lds, st, a);
-    (void)red;
-    return;
-  }
 #define QOP_LAUNCH(RD, HX) \
   hipLaunchKernelGGL((hop_kernel<P, NL, NB, RD, HX, NT, SGL, STG, LP, BUF>), grid, block, lds, st, a)
   if (red == RED_NONE) { if (hasx) QOP_LAUNCH(RED_NONE, true); else QOP_LAUNCH(RED_NONE, false); }
@@ -809,26 +916,6 @@ static void hop_dispatch_nb(const HopArgs &a, int nb, dim3 grid, dim3 block,
       fatal(__FILE__, __LINE__, "hop: single-stored links exist in FP64 and FP32 only");
     }
     return;
-  }
-  if (a.slots) {
-    if constexpr (P == P64) {
-      if (a.stage) {
-        if constexpr (NL == 16) {
-          if (nb == 2) hop_dispatch_red<P, NL, 2, false, false, true, LP, false, true>(a, grid, block, red, hasx, st);
-          else hop_dispatch_red<P, NL, 4, false, false, true, LP, false, true>(a, grid, block, red, hasx, st);
-        } else {
-          fatal(__FILE__, __LINE__, "hop: LDS staging needs Naik links");
-        }
-        return;
-      }
-      switch (nb) {
-        case 1: hop_dispatch_red<P, NL, 1, false, false, false, LP, false, true>(a, grid, block, red, hasx, st); break;
-        case 2: hop_dispatch_red<P, NL, 2, false, false, false, LP, false, true>(a, grid, block, red, hasx, st); break;
-        case 4: hop_dispatch_red<P, NL, 4, false, false, false, LP, false, true>(a, grid, block, red, hasx, st); break;
-        default: hop_dispatch_red<P, NL, 8, false, false, false, LP, false, true>(a, grid, block, red, hasx, st); break;
-      }
-      return;
-    }
   }
   if (!a.buf) {
     // offsets beyond the buffer range: one RHS per thread, plain loads
@@ -891,18 +978,8 @@ static bool hop_buf_fits(const HopArgs &a, int prec, int nb) {
          ((long)(nb - 1) * a.nstride + Vh) * 4 < lim && 9 * Vh * lesz < lim;
 }
 
-void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
-                     bool hasx, hipStream_t st) {
-  QOP_REQUIRE(nb == 1 || nb == 2 || nb == 4 || nb == 8 || nb == 16, "hop: rhs per thread must be 1,2,4,8,16");
-  QOP_REQUIRE(block % 64 == 0 && block >= 64 && block <= (a.stage ? 512 : 256),
-              "hop: block must be a multiple of 64, 64..256 (512 with LDS staging)");
-  QOP_REQUIRE(red == RED_NONE || hasx || red == RED_OUT2, "hop: RED_X2 / RED_CG need x");
-  QOP_REQUIRE(red != RED_CG || (a.cg_alpha && a.xs.data && prec != P64), "hop: RED_CG needs alpha and xs");
-  QOP_REQUIRE(red != RED_R || a.cg_alpha, "hop: RED_R needs alpha");
-  QOP_REQUIRE(a.n >= 1, "hop: n >= 1");
-  QOP_REQUIRE(!a.slots || (prec == P64 && !a.single && red == RED_NONE && nb <= 8),
-              "hop: a compacted slot list is for FP64 double-stored hops without reductions, at "
-              "most 8 RHS per thread");
+// staging and site order fit the lattice and the kernels
+static void check_hop_order(const HopArgs &a, int prec, int nl, int nb, int block) {
   if (a.stage) {
     QOP_REQUIRE(nl == 16 && nb <= 8 && !a.single && !a.nt && (prec != P64 || nb == 2 || nb == 4),
                 "hop: LDS staging needs Naik links, at most 8 RHS per thread (FP64: 2 or 4) and "
@@ -920,6 +997,19 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
     const int slab = a.g.Vh / a.g.L[0];
     QOP_REQUIRE(a.tile % block == 0 && slab % a.tile == 0, "hop: tile must divide the x0 slab");
   }
+}
+
+void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
+                     bool hasx, hipStream_t st) {
+  QOP_REQUIRE(nb == 1 || nb == 2 || nb == 4 || nb == 8 || nb == 16, "hop: rhs per thread must be 1,2,4,8,16");
+  QOP_REQUIRE(block % 64 == 0 && block >= 64 && block <= (a.stage ? 512 : 256),
+              "hop: block must be a multiple of 64, 64..256 (512 with LDS staging)");
+  QOP_REQUIRE(red == RED_NONE || hasx || red == RED_OUT2, "hop: RED_X2 / RED_CG need x");
+  QOP_REQUIRE(red != RED_CG || (a.cg_alpha && a.xs.data && prec != P64), "hop: RED_CG needs alpha and xs");
+  QOP_REQUIRE(red != RED_R || a.cg_alpha, "hop: RED_R needs alpha");
+  QOP_REQUIRE(a.n >= 1, "hop: n >= 1");
+  QOP_REQUIRE(!a.slots && red < RED_SADD, "hop: slot subsets go through launch_hop_flagged");
+  check_hop_order(a, prec, nl, nb, block);
   // otherwise (or when a.plain asks for it) one RHS per thread with plain loads
   a.buf = hop_buf_fits(a, prec, nb);
   if (prec != P64 && !a.single && !a.buf) {
@@ -930,7 +1020,6 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
   }
   int nblk = (a.g.Vh + block - 1) / block;
   a.ngroups = (a.n + nb - 1) / nb;
-  if (a.slots) a.rhs_inner = 1;  // the GL kernel orders the groups innermost itself
   dim3 grid, blk(block);
   if (a.rhs_inner) {
     int tot = nblk * a.ngroups;
@@ -954,6 +1043,56 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
     if (nl == 16) hop_dispatch_nb<P16, 16>(a, nb, grid, blk, red, hasx, st);
     else hop_dispatch_nb<P16, 8>(a, nb, grid, blk, red, hasx, st);
   }
+  QOP_CHECK_HIP(hipGetLastError());
+}
+
+template <int NL, int NB, bool STG>
+static void hop_flag_launch(const HopFlagArgs &a, dim3 grid, dim3 block, int red, bool hasx, hipStream_t st) {
+  const size_t lds = STG ? stage_bytes(P64, NB, (int)block.x) : 0;
+#define QOP_LAUNCH(RD, HX) hipLaunchKernelGGL((hop_flag_kernel<NL, NB, RD, HX, STG>), grid, block, lds, st, a)
+  if (red == RED_SADD) QOP_LAUNCH(RED_SADD, false);
+  else if (red == RED_RU32) QOP_LAUNCH(RED_RU32, true);
+  else if (red == RED_RU16) QOP_LAUNCH(RED_RU16, true);
+  else if (hasx) QOP_LAUNCH(RED_NONE, true);
+  else QOP_LAUNCH(RED_NONE, false);
+#undef QOP_LAUNCH
+}
+template <int NL>
+static void hop_flag_dispatch(const HopFlagArgs &a, int nb, dim3 grid, dim3 block, int red, bool hasx, hipStream_t st) {
+  if (a.stage) {
+    if constexpr (NL == 16) {
+      if (nb == 2) hop_flag_launch<NL, 2, true>(a, grid, block, red, hasx, st);
+      else hop_flag_launch<NL, 4, true>(a, grid, block, red, hasx, st);
+    } else {
+      fatal(__FILE__, __LINE__, "hop: LDS staging needs Naik links");
+    }
+    return;
+  }
+  switch (nb) {
+    case 1: hop_flag_launch<NL, 1, false>(a, grid, block, red, hasx, st); break;
+    case 2: hop_flag_launch<NL, 2, false>(a, grid, block, red, hasx, st); break;
+    case 4: hop_flag_launch<NL, 4, false>(a, grid, block, red, hasx, st); break;
+    default: hop_flag_launch<NL, 8, false>(a, grid, block, red, hasx, st); break;
+  }
+}
+
+void launch_hop_flagged(HopFlagArgs a, int nl, int nb, int block, int red, bool hasx, hipStream_t st) {
+  QOP_REQUIRE(nb == 1 || nb == 2 || nb == 4 || nb == 8, "hop: rhs per thread of flagged slots must be 1,2,4,8");
+  QOP_REQUIRE(block % 64 == 0 && block >= 64 && block <= (a.stage ? 512 : 256),
+              "hop: block must be a multiple of 64, 64..256 (512 with LDS staging)");
+  QOP_REQUIRE(a.flags && !a.single && a.n >= 1 && (red == RED_NONE || red >= RED_SADD),
+              "hop: flagged slots are for FP64 double-stored hops");
+  QOP_REQUIRE(red != RED_SADD || (a.src_add && !hasx), "hop: RED_SADD needs its increments");
+  QOP_REQUIRE((red != RED_RU32 && red != RED_RU16) ||
+                  (hasx && a.b64 && a.rs.data && a.r2 && (!a.ps.data || (a.re && a.im)) && a.xstride == a.sstride),
+              "hop: reliable update operands");
+  check_hop_order(a, P64, nl, nb, block);
+  const int nblk = (a.g.Vh + block - 1) / block;
+  a.ngroups = (a.n + nb - 1) / nb;
+  int tot = nblk * a.ngroups;
+  if (a.remap) tot = (tot + 7) / 8 * 8;
+  if (nl == 16) hop_flag_dispatch<16>(a, nb, dim3(tot), dim3(block), red, hasx, st);
+  else hop_flag_dispatch<8>(a, nb, dim3(tot), dim3(block), red, hasx, st);
   QOP_CHECK_HIP(hipGetLastError());
 }
 
@@ -1110,7 +1249,7 @@ static void launch_hop_pair(const HopArgs &a0, const HopArgs &b0, int prec, int 
 
 void launch_hop_one(const HopArgs &a, const HopArgs *b, int prec, int nl, int red, bool hasx, hipStream_t st) {
   QOP_REQUIRE(prec == P64 || prec == P32, "hop: the reference path has FP64 or FP32 vectors");
-  QOP_REQUIRE(a.n == 1 && !a.coef && !a.active && !a.slots && red != RED_CG, "hop: one unmasked RHS");
+  QOP_REQUIRE(a.n == 1 && !a.coef && !a.active && !a.slots && red < RED_SADD && red != RED_CG, "hop: one unmasked RHS");
   // Solves, one thread per site / four waves (ms): FP64 8^3x16 4.2 / 3.2,
   // 12^3x24 6.0 / 5.4, 16^3x24 8.3 / 8.4, 16^3x32 13.0 / 13.3; FP32 8^3x16
   // 2.5 / 1.9, 16^3x32 4.5 / 4.2, 16^2x20x32 5.1 / 5.1, 20^3x32 5.9 / 6.3

@@ -33,7 +33,6 @@ MultiShiftBatch::MultiShiftBatch(Links &L, int eo, int capacity, int sloppy_prec
     devbatch_alloc(xm_, lat_, P32, cap_ * ns_);
     devbatch_alloc(x64_, lat_, P64, cap_ * ns_);
     devbatch_alloc(t64_, lat_, P64, cap_);
-    devbatch_alloc(ax64_, lat_, P64, cap_);
     dev_alloc(&ru_, cap_ * sizeof(int));
     QOP_CHECK_HIP(hipMemset(ru_, 0, cap_ * sizeof(int)));
     dev_alloc(&slot_, cap_ * sizeof(MsSlot));
@@ -57,7 +56,10 @@ MultiShiftBatch::MultiShiftBatch(Links &L, int eo, int capacity, int sloppy_prec
     QOP_CHECK_HIP(hipMemcpy(coef_, hc.data(), hc.size() * sizeof(double), hipMemcpyHostToDevice));
     L_.get(hp_);  // convert the links before any graph capture
     L_.get(P64);
-    shape_ = tune_hop(L_, hp_, cap_, ps_, ts_, 1 - eo_);
+    // each hop of the iteration with its own epilogue (the second with alpha 0
+    // while no slot is loaded)
+    shape_ = tune_hop(L_, hp_, cap_, ps_, ts_, 1 - eo_, RED_OUT2);
+    shape2_ = tune_hop(L_, hp_, cap_, ts_, rs_, eo_, RED_CG, &ps_, &xm_);
     ru_shape_ = tune_hop(L_, P64, cap_, x64_, t64_, 1 - eo_);
     sync();
   } catch (const DeviceOutOfMemory &) {
@@ -71,7 +73,7 @@ MultiShiftBatch::~MultiShiftBatch() { release(); }
 void MultiShiftBatch::release() {
   sync();
   graph_.reset();
-  for (DevBatch *b : {&b64_, &rs_, &ps_, &ts_, &pm_, &xm_, &x64_, &t64_, &ax64_}) devbatch_free(*b);
+  for (DevBatch *b : {&b64_, &rs_, &ps_, &ts_, &pm_, &xm_, &x64_, &t64_}) devbatch_free(*b);
   dev_free(ru_);
   dev_free(slot_);
   host_free(slot_h_);
@@ -187,22 +189,23 @@ void MultiShiftBatch::enqueue_iteration() {
   b.cg_alpha = (const double *)((const char *)slot_ + offsetof(MsSlot, beta0));
   b.cg_stride = (int)(sizeof(MsSlot) / sizeof(double));
   b.partial = partC_;
-  launch_hop_args(b, hp_, ls.nl, shape_.nb, shape_.block, RED_CG, true, st);
+  shape2_.apply(b);
+  launch_hop_args(b, hp_, ls.nl, shape2_.nb, shape2_.block, RED_CG, true, st);
   ms_launch_scalarB(slot_, active_, partC_, nch_, cap_, ru_, st);
   ms_launch_update(slot_, active_, sp_, (int)Vh, rs_.slot(0), ps_.slot(0), pm_.slot(0), xm_.slot(0),
                    3 * Vh, 3 * Vh * cap_, cap_, ns_, partB_, st);
   enqueue_reliable_update();
 }
 
-// Masked by ru_: slots without a request skip every kernel (a masked hop group
-// with no flagged slot reads nothing).
+// Slots without a request in ru_ skip every kernel (the hops run over the
+// flagged slots).
 void MultiShiftBatch::enqueue_reliable_update() {
   hipStream_t st = stream();
   LinkSet &ls = L_.get(P64);
   const int opp = 1 - eo_;
   const long Vh = lat_->Vh;
   ms_launch_ru_fold(ru_, (int)Vh, x64_.slot(0), xm_.slot(0), 3 * Vh, cap_, ns_, st);
-  HopArgs a;
+  HopFlagArgs a;
   a.g = lat_->g;
   a.parity = opp;
   a.links = ls.parity_data(lat_, opp);
@@ -212,20 +215,21 @@ void MultiShiftBatch::enqueue_reliable_update() {
   a.sstride = a.dstride = a.xstride = 3 * Vh;
   a.nstride = Vh;
   a.n = cap_;
-  a.active = ru_;
+  a.flags = ru_;
   ru_shape_.apply(a);
-  launch_hop_args(a, P64, ls.nl, ru_shape_.nb, ru_shape_.block, RED_NONE, false, st);
-  HopArgs b = a;
+  launch_hop_flagged(a, ls.nl, ru_shape_.nb, ru_shape_.block, RED_NONE, false, st);
+  HopFlagArgs b = a;
   b.parity = eo_;
   b.links = ls.parity_data(lat_, eo_);
   b.lscale = ls.parity_scale(lat_, eo_);
   b.src = t64_.slot(0);
-  b.dst = ax64_.slot(0);
+  b.dst = VecView{};  // A_0 x is not stored
   b.x = x64_.slot(imin_ * cap_);
-  b.coef = coef_;  // A_0 x = m_0^2 x - D t
-  launch_hop_args(b, P64, ls.nl, ru_shape_.nb, ru_shape_.block, RED_NONE, true, st);
-  ms_launch_ru_resid(ru_, sp_, (int)Vh, b64_.slot(0), ax64_.slot(0), rs_.slot(0), 3 * Vh, cap_,
-                     partC_, st);
+  b.coef = coef_;  // r = b - (m_0^2 x - D t) into rs
+  b.b64 = b64_.data;
+  b.rs = rs_.slot(0);
+  b.r2 = partC_;
+  launch_hop_flagged(b, ls.nl, ru_shape_.nb, ru_shape_.block, sp_ == P16 ? RED_RU16 : RED_RU32, true, st);
   ms_launch_ru_scalar(slot_, ru_, partC_, nch_, cap_, st);
 }
 

@@ -44,12 +44,10 @@ void ms_launch_scalarA(MsSlot *s, const int *active, const double *partA, const 
 void ms_launch_scalarB(MsSlot *s, int *active, const double *partC, int nch, int n, int *ru,
                        hipStream_t st);
 // Reliable update of the slots flagged in ru: fold x64[k] += xs[k], xs[k] = 0
-// for every shift (k = shift * cap + slot); residual r = b - ax into rs with
-// |r|^2 partials; scalars (r2, r2_max, clear the flag).
+// for every shift (k = shift * cap + slot); the scalars after the second
+// masked hop has formed the residual (r2, r2_max, clear the flag).
 void ms_launch_ru_fold(const int *ru, int Vh, VecView x64, VecView xs, long stride, int cap, int ns,
                        hipStream_t st);
-void ms_launch_ru_resid(const int *ru, int prec, int Vh, VecView b64, VecView ax64, VecView rs,
-                        long stride, int cap, double *part, hipStream_t st);
 void ms_launch_ru_scalar(MsSlot *s, int *ru, const double *part, int nch, int n, hipStream_t st);
 void ms_launch_update(const MsSlot *s, const int *active, int prec, int Vh, VecView rs,
                       VecView ps, VecView pm, VecView xm, long stride, long sstride, int cap,
@@ -89,7 +87,7 @@ class MultiShiftBatch {
   DevBatch pm_;  // [ns][cap] sloppy shifted directions (index imin unused)
   DevBatch xm_;  // [ns][cap] FP32 solution increments since the last reliable update
   DevBatch x64_; // [ns][cap] FP64 solutions
-  DevBatch t64_, ax64_;  // [cap] FP64 hop temporaries of the reliable update
+  DevBatch t64_;  // [cap] FP64 hop temporary of the reliable update
   int *ru_ = nullptr;    // [cap] reliable update requested
   HopShape ru_shape_;
   MsSlot *slot_ = nullptr, *slot_h_ = nullptr;
@@ -99,7 +97,7 @@ class MultiShiftBatch {
   double *coef_ = nullptr, *sums_ = nullptr;
   int *zero_status_ = nullptr;
   CapturedGraph graph_;
-  HopShape shape_;
+  HopShape shape_, shape2_;
 };
 
 }  // namespace qop

@@ -131,50 +131,6 @@ ms_ru_fold(const int *ru, int Vh, VecView x64, VecView xs, long stride, int cap)
   }
 }
 
-// r = b - ax (FP64) stored as the sloppy residual, |r|^2 partials
-template <int P>
-__global__ void __launch_bounds__(256)
-ms_ru_resid(const int *ru, int Vh, VecView b64, VecView ax64, VecView rs, long stride,
-            double *part) {
-  using R = typename MT<P>::R;
-  const int b = blockIdx.y;
-  if (!ru[b]) return;
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc = 0;
-  if (h < Vh) {
-    const double2 *bb = (const double2 *)b64.data + (size_t)b * stride;
-    const double2 *aa = (const double2 *)ax64.data + (size_t)b * stride;
-    R r[6];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      const double2 u = bb[c * Vh + h], w = aa[c * Vh + h];
-      const double xr = u.x - w.x, xi = u.y - w.y;
-      acc += xr * xr + xi * xi;
-      r[2 * c] = (R)xr;
-      r[2 * c + 1] = (R)xi;
-    }
-    const size_t cb = sizeof(typename MT<P>::S);
-    char *d = (char *)rs.data + (size_t)b * stride * cb;
-    if constexpr (P == P16) {
-      float *nm = rs.norm + (long)b * Vh;
-      float m = 0.f;
-#pragma unroll
-      for (int i = 0; i < 6; i++) m = fmaxf(m, fabsf(r[i]));
-      const float inv = m > 0.f ? 1.f / m : 0.f;
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-        ((__half2 *)d)[c * Vh + h] = __floats2half2_rn(r[2 * c] * inv, r[2 * c + 1] * inv);
-      nm[h] = m;
-    } else {
-#pragma unroll
-      for (int c = 0; c < 3; c++) ((float2 *)d)[c * Vh + h] = make_float2(r[2 * c], r[2 * c + 1]);
-    }
-  }
-  const int nch = (Vh + 63) / 64;
-  acc = msum(acc);
-  if ((threadIdx.x & 63) == 0 && (h >> 6) < nch) part[(long)b * nch + (h >> 6)] = acc;
-}
-
 // the true |r|^2 replaces the iterated one
 __global__ void __launch_bounds__(1024)
 ms_ru_scalar(MsSlot *S, int *ru, const double *part, int nch) {
@@ -297,13 +253,6 @@ void ms_launch_ru_fold(const int *ru, int Vh, VecView x64, VecView xs, long stri
                        hipStream_t st) {
   hipLaunchKernelGGL(ms_ru_fold, dim3((Vh + 255) / 256, cap * ns), dim3(256), 0, st, ru, Vh, x64, xs,
                      stride, cap);
-  QOP_CHECK_HIP(hipGetLastError());
-}
-void ms_launch_ru_resid(const int *ru, int prec, int Vh, VecView b64, VecView ax64, VecView rs,
-                        long stride, int cap, double *part, hipStream_t st) {
-  dim3 g((Vh + 255) / 256, cap), bl(256);
-  if (prec == P16) hipLaunchKernelGGL(ms_ru_resid<P16>, g, bl, 0, st, ru, Vh, b64, ax64, rs, stride, part);
-  else hipLaunchKernelGGL(ms_ru_resid<P32>, g, bl, 0, st, ru, Vh, b64, ax64, rs, stride, part);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void ms_launch_ru_scalar(MsSlot *s, int *ru, const double *part, int nch, int n, hipStream_t st) {
