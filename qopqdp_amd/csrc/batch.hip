@@ -171,7 +171,7 @@ bs_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, i
 // are part of the hops, the hops find the flagged slots themselves and one
 // kernel updates the search directions of all slots: eight launches per
 // iteration where there were twelve.  Twelve requests at 8x12^2x16 through
-// the server 10.9 -> 8.1 ms, 24 refinements and 4 x 6 multi-shift at 16^3x32
+// the server 10.5 -> 9.1 ms, 24 refinements and 4 x 6 multi-shift at 16^3x32
 // 39.9 -> 36.0 ms, 16 FP16 solves at 24^3x48 unchanged within 1%.
 // x += xs, xs = 0 of the flagged slots
 __global__ void __launch_bounds__(256)

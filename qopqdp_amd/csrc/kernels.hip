@@ -551,7 +551,7 @@ __device__ __forceinline__ void hop_group(const A &a, int b0_in, int sb_in) {
       sl[b] = nth_flag(a.flags, a.n, j);
       act[b] = sl[b] >= 0;
       if (!act[b]) sl[b] = j;
-    } else if (a.slots) {
+    } else if (P == P64 && a.slots) {
       act[b] = j < a.slots[0];
       sl[b] = act[b] ? a.slots[1 + j] : j;
     } else {
@@ -1255,8 +1255,13 @@ void launch_hop_one(const HopArgs &a, const HopArgs *b, int prec, int nl, int re
   // 2.5 / 1.9, 16^3x32 4.5 / 4.2, 16^2x20x32 5.1 / 5.1, 20^3x32 5.9 / 6.3
   const int lim = prec == P64 ? 49152 : 81920;
   if (a.g.Vh > lim || (red == RED_OUT2 && hasx)) {
-    if (b) launch_hop_pair(a, *b, prec, nl, st);
-    else launch_hop_args(a, prec, nl, 1, 256, red, hasx, st);
+    // a launch less does not show above some 50 us per parity
+    if (b && a.g.Vh <= 262144) {
+      launch_hop_pair(a, *b, prec, nl, st);
+    } else {
+      launch_hop_args(a, prec, nl, 1, 256, red, hasx, st);
+      if (b) launch_hop_args(*b, prec, nl, 1, 256, red, hasx, st);
+    }
     return;
   }
   const int nblk = (((a.g.Vh + 63) / 64) + 7) / 8 * 8;
