@@ -1,0 +1,144 @@
+// Block cache of dev_alloc / dev_free and host_alloc / host_free.
+//
+// Solves, link construction and forces take their workspaces at every call;
+// hipMalloc and hipFree of a few GB take tens of milliseconds (one asqtad link
+// construction at 24^3x48: 8.5 ms of kernels in a 69 ms call), so freed blocks
+// are kept and handed out again.
+//  * A freed block may still be in use by work enqueued on any stream.  It is
+//    pending until a device synchronisation after its free (hipFree waits for
+//    the device too) and only then handed out, so a block never passes from
+//    one stream or thread to another with work in flight.  While another
+//    thread captures a stream the device cannot be synchronised: pending
+//    blocks then stay pending and a new block is allocated.
+//  * Bounded: blocks above `block` bytes go back to the driver at once
+//    (calls that use them run long enough that their allocation does not show:
+//    one 32^3x64 link-matrix field, 302 MB, is still kept), and the kept blocks
+//    of a device total at most `total` bytes.
+//  * Given back: at QOP_finalize, when a request server ends, and when
+//    an allocation fails (it is tried again then, and if it still fails the
+//    blocks freed while the failure unwinds are not kept).
+//
+// Api is the memory behind it (runtime.cpp: HIP device or page-locked memory):
+//   int device();                  // the device blocks are allocated on
+//   void *alloc(size_t bytes);     // null: out of memory
+//   void free(void *p);            // waits for the work that uses p
+//   bool try_sync();               // waits for all work of the device; false: not possible now
+//   [[noreturn]] void out_of_memory(size_t bytes);
+#pragma once
+#include <cstddef>
+#include <map>
+#include <mutex>
+#include <utility>
+
+namespace qop {
+
+template <class Api>
+class BlockCache {
+ public:
+  BlockCache(Api api, size_t block, size_t total) : api_(api), block_(block), total_(total) {}
+  void *alloc(size_t bytes) {
+    const int dev = api_.device();
+    const size_t want = bytes <= block_ ? round(bytes) : bytes;
+    std::lock_guard<std::mutex> lk(mu_);
+    void *p = nullptr;
+    if (want <= block_) {
+      p = take(ready_, dev, want);
+      if (!p && fits(pending_, dev, want)) {
+        if (api_.try_sync()) settle(dev);
+        p = take(ready_, dev, want);
+      }
+    }
+    if (!p) {
+      p = api_.alloc(want);
+      if (!p) {
+        trim_locked();
+        p = api_.alloc(want);
+      }
+      if (!p) {
+        failed_ = true;
+        api_.out_of_memory(bytes);
+      }
+      if (want <= block_) live_[p] = Block{want, dev};
+    }
+    failed_ = false;
+    return p;
+  }
+  void free(void *p) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(mu_);
+    auto it = live_.find(p);
+    if (it == live_.end() || failed_ || kept_ + it->second.bytes > total_) {
+      if (it != live_.end()) live_.erase(it);
+      api_.free(p);
+      return;
+    }
+    kept_ += it->second.bytes;
+    pending_.emplace(it->second.bytes, std::make_pair(p, it->second.dev));
+    live_.erase(it);
+  }
+  void trim() {
+    std::lock_guard<std::mutex> lk(mu_);
+    trim_locked();
+  }
+  size_t kept() {
+    std::lock_guard<std::mutex> lk(mu_);
+    return kept_;
+  }
+
+ private:
+  struct Block {
+    size_t bytes;
+    int dev;
+  };
+  using Kept = std::multimap<size_t, std::pair<void *, int>>;
+  // whole 512-byte units, and 1/16 of the size for large blocks, so nearby
+  // sizes share blocks
+  static size_t round(size_t bytes) {
+    size_t unit = 512;
+    while (unit * 16 < bytes) unit *= 2;
+    return bytes ? (bytes + unit - 1) / unit * unit : unit;
+  }
+  // a kept block of at least `want` bytes and at most 1/8 more
+  static Kept::iterator find(Kept &k, int dev, size_t want) {
+    for (auto it = k.lower_bound(want); it != k.end() && it->first <= want + want / 8; ++it)
+      if (it->second.second == dev) return it;
+    return k.end();
+  }
+  static bool fits(Kept &k, int dev, size_t want) { return find(k, dev, want) != k.end(); }
+  void *take(Kept &k, int dev, size_t want) {
+    auto it = find(k, dev, want);
+    if (it == k.end()) return nullptr;
+    void *p = it->second.first;
+    live_[p] = Block{it->first, dev};
+    kept_ -= it->first;
+    k.erase(it);
+    return p;
+  }
+  // the pending blocks of a device that has been synchronised
+  void settle(int dev) {
+    for (auto it = pending_.begin(); it != pending_.end();) {
+      if (it->second.second == dev) {
+        ready_.insert(*it);
+        it = pending_.erase(it);
+      } else {
+        ++it;
+      }
+    }
+  }
+  void trim_locked() {
+    for (Kept *k : {&ready_, &pending_}) {
+      for (auto &b : *k) api_.free(b.second.first);
+      k->clear();
+    }
+    kept_ = 0;
+  }
+  Api api_;
+  const size_t block_, total_;
+  std::mutex mu_;
+  Kept ready_, pending_;
+  std::map<void *, Block> live_;
+  size_t kept_ = 0;
+  bool failed_ = false;  // the last allocation failed: its frees are not kept
+};
+
+}  // namespace qop

@@ -54,7 +54,7 @@ template <class T>
 inline void dev_alloc(T **p, size_t bytes) {
   dev_alloc_bytes((void **)p, bytes);
 }
-// Gives memory of dev_alloc back (to the block cache of runtime.cpp: work
+// Gives memory of dev_alloc back (to the block cache, block_cache.h: work
 // enqueued before the call may still use it).
 void dev_free(void *p);
 // Page-locked host memory of the solvers' status words and staging.
@@ -66,6 +66,11 @@ inline void host_alloc(T **p, size_t bytes) {
 void host_free(void *p);
 void cache_trim();         // kept blocks go back to the driver
 size_t dev_cache_bytes();  // device memory held in kept blocks
+// Captures of a stream (thread-local mode) and waits for the whole device
+// exclude each other across threads.
+void capture_begin(hipStream_t st);
+hipGraph_t capture_end(hipStream_t st);
+void device_sync();
 // Owning device buffer for temporaries: freed when it goes out of scope,
 // also while a DeviceOutOfMemory unwinds.
 template <class T>
@@ -98,10 +103,10 @@ struct CapturedGraph {
   explicit operator bool() const { return exec != nullptr; }
   void begin(hipStream_t st) {
     reset();
-    QOP_CHECK_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    capture_begin(st);
   }
   void end(hipStream_t st) {
-    QOP_CHECK_HIP(hipStreamEndCapture(st, &graph));
+    graph = capture_end(st);
     QOP_CHECK_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
   }
   void launch(hipStream_t st) const { QOP_CHECK_HIP(hipGraphLaunch(exec, st)); }

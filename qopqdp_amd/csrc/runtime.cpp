@@ -3,6 +3,8 @@
 #include <map>
 #include <mutex>
 
+#include "block_cache.h"
+#include "capture_gate.h"
 #include "common.h"
 #include "eigcg.h"
 
@@ -15,153 +17,69 @@ namespace qop {
 }
 
 // ---------------------------------------------------------------------------
-// Block cache of dev_alloc / dev_free and host_alloc / host_free.
-//
-// Solves, link construction and forces take their workspaces at every call;
-// hipMalloc and hipFree of a few GB take tens of milliseconds (one asqtad link
-// construction at 24^3x48: 8.5 ms of kernels in a 69 ms call), so freed blocks
-// are kept and handed out again.
-//  * A freed block may still be in use by work enqueued on any stream.  It is
-//    pending until a device synchronisation after its free (hipFree waits for
-//    the device too) and only then handed out, so a block never passes from
-//    one stream or thread to another with work in flight.
-//  * Bounded: blocks above CACHE_BLOCK bytes go back to the driver at once
-//    (calls that use them run long enough that their allocation does not show:
-//    one 32^3x64 link-matrix field, 302 MB, is still kept), and the kept blocks
-//    of a device total at most CACHE_TOTAL bytes.
-//  * Given back: at QOP_finalize, when a request server ends, and when
-//    an allocation fails (it is tried again then, and if it still fails the
-//    blocks freed while the failure unwinds are not kept).
+// stream captures and device synchronisations (capture_gate.h)
+static CaptureGate &capture_gate() {
+  static CaptureGate *g = new CaptureGate;
+  return *g;
+}
+void capture_begin(hipStream_t st) {
+  capture_gate().capture_begin();
+  QOP_CHECK_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+}
+hipGraph_t capture_end(hipStream_t st) {
+  hipGraph_t g = nullptr;
+  const hipError_t e = hipStreamEndCapture(st, &g);
+  capture_gate().capture_end();
+  QOP_CHECK_HIP(e);
+  return g;
+}
+static bool device_sync_gated(bool wait) {
+  if (!capture_gate().sync_begin(wait)) return false;
+  const hipError_t e = hipDeviceSynchronize();
+  capture_gate().sync_end();
+  QOP_CHECK_HIP(e);
+  return true;
+}
+void device_sync() { (void)device_sync_gated(true); }
+
+// ---------------------------------------------------------------------------
+// device and page-locked memory (block_cache.h)
 namespace {
 constexpr size_t CACHE_BLOCK = (size_t)384 << 20, CACHE_TOTAL = (size_t)8 << 30;
 constexpr size_t CACHE_HOST_BLOCK = (size_t)1 << 20, CACHE_HOST_TOTAL = (size_t)64 << 20;
 
-class BlockCache {
- public:
-  BlockCache(bool host, size_t block, size_t total) : host_(host), block_(block), total_(total) {}
-  void *alloc(size_t bytes) {
+struct HipMemory {
+  bool host;
+  int device() {
     int dev = 0;
     QOP_CHECK_HIP(hipGetDevice(&dev));
-    const size_t want = bytes <= block_ ? round(bytes) : bytes;
-    std::lock_guard<std::mutex> lk(mu_);
+    return dev;
+  }
+  void *alloc(size_t n) {
     void *p = nullptr;
-    if (want <= block_) {
-      p = take(ready_, dev, want);
-      if (!p && fits(pending_, dev, want)) {
-        QOP_CHECK_HIP(hipDeviceSynchronize());
-        settle(dev);
-        p = take(ready_, dev, want);
-      }
+    const hipError_t e = host ? hipHostMalloc(&p, n, hipHostMallocDefault) : hipMalloc(&p, n);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();  // clear the error state of this thread
+      return nullptr;
     }
-    if (!p) {
-      hipError_t e = raw_alloc(&p, want);
-      if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();  // clear the error state of this thread
-        trim_locked();
-        e = raw_alloc(&p, want);
-      }
-      if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        failed_ = true;
-        throw DeviceOutOfMemory{bytes};
-      }
-      if (e != hipSuccess) fatal(__FILE__, __LINE__, hipGetErrorString(e));
-      if (want <= block_) live_[p] = Block{want, dev};
-    }
-    failed_ = false;
+    QOP_CHECK_HIP(e);
     return p;
   }
   void free(void *p) {
-    if (!p) return;
-    std::lock_guard<std::mutex> lk(mu_);
-    auto it = live_.find(p);
-    if (it == live_.end() || failed_ || kept_ + it->second.bytes > total_) {
-      if (it != live_.end()) live_.erase(it);
-      raw_free(p);
-      return;
-    }
-    kept_ += it->second.bytes;
-    pending_.emplace(it->second.bytes, std::make_pair(p, it->second.dev));
-    live_.erase(it);
+    if (host) QOP_CHECK_HIP(hipHostFree(p));
+    else QOP_CHECK_HIP(hipFree(p));
   }
-  void trim() {
-    std::lock_guard<std::mutex> lk(mu_);
-    trim_locked();
-  }
-  size_t kept() {
-    std::lock_guard<std::mutex> lk(mu_);
-    return kept_;
-  }
-
- private:
-  struct Block {
-    size_t bytes;
-    int dev;
-  };
-  using Kept = std::multimap<size_t, std::pair<void *, int>>;
-  // whole 512-byte units, and 1/16 of the size for large blocks, so nearby
-  // sizes share blocks
-  static size_t round(size_t bytes) {
-    size_t unit = 512;
-    while (unit * 16 < bytes) unit *= 2;
-    return bytes ? (bytes + unit - 1) / unit * unit : unit;
-  }
-  // a kept block of at least `want` bytes and at most 1/8 more
-  static Kept::iterator find(Kept &k, int dev, size_t want) {
-    for (auto it = k.lower_bound(want); it != k.end() && it->first <= want + want / 8; ++it)
-      if (it->second.second == dev) return it;
-    return k.end();
-  }
-  static bool fits(Kept &k, int dev, size_t want) { return find(k, dev, want) != k.end(); }
-  void *take(Kept &k, int dev, size_t want) {
-    auto it = find(k, dev, want);
-    if (it == k.end()) return nullptr;
-    void *p = it->second.first;
-    live_[p] = Block{it->first, dev};
-    kept_ -= it->first;
-    k.erase(it);
-    return p;
-  }
-  // the pending blocks of a device that has been synchronised
-  void settle(int dev) {
-    for (auto it = pending_.begin(); it != pending_.end();) {
-      if (it->second.second == dev) {
-        ready_.insert(*it);
-        it = pending_.erase(it);
-      } else {
-        ++it;
-      }
-    }
-  }
-  hipError_t raw_alloc(void **p, size_t n) const {
-    return host_ ? hipHostMalloc(p, n, hipHostMallocDefault) : hipMalloc(p, n);
-  }
-  void raw_free(void *p) const {
-    if (host_) QOP_CHECK_HIP(hipHostFree(p));
-    else QOP_CHECK_HIP(hipFree(p));  // waits for the work that uses it
-  }
-  void trim_locked() {
-    for (Kept *k : {&ready_, &pending_}) {
-      for (auto &b : *k) raw_free(b.second.first);
-      k->clear();
-    }
-    kept_ = 0;
-  }
-  const bool host_;
-  const size_t block_, total_;
-  std::mutex mu_;
-  Kept ready_, pending_;
-  std::map<void *, Block> live_;
-  size_t kept_ = 0;
-  bool failed_ = false;  // the last allocation failed: its frees are not kept
+  bool try_sync() { return device_sync_gated(false); }
+  [[noreturn]] void out_of_memory(size_t bytes) { throw DeviceOutOfMemory{bytes}; }
 };
+using Cache = BlockCache<HipMemory>;
 // never destroyed: owners with static lifetime may free after main
-BlockCache &dev_cache() {
-  static BlockCache *c = new BlockCache(false, CACHE_BLOCK, CACHE_TOTAL);
+Cache &dev_cache() {
+  static Cache *c = new Cache(HipMemory{false}, CACHE_BLOCK, CACHE_TOTAL);
   return *c;
 }
-BlockCache &host_cache() {
-  static BlockCache *c = new BlockCache(true, CACHE_HOST_BLOCK, CACHE_HOST_TOTAL);
+Cache &host_cache() {
+  static Cache *c = new Cache(HipMemory{true}, CACHE_HOST_BLOCK, CACHE_HOST_TOTAL);
   return *c;
 }
 }  // namespace

@@ -1,0 +1,24 @@
+"""The block cache behind device allocations and the gate between stream
+captures and device synchronisations, on the CPU: tests/block_cache_host.cpp
+runs both over a memory that counts allocations, frees and synchronisations."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("block_cache") / "block_cache_host")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-Wall",
+                    "-I", os.path.join(HERE, "..", "qopqdp_amd", "csrc"),
+                    os.path.join(HERE, "block_cache_host.cpp"), "-o", exe], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("check", ["no_sync_in_capture", "captures_and_syncs_exclude_each_other"])
+def test_block_cache(program, check):
+    r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
