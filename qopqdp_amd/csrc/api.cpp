@@ -180,7 +180,7 @@ QOP_status_t QOP_init(QOP_layout_t *layout) {
 
 QOP_status_t QOP_finalize(void) {
   CHECK_INIT;
-  device_sync();
+  QOP_CHECK_HIP(hipDeviceSynchronize());
   cache_trim();
   G.inited = 0;
   return QOP_SUCCESS;

@@ -229,7 +229,7 @@ BatchSolver::BatchSolver(Links &L, int eo, int capacity, int sloppy_prec, double
     QOP_CHECK_HIP(hipMemcpyAsync(glob_, glob_h_, sizeof(BsGlobal), hipMemcpyHostToDevice, st_));
     loaded_.assign(cap_, 0);
     mass_.assign(cap_, 0.0);
-    // Build the sloppy and FP64 link sets now: the iteration is captured into
+    // Build the sloppy and FP64 link sets now: the iteration is recorded into
     // a graph later, and a conversion (allocation, host sync) cannot run then.
     L_.get(sp_);
     L_.get(P64);
@@ -516,9 +516,9 @@ void BatchSolver::enqueue_iteration() {
 void BatchSolver::build_graph() {
   const int chunk = options().chunk > 0 ? options().chunk : 16;
   if (graph_ && graph_chunk_ == chunk) return;
-  graph_.begin(st_);
+  graph_.begin();
   for (int c = 0; c < chunk; c++) enqueue_iteration();
-  graph_.end(st_);
+  graph_.end();
   graph_chunk_ = chunk;
 }
 

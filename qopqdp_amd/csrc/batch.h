@@ -168,7 +168,7 @@ class BatchSolver {
   double *hc_h_ = nullptr;      // pinned staging of the loaded slots' hop coefficients
   std::vector<int> loaded_;
   std::vector<double> mass_;
-  CapturedGraph graph_;
+  LaunchGraph graph_;
   int graph_chunk_ = 0;
   HopShape shape_;     // tuned launch shape of the first sloppy hop
   HopShape shape2_;    // tuned launch shape of the second (fused CG update)

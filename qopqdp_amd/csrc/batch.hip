@@ -166,7 +166,7 @@ bs_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, i
 //   stop / continue, beta                        (bs_ru_scalar)
 //   ps = (1 - beta <rs,ps>/|r|^2) rs + beta ps   (bs_pnext)
 // Unflagged slots skip every step, so a slot's arithmetic is the same
-// whatever the other slots do.  Every launch is in the captured iteration and
+// whatever the other slots do.  Every launch is in the recorded iteration and
 // costs a few microseconds also when no slot is flagged, so the vector steps
 // are part of the hops, the hops find the flagged slots themselves and one
 // kernel updates the search directions of all slots: eight launches per
@@ -298,38 +298,38 @@ bs_sum(const double *part, int nch, const int *sel, double *out) {
 
 void bs_launch_scalar1(BsRhs *rhs, const int *active, const int *status, const double *partA,
                        const double *partB, int nch, int n, int *ru_cont, hipStream_t st) {
-  hipLaunchKernelGGL(bs_scalar1, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, status, partA, partB, nch, ru_cont);
+  launch_kernel(bs_scalar1, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, status, partA, partB, nch, ru_cont);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, int nch,
                        int n, int *ru, hipStream_t st) {
-  hipLaunchKernelGGL(bs_scalar2, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, glob, partC, nch, ru);
+  launch_kernel(bs_scalar2, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, glob, partC, nch, ru);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_ru_join(BsRhs *rhs, const int *active, int *ru, int n, hipStream_t st) {
-  hipLaunchKernelGGL(bs_ru_join, dim3(1), dim3(64), 0, st, rhs, active, ru, n);
+  launch_kernel(bs_ru_join, dim3(1), dim3(64), 0, st, rhs, active, ru, n);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_pnext(const BsRhs *rhs, const int *active, const int *status, const int *ru_cont,
                      const double *lcoef, int prec, int Vh, VecView rs, VecView ps, long stride, int n,
                      double *partB, hipStream_t st) {
   dim3 g((Vh + 255) / 256, n), bl(256);
-  if (prec == P32) hipLaunchKernelGGL(bs_pnext<P32>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
-  else hipLaunchKernelGGL(bs_pnext<P16>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
+  if (prec == P32) launch_kernel(bs_pnext<P32>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
+  else launch_kernel(bs_pnext<P16>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_sum(const double *part, int nch, int n, const int *sel, double *out, hipStream_t st) {
-  hipLaunchKernelGGL(bs_sum, dim3(n), dim3(BS_THREADS), 0, st, part, nch, sel, out);
+  launch_kernel(bs_sum, dim3(n), dim3(BS_THREADS), 0, st, part, nch, sel, out);
   QOP_CHECK_HIP(hipGetLastError());
 }
 
 void bs_launch_ru_x(const int *ru, int n, int Vh, VecView x64, VecView xs, long stride, hipStream_t st) {
-  hipLaunchKernelGGL(bs_ru_x, dim3((Vh + 255) / 256), dim3(256), 0, st, ru, n, Vh, x64, xs, stride);
+  launch_kernel(bs_ru_x, dim3((Vh + 255) / 256), dim3(256), 0, st, ru, n, Vh, x64, xs, stride);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_ru_scalar(BsRhs *rhs, int *active, int *ru, int *ru_cont, double *lcoef, const double *pr2,
                          const double *pre, const double *pim, int nch, int n, hipStream_t st) {
-  hipLaunchKernelGGL(bs_ru_scalar, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, ru, ru_cont, lcoef, pr2, pre, pim, nch);
+  launch_kernel(bs_ru_scalar, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, ru, ru_cont, lcoef, pr2, pre, pim, nch);
   QOP_CHECK_HIP(hipGetLastError());
 }
 

@@ -7,9 +7,9 @@
 //  * A freed block may still be in use by work enqueued on any stream.  It is
 //    pending until a device synchronisation after its free (hipFree waits for
 //    the device too) and only then handed out, so a block never passes from
-//    one stream or thread to another with work in flight.  While another
-//    thread captures a stream the device cannot be synchronised: pending
-//    blocks then stay pending and a new block is allocated.
+//    one stream or thread to another with work in flight.  Where the device
+//    cannot be synchronised now, pending blocks stay pending and a new block
+//    is allocated.
 //  * Bounded: blocks above `block` bytes go back to the driver at once
 //    (calls that use them run long enough that their allocation does not show:
 //    one 32^3x64 link-matrix field, 302 MB, is still kept), and the kept blocks

@@ -230,24 +230,24 @@ cgms_xp(CgmsDev d, int Vh, VecView r, int ns, int what) {
 }
 
 void cgms_launch_scalarA(CgmsDev d, int nch, hipStream_t st) {
-  hipLaunchKernelGGL(cgms_scalarA, dim3(1), dim3(SUM_THREADS), 0, st, d, nch);
+  launch_kernel(cgms_scalarA, dim3(1), dim3(SUM_THREADS), 0, st, d, nch);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void cgms_launch_relnorm(CgmsDev d, int prec, int Vh, VecView r, VecView x,
                          hipStream_t st) {
   dim3 g((Vh + 255) / 256), b(256);
-  if (prec == P64) hipLaunchKernelGGL(cgms_relnorm<P64>, g, b, 0, st, d, Vh, r, x);
-  else hipLaunchKernelGGL(cgms_relnorm<P32>, g, b, 0, st, d, Vh, r, x);
+  if (prec == P64) launch_kernel(cgms_relnorm<P64>, g, b, 0, st, d, Vh, r, x);
+  else launch_kernel(cgms_relnorm<P32>, g, b, 0, st, d, Vh, r, x);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void cgms_launch_scalarB(CgmsDev d, int nch, int with_rel, int Vh, hipStream_t st) {
-  hipLaunchKernelGGL(cgms_scalarB, dim3(1), dim3(SUM_THREADS), 0, st, d, nch, with_rel, Vh);
+  launch_kernel(cgms_scalarB, dim3(1), dim3(SUM_THREADS), 0, st, d, nch, with_rel, Vh);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void cgms_launch_xp(CgmsDev d, int prec, int Vh, VecView r, int ns, int what, hipStream_t st) {
   dim3 g((Vh + 255) / 256), b(256);
-  if (prec == P64) hipLaunchKernelGGL(cgms_xp<P64>, g, b, 0, st, d, Vh, r, ns, what);
-  else hipLaunchKernelGGL(cgms_xp<P32>, g, b, 0, st, d, Vh, r, ns, what);
+  if (prec == P64) launch_kernel(cgms_xp<P64>, g, b, 0, st, d, Vh, r, ns, what);
+  else launch_kernel(cgms_xp<P32>, g, b, 0, st, d, Vh, r, ns, what);
   QOP_CHECK_HIP(hipGetLastError());
 }
 

@@ -23,6 +23,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <string>
+#include <tuple>
+#include <utility>
 #include <vector>
 
 namespace qop {
@@ -66,11 +68,6 @@ inline void host_alloc(T **p, size_t bytes) {
 void host_free(void *p);
 void cache_trim();         // kept blocks go back to the driver
 size_t dev_cache_bytes();  // device memory held in kept blocks
-// Captures of a stream (thread-local mode) and waits for the whole device
-// exclude each other across threads.
-void capture_begin(hipStream_t st);
-hipGraph_t capture_end(hipStream_t st);
-void device_sync();
 // Owning device buffer for temporaries: freed when it goes out of scope,
 // also while a DeviceOutOfMemory unwinds.
 template <class T>
@@ -90,33 +87,74 @@ struct DevBuf {
   }
 };
 
-// A stream-captured hipGraph and its executable instance, owned together:
-// the captured graph lives as long as the instance made from it and both are
+// A chain of kernel launches as a hipGraph and its executable instance, owned
+// together: the graph lives as long as the instance made from it and both are
 // destroyed in one place (instance first), also while an exception unwinds.
-struct CapturedGraph {
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  CapturedGraph() = default;
-  CapturedGraph(const CapturedGraph &) = delete;
-  CapturedGraph &operator=(const CapturedGraph &) = delete;
-  ~CapturedGraph() { reset(); }
-  explicit operator bool() const { return exec != nullptr; }
-  void begin(hipStream_t st) {
+// Between begin() and end() the launch_kernel() calls of this thread become
+// the chain's nodes instead of running.  No stream is captured for it: while
+// one is, no thread of the process may wait for the device or copy on the
+// default stream, and work that another thread enqueues on it is recorded
+// too, but the library stream and the device are shared between a program's
+// calls and the worker of a request server.
+class LaunchGraph {
+ public:
+  LaunchGraph() = default;
+  LaunchGraph(const LaunchGraph &) = delete;
+  LaunchGraph &operator=(const LaunchGraph &) = delete;
+  ~LaunchGraph() { reset(); }
+  explicit operator bool() const { return exec_ != nullptr; }
+  static LaunchGraph *&recording() {
+    static thread_local LaunchGraph *r = nullptr;
+    return r;
+  }
+  void begin() {
     reset();
-    capture_begin(st);
+    QOP_REQUIRE(!recording(), "launch graphs do not nest");
+    QOP_CHECK_HIP(hipGraphCreate(&graph_, 0));
+    recording() = this;
   }
-  void end(hipStream_t st) {
-    graph = capture_end(st);
-    QOP_CHECK_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+  void add(const void *kernel, dim3 grid, dim3 block, size_t lds, void **args) {
+    hipKernelNodeParams p{};
+    p.func = const_cast<void *>(kernel);
+    p.gridDim = grid;
+    p.blockDim = block;
+    p.sharedMemBytes = (unsigned)lds;
+    p.kernelParams = args;  // copied into the node
+    hipGraphNode_t prev = last_;
+    QOP_CHECK_HIP(hipGraphAddKernelNode(&last_, graph_, prev ? &prev : nullptr, prev ? 1 : 0, &p));
   }
-  void launch(hipStream_t st) const { QOP_CHECK_HIP(hipGraphLaunch(exec, st)); }
+  void end() {
+    recording() = nullptr;
+    QOP_CHECK_HIP(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0));
+  }
+  void launch(hipStream_t st) const { QOP_CHECK_HIP(hipGraphLaunch(exec_, st)); }
   void reset() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    exec = nullptr;
-    graph = nullptr;
+    if (recording() == this) recording() = nullptr;
+    if (exec_) (void)hipGraphExecDestroy(exec_);
+    if (graph_) (void)hipGraphDestroy(graph_);
+    exec_ = nullptr;
+    graph_ = nullptr;
+    last_ = nullptr;
   }
+
+ private:
+  hipGraph_t graph_ = nullptr;
+  hipGraphExec_t exec_ = nullptr;
+  hipGraphNode_t last_ = nullptr;
 };
+
+// A kernel launch on st, or a node of the graph this thread records.
+template <class... P, class... A>
+inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, A &&...args) {
+  std::tuple<P...> v(std::forward<A>(args)...);
+  std::apply(
+      [&](P &...p) {
+        void *ptrs[] = {(void *)&p...};
+        if (LaunchGraph *r = LaunchGraph::recording()) r->add((const void *)kernel, grid, block, lds, ptrs);
+        else QOP_CHECK_HIP(hipLaunchKernel((const void *)kernel, grid, block, ptrs, lds, st));
+      },
+      v);
+}
 
 // Lattice geometry passed by value to kernels.
 struct Geom {

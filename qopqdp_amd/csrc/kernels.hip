@@ -893,7 +893,7 @@ static void hop_dispatch_red(const HopArgs &a, dim3 grid, dim3 block, int red,
                              bool hasx, hipStream_t st) {
   const size_t lds = STG ? stage_bytes(P, NB, (int)block.x) : 0;
 #define QOP_LAUNCH(RD, HX) \
-  hipLaunchKernelGGL((hop_kernel<P, NL, NB, RD, HX, NT, SGL, STG, LP, BUF>), grid, block, lds, st, a)
+  launch_kernel((hop_kernel<P, NL, NB, RD, HX, NT, SGL, STG, LP, BUF>), grid, block, lds, st, a)
   if (red == RED_NONE) { if (hasx) QOP_LAUNCH(RED_NONE, true); else QOP_LAUNCH(RED_NONE, false); }
   else if (red == RED_OUT2) { if (hasx) QOP_LAUNCH(RED_OUT2, true); else QOP_LAUNCH(RED_OUT2, false); }
   else if (red == RED_CG) { QOP_LAUNCH(RED_CG, true); }
@@ -1049,7 +1049,7 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
 template <int NL, int NB, bool STG>
 static void hop_flag_launch(const HopFlagArgs &a, dim3 grid, dim3 block, int red, bool hasx, hipStream_t st) {
   const size_t lds = STG ? stage_bytes(P64, NB, (int)block.x) : 0;
-#define QOP_LAUNCH(RD, HX) hipLaunchKernelGGL((hop_flag_kernel<NL, NB, RD, HX, STG>), grid, block, lds, st, a)
+#define QOP_LAUNCH(RD, HX) launch_kernel((hop_flag_kernel<NL, NB, RD, HX, STG>), grid, block, lds, st, a)
   if (red == RED_SADD) QOP_LAUNCH(RED_SADD, false);
   else if (red == RED_RU32) QOP_LAUNCH(RED_RU32, true);
   else if (red == RED_RU16) QOP_LAUNCH(RED_RU16, true);
@@ -1220,7 +1220,7 @@ hop_split_kernel(const HopArgs a0, const PairOffs o2) {
 
 template <int P, int NL, bool SGL>
 static void hop_split_launch(const HopArgs &a, const PairOffs &b, dim3 grid, int red, bool hasx, hipStream_t st) {
-#define QOP_LAUNCH(RD, HX) hipLaunchKernelGGL((hop_split_kernel<P, NL, RD, HX, SGL>), grid, dim3(256), 0, st, a, b)
+#define QOP_LAUNCH(RD, HX) launch_kernel((hop_split_kernel<P, NL, RD, HX, SGL>), grid, dim3(256), 0, st, a, b)
   if (red == RED_NONE) { if (hasx) QOP_LAUNCH(RED_NONE, true); else QOP_LAUNCH(RED_NONE, false); }
   else if (red == RED_OUT2) QOP_LAUNCH(RED_OUT2, false);
   else if (red == RED_R) QOP_LAUNCH(RED_R, true);
@@ -1237,9 +1237,9 @@ static void launch_hop_pair(const HopArgs &a0, const HopArgs &b0, int prec, int 
   const dim3 grid(nblk, 2), blk(256);
 #define QOP_PAIR(P_, NL_)                                                                                     \
   do {                                                                                                        \
-    if (a.single) hipLaunchKernelGGL((hop_pair_kernel<P_, NL_, true, false>), grid, blk, 0, st, a, b);        \
-    else if (a.buf) hipLaunchKernelGGL((hop_pair_kernel<P_, NL_, false, P_ != P64>), grid, blk, 0, st, a, b); \
-    else hipLaunchKernelGGL((hop_pair_kernel<P_, NL_, false, false>), grid, blk, 0, st, a, b);                \
+    if (a.single) launch_kernel((hop_pair_kernel<P_, NL_, true, false>), grid, blk, 0, st, a, b);        \
+    else if (a.buf) launch_kernel((hop_pair_kernel<P_, NL_, false, P_ != P64>), grid, blk, 0, st, a, b); \
+    else launch_kernel((hop_pair_kernel<P_, NL_, false, false>), grid, blk, 0, st, a, b);                \
   } while (0)
   if (prec == P64) { if (nl == 16) QOP_PAIR(P64, 16); else QOP_PAIR(P64, 8); }
   else { if (nl == 16) QOP_PAIR(P32, 16); else QOP_PAIR(P32, 8); }
@@ -1296,7 +1296,7 @@ finalize_kernel(const double *partial, int m, int nval, double *result,
 
 void launch_finalize(const double *partial, int m, int n, double *result,
                      hipStream_t st, const int *status) {
-  hipLaunchKernelGGL(finalize_kernel, dim3(n), dim3(256), 0, st, partial, m, n,
+  launch_kernel(finalize_kernel, dim3(n), dim3(256), 0, st, partial, m, n,
                      result, status);
   QOP_CHECK_HIP(hipGetLastError());
 }
@@ -1363,7 +1363,7 @@ lincomb_kernel(const LincombArgs a) {
 template <int PO, int P0, int P1, int P2>
 static void lincomb_dispatch2(const LincombArgs &a, int nin, bool red, dim3 g,
                               dim3 bl, hipStream_t st) {
-#define QOP_L(N, RD) hipLaunchKernelGGL((lincomb_kernel<PO, P0, P1, P2, N, RD>), g, bl, 0, st, a)
+#define QOP_L(N, RD) launch_kernel((lincomb_kernel<PO, P0, P1, P2, N, RD>), g, bl, 0, st, a)
   if (nin == 1) { if (red) QOP_L(1, true); else QOP_L(1, false); }
   else if (nin == 2) { if (red) QOP_L(2, true); else QOP_L(2, false); }
   else { if (red) QOP_L(3, true); else QOP_L(3, false); }
@@ -1472,20 +1472,20 @@ void launch_dot(const DotArgs &a, int pu, int pv, int mode, hipStream_t st) {
   if (mode == 2) {
     dim3 g((a.Vh + 255) / 256, a.n), bl(256);
     QOP_REQUIRE(pu == pv, "relnorm: precisions must match");
-    if (pu == P64) hipLaunchKernelGGL((relnorm_kernel<P64>), g, bl, 0, st, a);
-    else if (pu == P32) hipLaunchKernelGGL((relnorm_kernel<P32>), g, bl, 0, st, a);
-    else hipLaunchKernelGGL((relnorm_kernel<P16>), g, bl, 0, st, a);
+    if (pu == P64) launch_kernel((relnorm_kernel<P64>), g, bl, 0, st, a);
+    else if (pu == P32) launch_kernel((relnorm_kernel<P32>), g, bl, 0, st, a);
+    else launch_kernel((relnorm_kernel<P16>), g, bl, 0, st, a);
     QOP_CHECK_HIP(hipGetLastError());
     return;
   }
   dim3 g((a.Vh + 255) / 256, a.n), bl(256);
 #define QOP_D(PU_, PV_, M_) \
-  if (pu == PU_ && pv == PV_ && mode == M_) { hipLaunchKernelGGL((dot_kernel<PU_, PV_, M_>), g, bl, 0, st, a); QOP_CHECK_HIP(hipGetLastError()); return; }
+  if (pu == PU_ && pv == PV_ && mode == M_) { launch_kernel((dot_kernel<PU_, PV_, M_>), g, bl, 0, st, a); QOP_CHECK_HIP(hipGetLastError()); return; }
   QOP_D(P64, P64, 0) QOP_D(P64, P64, 1)
   QOP_D(P32, P32, 0) QOP_D(P32, P32, 1)
   QOP_D(P16, P16, 0) QOP_D(P16, P16, 1)
   if (mode == 0) {
-    if (pu == P32) { hipLaunchKernelGGL((dot_kernel<P32, P32, 0>), g, bl, 0, st, a); QOP_CHECK_HIP(hipGetLastError()); return; }
+    if (pu == P32) { launch_kernel((dot_kernel<P32, P32, 0>), g, bl, 0, st, a); QOP_CHECK_HIP(hipGetLastError()); return; }
   }
 #undef QOP_D
   fatal(__FILE__, __LINE__, "dot: unsupported precision combination");
@@ -1531,9 +1531,9 @@ static void raw_to_vec_t(const Lattice *lat, const T *raw, DevVec &v, int eo, hi
   long b, e;
   eo_range(lat, eo, b, e);
   dim3 g((e - b + 255) / 256), bl(256);
-  if (v.prec == P64) hipLaunchKernelGGL((raw_to_vec_kernel<T, P64>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
-  else if (v.prec == P32) hipLaunchKernelGGL((raw_to_vec_kernel<T, P32>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
-  else hipLaunchKernelGGL((raw_to_vec_kernel<T, P16>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
+  if (v.prec == P64) launch_kernel((raw_to_vec_kernel<T, P64>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
+  else if (v.prec == P32) launch_kernel((raw_to_vec_kernel<T, P32>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
+  else launch_kernel((raw_to_vec_kernel<T, P16>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
   QOP_CHECK_HIP(hipGetLastError());
 }
 template <typename T>
@@ -1541,9 +1541,9 @@ static void vec_to_raw_t(const Lattice *lat, const DevVec &v, T *raw, int eo, hi
   long b, e;
   eo_range(lat, eo, b, e);
   dim3 g((e - b + 255) / 256), bl(256);
-  if (v.prec == P64) hipLaunchKernelGGL((vec_to_raw_kernel<T, P64>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
-  else if (v.prec == P32) hipLaunchKernelGGL((vec_to_raw_kernel<T, P32>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
-  else hipLaunchKernelGGL((vec_to_raw_kernel<T, P16>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
+  if (v.prec == P64) launch_kernel((vec_to_raw_kernel<T, P64>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
+  else if (v.prec == P32) launch_kernel((vec_to_raw_kernel<T, P32>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
+  else launch_kernel((vec_to_raw_kernel<T, P16>), g, bl, 0, st, raw, v.data, v.norm, lat->Vh, b, e);
   QOP_CHECK_HIP(hipGetLastError());
 }
 
@@ -1564,7 +1564,7 @@ __global__ void __launch_bounds__(256) copy_kernel(const float4 *__restrict__ in
 
 void launch_copy(const void *in, void *out, size_t bytes, hipStream_t st) {
   long n = (long)(bytes / 16);
-  hipLaunchKernelGGL(copy_kernel, dim3(8192), dim3(256), 0, st, (const float4 *)in, (float4 *)out, n);
+  launch_kernel(copy_kernel, dim3(8192), dim3(256), 0, st, (const float4 *)in, (float4 *)out, n);
   QOP_CHECK_HIP(hipGetLastError());
 }
 

@@ -54,7 +54,7 @@ MultiShiftBatch::MultiShiftBatch(Links &L, int eo, int capacity, int sloppy_prec
     std::vector<double> hc(2 * cap_);
     for (int b = 0; b < cap_; b++) { hc[2 * b] = -1.0; hc[2 * b + 1] = m0 * m0; }
     QOP_CHECK_HIP(hipMemcpy(coef_, hc.data(), hc.size() * sizeof(double), hipMemcpyHostToDevice));
-    L_.get(hp_);  // convert the links before any graph capture
+    L_.get(hp_);  // convert the links before an iteration is recorded
     L_.get(P64);
     // each hop of the iteration with its own epilogue (the second with alpha 0
     // while no slot is loaded)
@@ -238,9 +238,9 @@ void MultiShiftBatch::run() {
   const int chunk = options().chunk > 0 ? options().chunk : 16;
   const bool use_graph = options().use_graph != 0;
   if (use_graph && !graph_) {
-    graph_.begin(st);
+    graph_.begin();
     for (int c = 0; c < chunk; c++) enqueue_iteration();
-    graph_.end(st);
+    graph_.end();
   }
   while (true) {
     bool any = false;

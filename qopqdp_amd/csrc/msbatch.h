@@ -96,7 +96,7 @@ class MultiShiftBatch {
   double *partA_ = nullptr, *partB_ = nullptr, *partC_ = nullptr;
   double *coef_ = nullptr, *sums_ = nullptr;
   int *zero_status_ = nullptr;
-  CapturedGraph graph_;
+  LaunchGraph graph_;
   HopShape shape_, shape2_;
 };
 

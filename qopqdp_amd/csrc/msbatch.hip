@@ -241,30 +241,30 @@ ms_update(const MsSlot *S, const int *active, int Vh, VecView rs, VecView ps, Ve
 
 void ms_launch_scalarA(MsSlot *s, const int *active, const double *partA, const double *partB,
                        int nch, int n, hipStream_t st) {
-  hipLaunchKernelGGL(ms_scalarA, dim3(n), dim3(MS_THREADS), 0, st, s, const_cast<int *>(active), partA, partB, nch);
+  launch_kernel(ms_scalarA, dim3(n), dim3(MS_THREADS), 0, st, s, const_cast<int *>(active), partA, partB, nch);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void ms_launch_scalarB(MsSlot *s, int *active, const double *partC, int nch, int n, int *ru,
                        hipStream_t st) {
-  hipLaunchKernelGGL(ms_scalarB, dim3(n), dim3(MS_THREADS), 0, st, s, active, partC, nch, ru);
+  launch_kernel(ms_scalarB, dim3(n), dim3(MS_THREADS), 0, st, s, active, partC, nch, ru);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void ms_launch_ru_fold(const int *ru, int Vh, VecView x64, VecView xs, long stride, int cap, int ns,
                        hipStream_t st) {
-  hipLaunchKernelGGL(ms_ru_fold, dim3((Vh + 255) / 256, cap * ns), dim3(256), 0, st, ru, Vh, x64, xs,
+  launch_kernel(ms_ru_fold, dim3((Vh + 255) / 256, cap * ns), dim3(256), 0, st, ru, Vh, x64, xs,
                      stride, cap);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void ms_launch_ru_scalar(MsSlot *s, int *ru, const double *part, int nch, int n, hipStream_t st) {
-  hipLaunchKernelGGL(ms_ru_scalar, dim3(n), dim3(MS_THREADS), 0, st, s, ru, part, nch);
+  launch_kernel(ms_ru_scalar, dim3(n), dim3(MS_THREADS), 0, st, s, ru, part, nch);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void ms_launch_update(const MsSlot *s, const int *active, int prec, int Vh, VecView rs, VecView ps,
                       VecView pm, VecView xm, long stride, long sstride, int cap, int ns, double *partB,
                       hipStream_t st) {
   dim3 g((Vh + 255) / 256, cap), bl(256);
-  if (prec == P16) hipLaunchKernelGGL(ms_update<P16>, g, bl, 0, st, s, active, Vh, rs, ps, pm, xm, stride, sstride, cap, partB);
-  else hipLaunchKernelGGL(ms_update<P32>, g, bl, 0, st, s, active, Vh, rs, ps, pm, xm, stride, sstride, cap, partB);
+  if (prec == P16) launch_kernel(ms_update<P16>, g, bl, 0, st, s, active, Vh, rs, ps, pm, xm, stride, sstride, cap, partB);
+  else launch_kernel(ms_update<P32>, g, bl, 0, st, s, active, Vh, rs, ps, pm, xm, stride, sstride, cap, partB);
   QOP_CHECK_HIP(hipGetLastError());
   (void)ns;
 }

@@ -4,7 +4,6 @@
 #include <mutex>
 
 #include "block_cache.h"
-#include "capture_gate.h"
 #include "common.h"
 #include "eigcg.h"
 
@@ -15,32 +14,6 @@ namespace qop {
   fflush(stderr);
   abort();
 }
-
-// ---------------------------------------------------------------------------
-// stream captures and device synchronisations (capture_gate.h)
-static CaptureGate &capture_gate() {
-  static CaptureGate *g = new CaptureGate;
-  return *g;
-}
-void capture_begin(hipStream_t st) {
-  capture_gate().capture_begin();
-  QOP_CHECK_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-}
-hipGraph_t capture_end(hipStream_t st) {
-  hipGraph_t g = nullptr;
-  const hipError_t e = hipStreamEndCapture(st, &g);
-  capture_gate().capture_end();
-  QOP_CHECK_HIP(e);
-  return g;
-}
-static bool device_sync_gated(bool wait) {
-  if (!capture_gate().sync_begin(wait)) return false;
-  const hipError_t e = hipDeviceSynchronize();
-  capture_gate().sync_end();
-  QOP_CHECK_HIP(e);
-  return true;
-}
-void device_sync() { (void)device_sync_gated(true); }
 
 // ---------------------------------------------------------------------------
 // device and page-locked memory (block_cache.h)
@@ -69,7 +42,16 @@ struct HipMemory {
     if (host) QOP_CHECK_HIP(hipHostFree(p));
     else QOP_CHECK_HIP(hipFree(p));
   }
-  bool try_sync() { return device_sync_gated(false); }
+  // false while a capture of the program's own forbids it
+  bool try_sync() {
+    const hipError_t e = hipDeviceSynchronize();
+    if (e == hipErrorStreamCaptureUnsupported || e == hipErrorStreamCaptureImplicit) {
+      (void)hipGetLastError();
+      return false;
+    }
+    QOP_CHECK_HIP(e);
+    return true;
+  }
   [[noreturn]] void out_of_memory(size_t bytes) { throw DeviceOutOfMemory{bytes}; }
 };
 using Cache = BlockCache<HipMemory>;

@@ -92,7 +92,7 @@ struct CgmsBuffers {
 //   t = D p (|t|^2);  b = r^2 / (|t|^2 + m^2 |p|^2);
 //   r -= b (m^2 p - D t) in the second hop's epilogue (|r|^2);
 //   a = r'^2 / r^2 and the shift recurrences;  x_i += b_i p_i, p_i = zn_i r + a_i p_i (|p|^2),
-// five launches, captured as a chunk; kernels past a raised status do nothing.
+// five launches, recorded as a chunk; kernels past a raised status do nothing.
 class CgmsRun {
  public:
   CgmsRun(Links &L, int prec, double mass, int eo, int ns, bool with_rel, int irel, DevVec *const *x,
@@ -111,7 +111,7 @@ class CgmsRun {
     if (with_rel) xrel_ = x[irel]->half(eo);
     QOP_CHECK_HIP(hipMemcpyAsync(B.d.xs, hx_.data(), 2 * ns * sizeof(VecView), hipMemcpyHostToDevice, st));
     // link arguments of both hops: any link conversion is done here, before
-    // the iterations are captured into a graph
+    // the iterations are recorded into a graph
     set_hop_links(a1_, L, prec, opp);
     set_hop_links(a2_, L, prec, eo);
     a1_.g = a2_.g = lat->g;
@@ -151,9 +151,9 @@ class CgmsRun {
     hipStream_t st = stream();
     const int chunk = options().chunk > 0 ? options().chunk : 16;
     if (options().use_graph && !graph_) {
-      graph_.begin(st);
+      graph_.begin();
       for (int c = 0; c < chunk; c++) iteration();
-      graph_.end(st);
+      graph_.end();
     }
     do {
       if (graph_) graph_.launch(st);
@@ -181,7 +181,7 @@ class CgmsRun {
   VecView p_, r_, xrel_{};
   std::vector<VecView> hx_;
   HopArgs a1_, a2_;
-  CapturedGraph graph_;
+  LaunchGraph graph_;
 };
 
 }  // namespace

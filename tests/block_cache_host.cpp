@@ -1,5 +1,4 @@
-// Host checks of the block cache and of the gate between stream captures and
-// device synchronisations, over a memory whose allocations, frees and
+// Host checks of the block cache over a memory whose allocations, frees and
 // synchronisations are counted.  Usage: block_cache_host <check>.
 #include <atomic>
 #include <chrono>
@@ -11,7 +10,6 @@
 #include <vector>
 
 #include "block_cache.h"
-#include "capture_gate.h"
 
 using namespace qop;
 
@@ -26,8 +24,8 @@ using namespace qop;
 static void nap(int us) { std::this_thread::sleep_for(std::chrono::microseconds(us)); }
 
 struct Device {
-  CaptureGate gate;
-  std::atomic<int> capturing{0}, syncs{0}, allocs{0}, frees{0};
+  std::atomic<int> syncs{0}, allocs{0}, frees{0};
+  std::atomic<bool> busy{false};  // no synchronisation possible now
   int sync_us = 0;
 };
 struct Memory {
@@ -42,29 +40,26 @@ struct Memory {
     ::free(p);
   }
   bool try_sync() {
-    if (!d->gate.sync_begin(false)) return false;
-    CHECK(d->capturing == 0);
+    if (d->busy) return false;
     nap(d->sync_us);
-    CHECK(d->capturing == 0);
     d->syncs++;
-    d->gate.sync_end();
     return true;
   }
   [[noreturn]] void out_of_memory(size_t) { throw std::bad_alloc(); }
 };
 using Cache = BlockCache<Memory>;
 
-// A freed block is handed out again only after a synchronisation, and while
-// a stream is captured there is none: the request gets a new block.
-static void no_sync_in_capture() {
+// A freed block is handed out again only after a synchronisation; where there
+// can be none the request gets a new block.
+static void freed_blocks_wait_for_a_sync() {
   Device d;
   Cache c(Memory{&d}, 1 << 20, 8 << 20);
   void *a = c.alloc(4096);
   c.free(a);
-  d.gate.capture_begin();
+  d.busy = true;
   void *b = c.alloc(4096);
   CHECK(b != a && d.syncs == 0 && d.allocs == 2);
-  d.gate.capture_end();
+  d.busy = false;
   void *e = c.alloc(4096);
   CHECK(e == a && d.syncs == 1 && d.allocs == 2);
   c.free(b);
@@ -73,53 +68,12 @@ static void no_sync_in_capture() {
   CHECK(d.frees == 2);
 }
 
-// Threads that capture beside threads that allocate and free: no capture ever
-// overlaps a synchronisation (checked inside try_sync), also of one that waits.
-static void captures_and_syncs_exclude_each_other() {
-  Device d;
-  d.sync_us = 50;
-  Cache c(Memory{&d}, 1 << 20, 8 << 20);
-  std::atomic<bool> stop{false};
-  std::vector<std::thread> ts;
-  for (int i = 0; i < 2; i++)
-    ts.emplace_back([&] {
-      while (!stop) {
-        d.gate.capture_begin();
-        d.capturing++;
-        nap(30);
-        d.capturing--;
-        d.gate.capture_end();
-        nap(30);
-      }
-    });
-  for (int i = 0; i < 3; i++)
-    ts.emplace_back([&, i] {
-      for (int k = 0; k < 300; k++) {
-        void *p = c.alloc(1000 * (i + 1));
-        memset(p, i, 1000 * (i + 1));
-        c.free(p);
-        if (k % 50 == 0) {
-          CHECK(d.gate.sync_begin(true));
-          CHECK(d.capturing == 0);
-          d.gate.sync_end();
-        }
-      }
-    });
-  for (size_t i = 2; i < ts.size(); i++) ts[i].join();
-  stop = true;
-  ts[0].join();
-  ts[1].join();
-  c.trim();
-  CHECK(d.allocs == d.frees);
-}
-
 int main(int argc, char **argv) {
   const struct {
     const char *name;
     void (*run)();
   } checks[] = {
-      {"no_sync_in_capture", no_sync_in_capture},
-      {"captures_and_syncs_exclude_each_other", captures_and_syncs_exclude_each_other},
+      {"freed_blocks_wait_for_a_sync", freed_blocks_wait_for_a_sync},
   };
   for (auto &k : checks)
     if (argc == 2 && !strcmp(argv[1], k.name)) {

@@ -1,6 +1,6 @@
-"""The block cache behind device allocations and the gate between stream
-captures and device synchronisations, on the CPU: tests/block_cache_host.cpp
-runs both over a memory that counts allocations, frees and synchronisations."""
+"""The block cache behind device allocations, on the CPU:
+tests/block_cache_host.cpp runs it over a memory that counts allocations,
+frees and synchronisations."""
 import os
 import subprocess
 
@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["no_sync_in_capture", "captures_and_syncs_exclude_each_other"])
+@pytest.mark.parametrize("check", ["freed_blocks_wait_for_a_sync"])
 def test_block_cache(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
