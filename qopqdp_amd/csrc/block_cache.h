@@ -7,7 +7,8 @@
 //  * A freed block may still be in use by work enqueued on any stream.  It is
 //    pending until a device synchronisation after its free (hipFree waits for
 //    the device too) and only then handed out, so a block never passes from
-//    one stream or thread to another with work in flight.  Where the device
+//    one stream or thread to another with work in flight.  The waiting thread
+//    holds no lock: the others allocate and free meanwhile.  Where the device
 //    cannot be synchronised now, pending blocks stay pending and a new block
 //    is allocated.
 //  * Bounded: blocks above `block` bytes go back to the driver at once
@@ -28,7 +29,6 @@
 #include <cstddef>
 #include <map>
 #include <mutex>
-#include <utility>
 
 namespace qop {
 
@@ -39,12 +39,18 @@ class BlockCache {
   void *alloc(size_t bytes) {
     const int dev = api_.device();
     const size_t want = bytes <= block_ ? round(bytes) : bytes;
-    std::lock_guard<std::mutex> lk(mu_);
+    std::unique_lock<std::mutex> lk(mu_);
     void *p = nullptr;
     if (want <= block_) {
       p = take(ready_, dev, want);
       if (!p && fits(pending_, dev, want)) {
-        if (api_.try_sync()) settle(dev);
+        // other threads allocate and free meanwhile; what they free from here
+        // on is not settled by this synchronisation
+        const unsigned long before = ++epoch_;
+        lk.unlock();
+        const bool idle = api_.try_sync();
+        lk.lock();
+        if (idle) settle(dev, before);
         p = take(ready_, dev, want);
       }
     }
@@ -73,7 +79,7 @@ class BlockCache {
       return;
     }
     kept_ += it->second.bytes;
-    pending_.emplace(it->second.bytes, std::make_pair(p, it->second.dev));
+    pending_.emplace(it->second.bytes, KeptBlock{p, it->second.dev, epoch_});
     live_.erase(it);
   }
   void trim() {
@@ -90,7 +96,12 @@ class BlockCache {
     size_t bytes;
     int dev;
   };
-  using Kept = std::multimap<size_t, std::pair<void *, int>>;
+  struct KeptBlock {
+    void *p;
+    int dev;
+    unsigned long freed;  // epoch of its free
+  };
+  using Kept = std::multimap<size_t, KeptBlock>;
   // whole 512-byte units, and 1/16 of the size for large blocks, so nearby
   // sizes share blocks
   static size_t round(size_t bytes) {
@@ -99,25 +110,25 @@ class BlockCache {
     return bytes ? (bytes + unit - 1) / unit * unit : unit;
   }
   // a kept block of at least `want` bytes and at most 1/8 more
-  static Kept::iterator find(Kept &k, int dev, size_t want) {
+  static typename Kept::iterator find(Kept &k, int dev, size_t want) {
     for (auto it = k.lower_bound(want); it != k.end() && it->first <= want + want / 8; ++it)
-      if (it->second.second == dev) return it;
+      if (it->second.dev == dev) return it;
     return k.end();
   }
   static bool fits(Kept &k, int dev, size_t want) { return find(k, dev, want) != k.end(); }
   void *take(Kept &k, int dev, size_t want) {
     auto it = find(k, dev, want);
     if (it == k.end()) return nullptr;
-    void *p = it->second.first;
+    void *p = it->second.p;
     live_[p] = Block{it->first, dev};
     kept_ -= it->first;
     k.erase(it);
     return p;
   }
-  // the pending blocks of a device that has been synchronised
-  void settle(int dev) {
+  // the blocks freed before a synchronisation of their device began
+  void settle(int dev, unsigned long before) {
     for (auto it = pending_.begin(); it != pending_.end();) {
-      if (it->second.second == dev) {
+      if (it->second.dev == dev && it->second.freed < before) {
         ready_.insert(*it);
         it = pending_.erase(it);
       } else {
@@ -127,7 +138,7 @@ class BlockCache {
   }
   void trim_locked() {
     for (Kept *k : {&ready_, &pending_}) {
-      for (auto &b : *k) api_.free(b.second.first);
+      for (auto &b : *k) api_.free(b.second.p);
       k->clear();
     }
     kept_ = 0;
@@ -138,6 +149,7 @@ class BlockCache {
   Kept ready_, pending_;
   std::map<void *, Block> live_;
   size_t kept_ = 0;
+  unsigned long epoch_ = 0;
   bool failed_ = false;  // the last allocation failed: its frees are not kept
 };
 

@@ -26,7 +26,7 @@ static void nap(int us) { std::this_thread::sleep_for(std::chrono::microseconds(
 struct Device {
   std::atomic<int> syncs{0}, allocs{0}, frees{0};
   std::atomic<bool> busy{false};  // no synchronisation possible now
-  int sync_us = 0;
+  std::atomic<bool> waiting{false}, release{true};  // a synchronisation lasts until released
 };
 struct Memory {
   Device *d;
@@ -41,7 +41,9 @@ struct Memory {
   }
   bool try_sync() {
     if (d->busy) return false;
-    nap(d->sync_us);
+    d->waiting = true;
+    while (!d->release) nap(20);
+    d->waiting = false;
     d->syncs++;
     return true;
   }
@@ -68,12 +70,68 @@ static void freed_blocks_wait_for_a_sync() {
   CHECK(d.frees == 2);
 }
 
+// While one thread waits for the device the others allocate and free, and a
+// block freed during the wait is not handed out by it.
+static void nobody_waits_behind_a_sync() {
+  Device d;
+  Cache c(Memory{&d}, 1 << 20, 8 << 20);
+  void *a = c.alloc(4096), *b = c.alloc(4096);
+  c.free(a);
+  d.release = false;
+  void *got = nullptr;
+  std::thread t([&] { got = c.alloc(4096); });
+  while (!d.waiting) nap(20);
+  std::atomic<bool> done{false};
+  std::thread u([&] {
+    void *x = c.alloc(100000);
+    c.free(x);
+    c.free(b);
+    done = true;
+  });
+  for (int i = 0; i < 10000 && !done; i++) nap(100);
+  const bool went_on = done;
+  d.release = true;
+  t.join();
+  u.join();
+  CHECK(went_on);
+  CHECK(got == a && d.syncs == 1);
+  void *e = c.alloc(4096);  // b, freed during the wait, needs a sync of its own
+  CHECK(e == b && d.syncs == 2);
+  c.free(got);
+  c.free(e);
+  c.trim();
+  CHECK(d.allocs == 3 && d.frees == 3);
+}
+
+// Threads that write their blocks and free them: no block has two owners, and
+// all go back.
+static void blocks_have_one_owner() {
+  Device d;
+  Cache c(Memory{&d}, 1 << 20, 8 << 20);
+  std::vector<std::thread> ts;
+  for (int i = 0; i < 4; i++)
+    ts.emplace_back([&, i] {
+      const size_t n = 1000 * (1 + i % 2);
+      for (int k = 0; k < 3000; k++) {
+        unsigned char *p = (unsigned char *)c.alloc(n);
+        memset(p, i + 1, n);
+        for (size_t j = 0; j < n; j++) CHECK(p[j] == i + 1);
+        c.free(p);
+      }
+    });
+  for (auto &t : ts) t.join();
+  c.trim();
+  CHECK(d.allocs == d.frees && c.kept() == 0);
+}
+
 int main(int argc, char **argv) {
   const struct {
     const char *name;
     void (*run)();
   } checks[] = {
       {"freed_blocks_wait_for_a_sync", freed_blocks_wait_for_a_sync},
+      {"nobody_waits_behind_a_sync", nobody_waits_behind_a_sync},
+      {"blocks_have_one_owner", blocks_have_one_owner},
   };
   for (auto &k : checks)
     if (argc == 2 && !strcmp(argv[1], k.name)) {
