@@ -8,7 +8,8 @@
 //    pending until a device synchronisation after its free (hipFree waits for
 //    the device too) and only then handed out, so a block never passes from
 //    one stream or thread to another with work in flight.  The waiting thread
-//    holds no lock: the others allocate and free meanwhile.  Where the device
+//    holds no lock, here and in the calls of Api: the others allocate and free
+//    meanwhile.  Where the device
 //    cannot be synchronised now, pending blocks stay pending and a new block
 //    is allocated.
 //  * Bounded: blocks above `block` bytes go back to the driver at once
@@ -34,6 +35,17 @@ namespace qop {
 
 template <class Api>
 class BlockCache {
+  struct Block {
+    size_t bytes;
+    int dev;
+  };
+  struct KeptBlock {
+    void *p;
+    int dev;
+    unsigned long freed;  // epoch of its free
+  };
+  using Kept = std::multimap<size_t, KeptBlock>;
+
  public:
   BlockCache(Api api, size_t block, size_t total) : api_(api), block_(block), total_(total) {}
   void *alloc(size_t bytes) {
@@ -55,11 +67,13 @@ class BlockCache {
       }
     }
     if (!p) {
+      lk.unlock();
       p = api_.alloc(want);
       if (!p) {
-        trim_locked();
+        trim();
         p = api_.alloc(want);
       }
+      lk.lock();
       if (!p) {
         failed_ = true;
         api_.out_of_memory(bytes);
@@ -71,10 +85,11 @@ class BlockCache {
   }
   void free(void *p) {
     if (!p) return;
-    std::lock_guard<std::mutex> lk(mu_);
+    std::unique_lock<std::mutex> lk(mu_);
     auto it = live_.find(p);
     if (it == live_.end() || failed_ || kept_ + it->second.bytes > total_) {
       if (it != live_.end()) live_.erase(it);
+      lk.unlock();
       api_.free(p);
       return;
     }
@@ -82,9 +97,19 @@ class BlockCache {
     pending_.emplace(it->second.bytes, KeptBlock{p, it->second.dev, epoch_});
     live_.erase(it);
   }
+  // When it returns, what was kept at the call has gone back, also where
+  // another thread's trim had taken it.
   void trim() {
-    std::lock_guard<std::mutex> lk(mu_);
-    trim_locked();
+    std::lock_guard<std::mutex> tk(trim_mu_);
+    Kept ready, pending;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      ready.swap(ready_);
+      pending.swap(pending_);
+      kept_ = 0;
+    }
+    for (Kept *k : {&ready, &pending})
+      for (auto &b : *k) api_.free(b.second.p);
   }
   size_t kept() {
     std::lock_guard<std::mutex> lk(mu_);
@@ -92,16 +117,6 @@ class BlockCache {
   }
 
  private:
-  struct Block {
-    size_t bytes;
-    int dev;
-  };
-  struct KeptBlock {
-    void *p;
-    int dev;
-    unsigned long freed;  // epoch of its free
-  };
-  using Kept = std::multimap<size_t, KeptBlock>;
   // whole 512-byte units, and 1/16 of the size for large blocks, so nearby
   // sizes share blocks
   static size_t round(size_t bytes) {
@@ -136,16 +151,9 @@ class BlockCache {
       }
     }
   }
-  void trim_locked() {
-    for (Kept *k : {&ready_, &pending_}) {
-      for (auto &b : *k) api_.free(b.second.p);
-      k->clear();
-    }
-    kept_ = 0;
-  }
   Api api_;
   const size_t block_, total_;
-  std::mutex mu_;
+  std::mutex mu_, trim_mu_;
   Kept ready_, pending_;
   std::map<void *, Block> live_;
   size_t kept_ = 0;

@@ -26,7 +26,12 @@ static void nap(int us) { std::this_thread::sleep_for(std::chrono::microseconds(
 struct Device {
   std::atomic<int> syncs{0}, allocs{0}, frees{0};
   std::atomic<bool> busy{false};  // no synchronisation possible now
-  std::atomic<bool> waiting{false}, release{true};  // a synchronisation lasts until released
+  std::atomic<bool> waiting{false}, release{true};  // synchronisations and frees last until released
+  void wait() {
+    waiting = true;
+    while (!release) std::this_thread::sleep_for(std::chrono::microseconds(20));
+    waiting = false;
+  }
 };
 struct Memory {
   Device *d;
@@ -37,13 +42,12 @@ struct Memory {
   }
   void free(void *p) {
     d->frees++;
+    d->wait();
     ::free(p);
   }
   bool try_sync() {
     if (d->busy) return false;
-    d->waiting = true;
-    while (!d->release) nap(20);
-    d->waiting = false;
+    d->wait();
     d->syncs++;
     return true;
   }
@@ -103,6 +107,37 @@ static void nobody_waits_behind_a_sync() {
   CHECK(d.allocs == 3 && d.frees == 3);
 }
 
+// The same while a thread gives blocks back: one above the bound, and all of
+// them in a trim.
+static void nobody_waits_behind_a_free() {
+  for (int trim = 0; trim < 2; trim++) {
+    Device d;
+    Cache c(Memory{&d}, 1 << 20, 8 << 20);
+    void *big = c.alloc(2 << 20);
+    c.free(c.alloc(4096));
+    d.release = false;
+    std::thread t([&] {
+      if (trim) c.trim();
+      else c.free(big);
+    });
+    while (!d.waiting) nap(20);
+    std::atomic<bool> done{false};
+    std::thread u([&] {
+      c.free(c.alloc(100000));
+      done = true;
+    });
+    for (int i = 0; i < 10000 && !done; i++) nap(100);
+    const bool went_on = done;
+    d.release = true;
+    t.join();
+    u.join();
+    CHECK(went_on);
+    if (trim) c.free(big);
+    c.trim();
+    CHECK(d.allocs == d.frees);
+  }
+}
+
 // Threads that write their blocks and free them: no block has two owners, and
 // all go back.
 static void blocks_have_one_owner() {
@@ -131,6 +166,7 @@ int main(int argc, char **argv) {
   } checks[] = {
       {"freed_blocks_wait_for_a_sync", freed_blocks_wait_for_a_sync},
       {"nobody_waits_behind_a_sync", nobody_waits_behind_a_sync},
+      {"nobody_waits_behind_a_free", nobody_waits_behind_a_free},
       {"blocks_have_one_owner", blocks_have_one_owner},
   };
   for (auto &k : checks)

@@ -19,7 +19,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["freed_blocks_wait_for_a_sync", "nobody_waits_behind_a_sync",
-                                   "blocks_have_one_owner"])
+                                   "nobody_waits_behind_a_free", "blocks_have_one_owner"])
 def test_block_cache(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
