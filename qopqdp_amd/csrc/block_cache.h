@@ -15,7 +15,7 @@
 //  * Bounded: blocks above `block` bytes go back to the driver at once
 //    (calls that use them run long enough that their allocation does not show:
 //    one 32^3x64 link-matrix field, 302 MB, is still kept), and the kept blocks
-//    of a device total at most `total` bytes.
+//    total at most `total` bytes.
 //  * Given back: at QOP_finalize, when a request server ends, and when
 //    an allocation fails (it is tried again then, and if it still fails the
 //    blocks freed while the failure unwinds are not kept).
@@ -50,7 +50,7 @@ class BlockCache {
   BlockCache(Api api, size_t block, size_t total) : api_(api), block_(block), total_(total) {}
   void *alloc(size_t bytes) {
     const int dev = api_.device();
-    const size_t want = bytes <= block_ ? round(bytes) : bytes;
+    const size_t want = size_of(bytes);
     std::unique_lock<std::mutex> lk(mu_);
     void *p = nullptr;
     if (want <= block_) {
@@ -111,22 +111,26 @@ class BlockCache {
     for (Kept *k : {&ready, &pending})
       for (auto &b : *k) api_.free(b.second.p);
   }
+  // What an allocation of `bytes` takes: up to `block` whole units of 512
+  // bytes or of a power of two that is at most 1/16 of the size, above 16 MB
+  // at least whole 2 MB pages.  So nearby sizes share blocks, and none is more
+  // than 1/16 (1/8 from 16 to 32 MB), or 512 bytes, larger than asked for.
+  size_t size_of(size_t bytes) const {
+    size_t unit = 512;
+    while (unit * 32 <= bytes) unit *= 2;
+    if (bytes > ((size_t)16 << 20) && unit < ((size_t)2 << 20)) unit = (size_t)2 << 20;
+    const size_t n = bytes ? (bytes + unit - 1) / unit * unit : unit;
+    return n <= block_ ? n : bytes;
+  }
   size_t kept() {
     std::lock_guard<std::mutex> lk(mu_);
     return kept_;
   }
 
  private:
-  // whole 512-byte units, and 1/16 of the size for large blocks, so nearby
-  // sizes share blocks
-  static size_t round(size_t bytes) {
-    size_t unit = 512;
-    while (unit * 16 < bytes) unit *= 2;
-    return bytes ? (bytes + unit - 1) / unit * unit : unit;
-  }
-  // a kept block of at least `want` bytes and at most 1/8 more
+  // a kept block of `want` bytes
   static typename Kept::iterator find(Kept &k, int dev, size_t want) {
-    for (auto it = k.lower_bound(want); it != k.end() && it->first <= want + want / 8; ++it)
+    for (auto it = k.lower_bound(want); it != k.end() && it->first == want; ++it)
       if (it->second.dev == dev) return it;
     return k.end();
   }

@@ -76,28 +76,32 @@ struct Engine {
   double last_used = 0;
 };
 
+// Device memory of a link set and of an engine, block by block as they are
+// allocated.
 size_t link_bytes(const Lattice *lat, int prec) {
   const size_t n = (size_t)2 * 16 * 9 * lat->Vh;
-  if (prec == P64) return n * 16;
-  if (prec == P32) return n * 8;
-  return n * 4 + (size_t)2 * 16 * lat->Vh * sizeof(float);
+  const size_t scale = prec == P16 ? dev_block_bytes((size_t)2 * 16 * lat->Vh * sizeof(float)) : 0;
+  return dev_block_bytes(n * prec_cbytes(prec)) + scale;
 }
 
 size_t engine_bytes(const Lattice *lat, int cap, int prec) {
-  const size_t vh = lat->Vh;
-  const size_t fp64 = 48 * vh;                                  // one parity, FP64
-  const size_t sl = prec == P16 ? 12 * vh + 4 * vh : 24 * vh;   // one parity, sloppy
-  const size_t nch = (vh + 63) / 64;
-  size_t per_slot = 5 * fp64 + 3 * sl + 24 * vh + 3 * nch * sizeof(double) + 256;
-  if (prec == P64) per_slot = 0;
-  return (size_t)cap * per_slot + 2 * fp64 /* stage */ + 2 * fp64 /* raw */ + (1u << 20);
+  const size_t vh = lat->Vh, nch = (vh + 63) / 64, n = cap;
+  auto vectors = [&](size_t count, int p) { return dev_block_bytes(count * 3 * vh * prec_cbytes(p)); };
+  size_t bytes = 2 * vectors(2, P64);  // stage, raw
+  if (prec != P64) {  // the vectors of BatchSolver, norms, reduction partials
+    bytes += 5 * vectors(n, P64) + 3 * vectors(n, prec) + vectors(n, P32);
+    if (prec == P16) bytes += 3 * dev_block_bytes(n * vh * sizeof(float));
+    bytes += dev_block_bytes(3 * n * nch * sizeof(double));
+  }
+  return bytes + (1u << 20);  // masks, scalars
 }
 
 }  // namespace
 
 class Server {
  public:
-  Server(int capacity, int prec, size_t budget) : cap_(capacity), prec_(prec), budget_(budget) {
+  Server(int capacity, int prec, size_t budget)
+      : cap_(capacity), prec_(prec), capped_(budget > 0), budget_(budget) {
     size_t fr = 0, tot = 0;
     QOP_CHECK_HIP(hipMemGetInfo(&fr, &tot));
     fr += dev_cache_bytes();  // given back when an allocation needs it
@@ -140,6 +144,7 @@ class Server {
       used_ -= cf->bytes;
       return -1;
     }
+    keep_within_budget();
     std::lock_guard<std::mutex> lk(mu_);
     cfgs_.push_back(std::move(cf));
     return (int)cfgs_.size() - 1;
@@ -302,6 +307,16 @@ class Server {
     e.st = nullptr;
   }
 
+  // Blocks that the allocator keeps count against a budget the caller set.
+  void keep_within_budget() {
+    size_t used;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      used = used_;
+    }
+    if (capped_ && used + dev_cache_bytes() > budget_) cache_trim();
+  }
+
   // Create an engine for (cfg, eo) if memory allows, evicting idle engines
   // (least recently used first).  Returns null if it cannot be made now.
   Engine *make_engine(int cfg, int eo, bool *never) {
@@ -348,6 +363,7 @@ class Server {
       std::lock_guard<std::mutex> lk(mu_);
       used_ += need;
     }
+    keep_within_budget();
     try {
       devvec_alloc(e->stage, c.lat, P64);
       dev_alloc(&e->raw, (size_t)c.lat->V * 6 * sizeof(double));
@@ -491,6 +507,7 @@ class Server {
   }
 
   const int cap_, prec_;
+  const bool capped_;  // the caller set the budget
   size_t budget_, reserve_ = 0, used_ = 0;
   std::vector<std::unique_ptr<Config>> cfgs_;
   std::vector<std::unique_ptr<Engine>> engines_;  // worker thread only

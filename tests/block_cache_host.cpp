@@ -25,6 +25,7 @@ static void nap(int us) { std::this_thread::sleep_for(std::chrono::microseconds(
 
 struct Device {
   std::atomic<int> syncs{0}, allocs{0}, frees{0};
+  std::atomic<size_t> room{(size_t)1 << 40};  // bytes left
   std::atomic<bool> busy{false};  // no synchronisation possible now
   std::atomic<bool> waiting{false}, release{true};  // synchronisations and frees last until released
   void wait() {
@@ -37,13 +38,19 @@ struct Memory {
   Device *d;
   int device() { return 0; }
   void *alloc(size_t n) {
+    if (n > d->room) return nullptr;
+    d->room -= n;
     d->allocs++;
-    return malloc(n < 64 ? 64 : n);
+    size_t *p = (size_t *)malloc(n + 16);
+    p[0] = n;
+    return p + 2;
   }
   void free(void *p) {
     d->frees++;
     d->wait();
-    ::free(p);
+    size_t *q = (size_t *)p - 2;
+    d->room += q[0];
+    ::free(q);
   }
   bool try_sync() {
     if (d->busy) return false;
@@ -138,6 +145,72 @@ static void nobody_waits_behind_a_free() {
   }
 }
 
+// A block is at most 1/16, 512 bytes or, above 16 MB, 2 MB larger than asked
+// for; a kept block serves only requests of its size.
+static void blocks_are_little_larger_than_asked() {
+  Device d;
+  Cache c(Memory{&d}, 384 << 20, (size_t)8 << 30);
+  for (size_t n = 0; n < ((size_t)300 << 20); n = n * 9 / 8 + 37)
+    for (size_t m : {n, n + 1, (n & (n - 1)) ? n : n + 3}) {
+      const size_t s = c.size_of(m);
+      const size_t least = m > ((size_t)16 << 20) ? (size_t)2 << 20 : 512;
+      CHECK(s >= m && s > 0 && s % 512 == 0 && s - m <= (m / 16 > least ? m / 16 : least));
+      CHECK(c.size_of(s) == s);
+    }
+  CHECK(c.size_of((size_t)257 << 20) <= (size_t)273 << 20);
+  CHECK(c.size_of((size_t)400 << 20) == (size_t)400 << 20);
+  void *a = c.alloc(64 << 10);
+  c.free(a);
+  CHECK(c.kept() == 64 << 10);
+  void *b = c.alloc(60 << 10);  // a size class below
+  CHECK(b != a);
+  c.free(b);
+  c.trim();
+}
+
+// Blocks above the bound are not kept, nor any past the total.
+static void kept_memory_is_bounded() {
+  Device d;
+  Cache c(Memory{&d}, 1 << 20, 4 << 20);
+  c.free(c.alloc((1 << 20) + 1));
+  CHECK(c.kept() == 0 && d.frees == 1);
+  std::vector<void *> v;
+  for (int i = 0; i < 8; i++) v.push_back(c.alloc(1 << 20));
+  for (void *p : v) c.free(p);
+  CHECK(c.kept() == 4 << 20 && d.frees == 5);
+  c.trim();
+  CHECK(c.kept() == 0 && d.frees == 9);
+}
+
+// An allocation that fails is tried again without the kept blocks; if it
+// fails again the caller hears of it and what it gives back is not kept.
+static void failed_allocations_give_kept_blocks_back() {
+  Device d;
+  d.room = 8 << 20;
+  Cache c(Memory{&d}, 2 << 20, 64 << 20);
+  std::vector<void *> v;
+  for (int i = 0; i < 6; i++) v.push_back(c.alloc(1 << 20));
+  for (void *p : v) c.free(p);
+  CHECK(c.kept() == 6 << 20 && d.frees == 0);
+  void *a = c.alloc(7 << 20);  // fits only without them
+  CHECK(c.kept() == 0 && d.frees == 6);
+  void *b = c.alloc(1 << 20);
+  bool failed = false;
+  try {
+    c.alloc(1 << 20);
+  } catch (const std::bad_alloc &) {
+    failed = true;
+  }
+  CHECK(failed);
+  c.free(b);
+  CHECK(c.kept() == 0 && d.frees == 7);
+  c.free(c.alloc(1 << 20));  // works again, and is kept again
+  CHECK(c.kept() == 1 << 20);
+  c.free(a);
+  c.trim();
+  CHECK(d.allocs == d.frees);
+}
+
 // Threads that write their blocks and free them: no block has two owners, and
 // all go back.
 static void blocks_have_one_owner() {
@@ -168,6 +241,9 @@ int main(int argc, char **argv) {
       {"nobody_waits_behind_a_sync", nobody_waits_behind_a_sync},
       {"nobody_waits_behind_a_free", nobody_waits_behind_a_free},
       {"blocks_have_one_owner", blocks_have_one_owner},
+      {"blocks_are_little_larger_than_asked", blocks_are_little_larger_than_asked},
+      {"kept_memory_is_bounded", kept_memory_is_bounded},
+      {"failed_allocations_give_kept_blocks_back", failed_allocations_give_kept_blocks_back},
   };
   for (auto &k : checks)
     if (argc == 2 && !strcmp(argv[1], k.name)) {

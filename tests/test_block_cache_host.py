@@ -19,7 +19,9 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["freed_blocks_wait_for_a_sync", "nobody_waits_behind_a_sync",
-                                   "nobody_waits_behind_a_free", "blocks_have_one_owner"])
+                                   "nobody_waits_behind_a_free", "blocks_have_one_owner",
+                                   "blocks_are_little_larger_than_asked", "kept_memory_is_bounded",
+                                   "failed_allocations_give_kept_blocks_back"])
 def test_block_cache(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr

@@ -130,3 +130,37 @@ def test_fp64_server_and_zero_source(world, oracle):
         check_resid(oracle, cfgs, r, out)
     finally:
         srv.close()
+
+
+def test_device_memory_stays_within_a_budget_the_caller_set():
+    """What the process takes from the device, kept blocks included, stays
+    below max_bytes.  The vectors of a batch are a little above a power of two
+    bytes, where a coarse rounding would show most; the slack is for code and
+    page tables."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        fr, tot = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(fr), C.byref(tot)) == 0
+        return fr.value
+
+    L = [16, 16, 16, 34]
+    U = q.gen_gauge(L, 3300, 0.3)
+    src = q.gen_source(L, 3301, EVEN)
+    probe = q.Server(capacity=41, prec=16)
+    probe.add_gauge(L, U, MILC)
+    probe.wait(probe.submit(0, src, 0.3, 1e-6, EVEN))
+    used = int(probe.stats()["bytes_used"])
+    probe.close()
+    before = free_bytes()
+    srv = q.Server(capacity=41, prec=16, max_bytes=used)
+    try:
+        srv.add_gauge(L, U, MILC)
+        assert before - free_bytes() <= used + (48 << 20)
+        out, st, res, lat = srv.wait(srv.submit(0, src, 0.3, 1e-6, EVEN))
+        assert st == 0
+        assert before - free_bytes() <= used + (48 << 20)
+        assert srv.stats()["bytes_used"] <= used
+    finally:
+        srv.close()
