@@ -12,10 +12,12 @@
 //    meanwhile.  Where the device
 //    cannot be synchronised now, pending blocks stay pending and a new block
 //    is allocated.
-//  * Bounded: blocks above `block` bytes go back to the driver at once
-//    (calls that use them run long enough that their allocation does not show:
-//    one 32^3x64 link-matrix field, 302 MB, is still kept), and the kept blocks
-//    total at most `total` bytes.
+//  * Bounded: blocks above `block` bytes go back to the driver at once (the
+//    largest kept are the 302 MB matrix fields of 32^3x64), and the kept blocks
+//    total at most `total` bytes.  A call on a larger lattice pays for its
+//    allocations: little while the card has memory the driver has already
+//    cleared, then about 1 s for 35 to 50 GB (asqtad force at 40^3x64, 15 GB
+//    of workspace: 81 ms and 430 to 510 ms).
 //  * Given back: at QOP_finalize, when a request server ends, and when
 //    an allocation fails (it is tried again then, and if it still fails the
 //    blocks freed while the failure unwinds are not kept).

@@ -211,26 +211,38 @@ struct MidPtr {
   double2 *p[8];
 };
 
-// Site-innermost fields of one call, allocated one by one (fields of the size
-// the block cache of dev_alloc keeps from call to call).
+// The `n` site-innermost fields of one call.  Fields that the block cache of
+// dev_alloc keeps are allocated one by one, so their blocks fit the next call;
+// larger ones, which it does not keep, are one allocation.  Best of 14 calls
+// one by one and as one: 40^3x64 asqtad force (26 fields) 84.5 / 80.9 ms, HISQ
+// force (34) 163 / 157, asqtad links (12) 27.1 / 24.9.
 class Fields {
  public:
-  explicit Fields(long V) : bytes_((size_t)9 * V * sizeof(double2)) {}
+  Fields(long V, int n) : bytes_((size_t)9 * V * sizeof(double2)), left_(n), whole_(!dev_block_kept(bytes_)) {
+    f_.reserve(n);
+  }
   Fields(const Fields &) = delete;
   Fields &operator=(const Fields &) = delete;
   ~Fields() {
     for (double2 *f : f_) dev_free(f);
   }
   double2 *take() {
-    f_.reserve(f_.size() + 1);
-    double2 *f = nullptr;
-    dev_alloc(&f, bytes_);
-    f_.push_back(f);
+    QOP_REQUIRE(left_ > 0, "workspace: more fields taken than counted");
+    if (!whole_ || f_.empty()) {
+      dev_alloc(&next_, whole_ ? left_ * bytes_ : bytes_);
+      f_.push_back(next_);
+    }
+    left_--;
+    double2 *f = next_;
+    next_ += bytes_ / sizeof(double2);
     return f;
   }
 
  private:
   size_t bytes_;
+  int left_;
+  bool whole_;
+  double2 *next_ = nullptr;
   std::vector<double2 *> f_;
 };
 
@@ -887,13 +899,14 @@ constexpr double SIDE_FORCE_FLOPS = 7 * 198 + 3 * 216 + 3 * 18;
 namespace {
 
 // One force evaluation: launch geometry, site-innermost workspace and the
-// device table of vector pointers and eps.
+// device table of vector pointers and eps.  nfields: fields besides the
+// derivative scratch (stpl3[4], mid5[4], stpl5, mid3).
 class ForceRun {
  public:
-  ForceRun(const Lattice *lat, const double *eps, const DevVec *const *xs, int n,
+  ForceRun(const Lattice *lat, int nfields, const double *eps, const DevVec *const *xs, int n,
            hipStream_t st)
       : g_(lat->g), V_(lat->V), n9_(9 * lat->V), st_(st), sq_(make_sched(lat)),
-        b_(TPB), gs_(grid(lat->V)), ge_(grid(9 * lat->V)), gx_(8 * sq_.per), buf_(lat->V) {
+        b_(TPB), gs_(grid(lat->V)), ge_(grid(9 * lat->V)), gx_(8 * sq_.per), buf_(lat->V, nfields + 10) {
     if (V_ >= (1L << 27))
       throw std::runtime_error("fermion force: lattice volume of 2^27 sites or more (32-bit offsets)");
     prec_ = n > 0 ? xs[0]->prec : P64;
@@ -1132,7 +1145,7 @@ void asqtad_force_dev(const Lattice *lat, double *const U_raw[4], double *F_raw[
                       double *flops, hipStream_t st) {
   const bool naik = coef[5] != 0;
   const int nmid = naik ? 8 : 4;
-  ForceRun r(lat, eps, xs, n, st);
+  ForceRun r(lat, 4 + nmid + 4, eps, xs, n, st);
   double2 *U[4], *mid[8] = {}, *D[4];
   for (auto &u : U) u = r.take();
   for (int i = 0; i < nmid; i++) mid[i] = r.take();
@@ -1156,7 +1169,7 @@ void hisq_force_dev(const Lattice *lat, double *const U_raw[4], double *const V_
                     double *flops, int *nfilt, hipStream_t st) {
   int nterms = 0;
   for (int k = 0; k < n_naiks; k++) nterms += n_orders[k];
-  ForceRun r(lat, eps, xs, nterms, st);
+  ForceRun r(lat, 4 + 4 + 8 + 4 + 4, eps, xs, nterms, st);
   double2 *U[4], *W[4], *mid[8], *F1[4], *F2[4];
   for (auto &u : U) u = r.take();
   for (auto &w : W) w = r.take();
@@ -1217,7 +1230,7 @@ static void fatten_run(const Lattice *lat, const double *const gf[4], const doub
   const bool naik = dst ? c[5] != 0 : lng_raw != nullptr;
   const int nl = naik ? 16 : 8, per = nl / 4;
   const bool sep_long = naik && (gl[0] != gf[0] || gl[1] != gf[1] || gl[2] != gf[2] || gl[3] != gf[3]);
-  Fields buf(V);
+  Fields buf(V, 1 + naik + 4 + (sep_long ? 4 : 0) + (coef7 != 0 ? 3 : 0) + (hasR ? 3 : 0));
   Ptr4 U{}, UL{}, T{}, R{};
   MidPtr Tw{}, Rw{};
   double2 *F = buf.take(), *Lk = naik ? buf.take() : nullptr;
