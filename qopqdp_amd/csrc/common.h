@@ -285,7 +285,8 @@ void fatten_dev(const Lattice *lat, const double *const gf[4], const double *con
                 const double coef[6], double *fat[4], double *lng[4], hipStream_t st);
 
 // The same smearing written straight into the double-stored FP64 links of L
-// (Naik links when c[5] != 0).
+// (Naik links when c[5] != 0), or where the memory for that is short by way of
+// the raw links, with the same bits.
 void fatten_links64(const Lattice *lat, Links &L, const double *const gf[4],
                     const double *const gl[4], const double coef[6], hipStream_t st);
 

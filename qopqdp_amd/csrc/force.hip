@@ -1309,7 +1309,28 @@ void fatten_dev(const Lattice *lat, const double *const gf[4], const double *con
 
 void fatten_links64(const Lattice *lat, Links &L, const double *const gf[4], const double *const gl[4],
                     const double c[6], hipStream_t st) {
-  fatten_run(lat, gf, gl, c, nullptr, nullptr, &L, st);
+  try {
+    fatten_run(lat, gf, gl, c, nullptr, nullptr, &L, st);
+    return;
+  } catch (const DeviceOutOfMemory &) {
+  }
+  // The workspace (12 fields of 144 B per site) and the double-stored links
+  // (16) do not fit together: by way of the raw links (8), 24 fields at most.
+  const bool naik = c[5] != 0;
+  const size_t bytes = (size_t)lat->V * 18 * sizeof(double);
+  DevBuf<double> fat[4], lng[4];
+  double *f[4], *l[4];
+  for (int mu = 0; mu < 4; mu++) {
+    dev_alloc(&fat[mu].p, bytes);
+    if (naik) dev_alloc(&lng[mu].p, bytes);
+    f[mu] = fat[mu].p;
+    l[mu] = lng[mu].p;
+  }
+  fatten_run(lat, gf, gl, c, f, naik ? l : nullptr, nullptr, st);
+  L.lat = const_cast<Lattice *>(lat);
+  const double *fc[4] = {f[0], f[1], f[2], f[3]}, *lc[4] = {l[0], l[1], l[2], l[3]};
+  build_links64(L, fc, naik ? lc : nullptr, st);
+  QOP_CHECK_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace qop
