@@ -62,11 +62,11 @@ struct CgmsBuffers {
       d.partD = d.partC + nch;
       dev_alloc(&d.xs, 2 * (size_t)ns * sizeof(VecView));
       d.pms = d.xs + ns;
+      host_alloc(&host, sizeof(CgmsState));
     } catch (const DeviceOutOfMemory &) {
       release();
       throw;
     }
-    host_alloc(&host, sizeof(CgmsState));
   }
   ~CgmsBuffers() { release(); }
   void release() {

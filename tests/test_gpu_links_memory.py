@@ -1,7 +1,8 @@
-"""Link construction where device memory is short: a 32^3x64 configuration
+"""Link construction where device memory is short.  A 32^3x64 configuration
 whose links and workspace (28 fields of 302 MB beside the gauge field) do not
 fit in what is left, while the links and the raw links (24) do, gets the same
-links as with memory to spare."""
+links as with memory to spare.  Where no way fits, the request server refuses
+the configuration and all it had taken is free again."""
 import ctypes as C
 
 import numpy as np
@@ -28,6 +29,11 @@ class Ballast:
                     break
                 self.held.append(p)
         assert left <= fr.value < left + (128 << 20)
+
+    def free(self):
+        fr, tot = C.c_size_t(), C.c_size_t()
+        assert self.hip.hipMemGetInfo(C.byref(fr), C.byref(tot)) == 0
+        return fr.value
 
     def drop(self):
         for p in self.held:
@@ -64,3 +70,18 @@ def test_links_where_the_direct_way_does_not_fit():
         s.lib.QOP_D3_destroy_G(g)
         s.close()
     assert np.array_equal(got, want)
+
+
+def test_a_refused_configuration_leaves_nothing_behind():
+    U = q.gen_gauge(L, 9002, 0.3)
+    srv = q.Server(capacity=1, prec=32, max_bytes=1 << 40)
+    ballast = Ballast(20 * FIELD)
+    try:
+        before = ballast.free()
+        with pytest.raises(RuntimeError):
+            srv.add_gauge(L, U)
+        assert ballast.free() >= before - (64 << 20)
+        assert srv.stats()["bytes_used"] == 0
+    finally:
+        ballast.drop()
+        srv.close()
