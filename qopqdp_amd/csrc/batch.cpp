@@ -210,8 +210,6 @@ BatchSolver::BatchSolver(Links &L, int eo, int capacity, int sloppy_prec, double
     dev_alloc(&ru_, 2 * cap_ * sizeof(int));
     ru_cont_ = ru_ + cap_;
     QOP_CHECK_HIP(hipMemsetAsync(ru_, 0, 2 * cap_ * sizeof(int), st_));
-    dev_alloc(&glob_, sizeof(BsGlobal));
-    host_alloc(&glob_h_, sizeof(BsGlobal));
     dev_alloc(&partA_, 3 * (size_t)cap_ * nch_ * sizeof(double));
     partB_ = partA_ + (size_t)cap_ * nch_;
     partC_ = partB_ + (size_t)cap_ * nch_;
@@ -222,11 +220,8 @@ BatchSolver::BatchSolver(Links &L, int eo, int capacity, int sloppy_prec, double
     host_alloc(&hc_h_, 2 * (size_t)cap_ * sizeof(double));
     memset(rhs_h_, 0, cap_ * sizeof(BsRhs));
     memset(active_h_, 0, 2 * cap_ * sizeof(int));
-    glob_h_->status = 0;
-    glob_h_->pending = 0;  // the status word stays 0: slots never pause the batch
     QOP_CHECK_HIP(hipMemcpyAsync(rhs_, rhs_h_, cap_ * sizeof(BsRhs), hipMemcpyHostToDevice, st_));
     QOP_CHECK_HIP(hipMemcpyAsync(active_, active_h_, 2 * cap_ * sizeof(int), hipMemcpyHostToDevice, st_));
-    QOP_CHECK_HIP(hipMemcpyAsync(glob_, glob_h_, sizeof(BsGlobal), hipMemcpyHostToDevice, st_));
     loaded_.assign(cap_, 0);
     mass_.assign(cap_, 0.0);
     // Build the sloppy and FP64 link sets now: the iteration is recorded into
@@ -261,8 +256,6 @@ void BatchSolver::release() {
   dev_free(active_);
   dev_free(ru_);
   host_free(active_h_);
-  dev_free(glob_);
-  host_free(glob_h_);
   dev_free(partA_);
   dev_free(coef_);
   dev_free(sums_);
@@ -483,7 +476,6 @@ void BatchSolver::enqueue_iteration() {
   a.nstride = Vh;
   a.n = cap_;
   a.active = active_;
-  a.status = &glob_->status;
   a.partial = partA_;
   shape_.apply(a);
   launch_hop_args(a, sp_, ls.nl, shape_.nb, shape_.block, RED_OUT2, false, st);
@@ -500,16 +492,16 @@ void BatchSolver::enqueue_iteration() {
   b.cg_alpha = (const double *)((const char *)rhs_ + offsetof(BsRhs, alpha));
   b.cg_stride = (int)(sizeof(BsRhs) / sizeof(double));
   b.partial = partC_;
-  bs_launch_scalar1(rhs_, active_, &glob_->status, partA_, partB_, nch_, cap_, ru_cont_, st);
+  bs_launch_scalar1(rhs_, active_, partA_, partB_, nch_, cap_, ru_cont_, st);
   shape2_.apply(b);
   launch_hop_args(b, sp_, ls.nl, shape2_.nb, shape2_.block, RED_CG, true, st);
-  bs_launch_scalar2(rhs_, active_, glob_, partC_, nch_, cap_, ru_, st);
+  bs_launch_scalar2(rhs_, active_, partC_, nch_, cap_, ru_, st);
   if (join_ > 0) bs_launch_ru_join(rhs_, active_, ru_, cap_, st);
   // reliable update of the flagged slots, all on the device, then the search
   // directions of all slots
   apply_A64(ru_, true);
   bs_launch_ru_scalar(rhs_, active_, ru_, ru_cont_, lcoef_, partA_, partB_, partC_, nch_, cap_, st);
-  bs_launch_pnext(rhs_, active_, &glob_->status, ru_cont_, lcoef_, sp_, (int)Vh, rs_.slot(0), ps_.slot(0), 3 * Vh,
+  bs_launch_pnext(rhs_, active_, ru_cont_, lcoef_, sp_, (int)Vh, rs_.slot(0), ps_.slot(0), 3 * Vh,
                   cap_, partB_, st);
 }
 

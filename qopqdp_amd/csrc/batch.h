@@ -20,12 +20,10 @@
 namespace qop {
 
 struct BsRhs {
-  int need_update;  // reliable update requested by the scalar kernel
   int iter;         // sloppy iterations done
   int max_iter;
   int reason;       // 0 running, 1 converged, 2 iteration limit, 3 breakdown
   int nupdate;      // reliable updates done
-  int pad;
   double m2;        // mass^2 of the slot's operator
   double r2;        // iterated residual norm^2
   double r2_old;    // iterated residual norm^2 of the previous iteration
@@ -37,17 +35,11 @@ struct BsRhs {
   double join2;     // joins another slot's update below join2 * r2_rel (0: never)
 };
 
-struct BsGlobal {
-  int status;   // 0 running, 1 host attention needed (read by every kernel)
-  int pending;  // set by slots during an iteration, committed at its end
-};
-
 // Kernels (batch.hip)
-void bs_launch_scalar1(BsRhs *rhs, const int *active, const int *status,
-                       const double *partA, const double *partB, int nch, int n,
+void bs_launch_scalar1(BsRhs *rhs, const int *active, const double *partA, const double *partB, int nch, int n,
                        int *ru_cont, hipStream_t st);
-void bs_launch_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob,
-                       const double *partC, int nch, int n, int *ru, hipStream_t st);
+void bs_launch_scalar2(BsRhs *rhs, const int *active, const double *partC, int nch, int n, int *ru,
+                       hipStream_t st);
 // x += xs, xs = 0 of the flagged slots, where it is a pass of its own.
 void bs_launch_ru_x(const int *ru, int n, int Vh, VecView x64, VecView xs, long stride, hipStream_t st);
 // Decisions of the reliable updates of the flagged slots, from the partials
@@ -59,9 +51,8 @@ void bs_launch_ru_scalar(BsRhs *rhs, int *active, int *ru, int *ru_cont, double 
 // update of this iteration when another slot is flagged for one.
 void bs_launch_ru_join(BsRhs *rhs, const int *active, int *ru, int n, hipStream_t st);
 // Search directions of the running slots, after any reliable updates.
-void bs_launch_pnext(const BsRhs *rhs, const int *active, const int *status, const int *ru_cont,
-                     const double *lcoef, int prec, int Vh, VecView rs, VecView ps, long stride,
-                     int n, double *partB, hipStream_t st);
+void bs_launch_pnext(const BsRhs *rhs, const int *active, const int *ru_cont, const double *lcoef,
+                     int prec, int Vh, VecView rs, VecView ps, long stride, int n, double *partB, hipStream_t st);
 void bs_launch_sum(const double *part, int nch, int n, const int *sel,
                    double *out, hipStream_t st);
 
@@ -160,7 +151,6 @@ class BatchSolver {
   int *active_ = nullptr, *active_h_ = nullptr;
   int *sel_ = nullptr, *sel_h_ = nullptr;
   int *ru_ = nullptr, *ru_cont_ = nullptr;  // device reliable-update masks
-  BsGlobal *glob_ = nullptr, *glob_h_ = nullptr;
   double *partA_ = nullptr, *partB_ = nullptr, *partC_ = nullptr;
   double *coef_ = nullptr;      // [cap][2] hop coefficients (-1, m2)
   double *lcoef_ = nullptr;     // [cap][3][2] lincomb coefficients

@@ -117,10 +117,8 @@ __device__ __forceinline__ void st3_q(void *data, float *norm, long h, long Vh,
 
 // pAp = |D p|^2 + m^2 |p|^2 ; alpha = r2 / pAp
 __global__ void __launch_bounds__(1024)
-bs_scalar1(BsRhs *rhs, const int *active, const int *status, const double *partA,
-           const double *partB, int nch, int *ru_cont) {
+bs_scalar1(BsRhs *rhs, const int *active, const double *partA, const double *partB, int nch, int *ru_cont) {
   __shared__ double sh[17];
-  if (*status != 0) return;
   const int b = blockIdx.x;
   BsRhs &R = rhs[b];
   if (threadIdx.x == 0) ru_cont[b] = 0;  // previous iteration's p fix is done
@@ -135,9 +133,8 @@ bs_scalar1(BsRhs *rhs, const int *active, const int *status, const double *partA
 
 // new r2, reliable-update and stopping decisions, beta
 __global__ void __launch_bounds__(1024)
-bs_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, int nch, int *ru) {
+bs_scalar2(BsRhs *rhs, const int *active, const double *partC, int nch, int *ru) {
   __shared__ double sh[17];
-  if (glob->status != 0) return;
   const int b = blockIdx.x;
   BsRhs &R = rhs[b];
   if (!active[b]) return;
@@ -149,12 +146,8 @@ bs_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, i
   if (!(R.pAp > 0)) { flag = true; }
   else if (r2new <= R.delta2 * R.r2_rel || r2new <= R.stop2 || R.iter >= R.max_iter) flag = true;
   R.r2 = r2new;
-  if (flag) {
-    R.need_update = 1;
-    ru[b] = 1;  // reliable update later in this iteration
-  } else {
-    R.beta = r2new / R.r2_old;
-  }
+  if (flag) ru[b] = 1;  // reliable update later in this iteration
+  else R.beta = r2new / R.r2_old;
 }
 
 // ---------------------------------------------------------------------------
@@ -206,7 +199,6 @@ bs_ru_scalar(BsRhs *rhs, int *active, int *ru, int *ru_cont, double *lcoef,
   if (threadIdx.x != 0) return;
   BsRhs &R = rhs[b];
   R.nupdate++;
-  R.need_update = 0;
   ru[b] = 0;
   const double r2_old = R.r2_old;
   R.r2 = r2t;
@@ -228,10 +220,9 @@ bs_ru_scalar(BsRhs *rhs, int *active, int *ru, int *ru_cont, double *lcoef,
 // partial |ps|^2 of the stored ps (the next iteration's p.Ap needs it).
 template <int P>
 __global__ void __launch_bounds__(256)
-bs_pnext(const BsRhs *rhs, const int *active, const int *status, const int *ru_cont, const double *lcoef, int Vh,
-         VecView rs, VecView ps, long stride, double *partB) {
+bs_pnext(const BsRhs *rhs, const int *active, const int *ru_cont, const double *lcoef, int Vh, VecView rs,
+         VecView ps, long stride, double *partB) {
   using R = typename BT<P>::R;
-  if (*status != 0) return;
   const int b = blockIdx.y;
   if (!active[b]) return;
   const bool fix = ru_cont[b] != 0;
@@ -281,7 +272,6 @@ __global__ void bs_ru_join(BsRhs *rhs, const int *active, int *ru, int n) {
   for (int b = 0; b < n; b++) {
     BsRhs &R = rhs[b];
     if (!active[b] || ru[b] || !(R.join2 > 0) || !(R.r2 <= R.join2 * R.r2_rel)) continue;
-    R.need_update = 1;
     ru[b] = 1;
   }
 }
@@ -296,26 +286,24 @@ bs_sum(const double *part, int nch, const int *sel, double *out) {
   if (threadIdx.x == 0) out[b] = s;
 }
 
-void bs_launch_scalar1(BsRhs *rhs, const int *active, const int *status, const double *partA,
-                       const double *partB, int nch, int n, int *ru_cont, hipStream_t st) {
-  launch_kernel(bs_scalar1, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, status, partA, partB, nch, ru_cont);
+void bs_launch_scalar1(BsRhs *rhs, const int *active, const double *partA, const double *partB, int nch, int n, int *ru_cont, hipStream_t st) {
+  launch_kernel(bs_scalar1, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, partA, partB, nch, ru_cont);
   QOP_CHECK_HIP(hipGetLastError());
 }
-void bs_launch_scalar2(BsRhs *rhs, const int *active, BsGlobal *glob, const double *partC, int nch,
-                       int n, int *ru, hipStream_t st) {
-  launch_kernel(bs_scalar2, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, glob, partC, nch, ru);
+void bs_launch_scalar2(BsRhs *rhs, const int *active, const double *partC, int nch, int n, int *ru,
+                       hipStream_t st) {
+  launch_kernel(bs_scalar2, dim3(n), dim3(BS_THREADS), 0, st, rhs, active, partC, nch, ru);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_ru_join(BsRhs *rhs, const int *active, int *ru, int n, hipStream_t st) {
   launch_kernel(bs_ru_join, dim3(1), dim3(64), 0, st, rhs, active, ru, n);
   QOP_CHECK_HIP(hipGetLastError());
 }
-void bs_launch_pnext(const BsRhs *rhs, const int *active, const int *status, const int *ru_cont,
-                     const double *lcoef, int prec, int Vh, VecView rs, VecView ps, long stride, int n,
+void bs_launch_pnext(const BsRhs *rhs, const int *active, const int *ru_cont, const double *lcoef, int prec, int Vh, VecView rs, VecView ps, long stride, int n,
                      double *partB, hipStream_t st) {
   dim3 g((Vh + 255) / 256, n), bl(256);
-  if (prec == P32) launch_kernel(bs_pnext<P32>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
-  else launch_kernel(bs_pnext<P16>, g, bl, 0, st, rhs, active, status, ru_cont, lcoef, Vh, rs, ps, stride, partB);
+  if (prec == P32) launch_kernel(bs_pnext<P32>, g, bl, 0, st, rhs, active, ru_cont, lcoef, Vh, rs, ps, stride, partB);
+  else launch_kernel(bs_pnext<P16>, g, bl, 0, st, rhs, active, ru_cont, lcoef, Vh, rs, ps, stride, partB);
   QOP_CHECK_HIP(hipGetLastError());
 }
 void bs_launch_sum(const double *part, int nch, int n, const int *sel, double *out, hipStream_t st) {

@@ -45,8 +45,6 @@ MultiShiftBatch::MultiShiftBatch(Links &L, int eo, int capacity, int sloppy_prec
     partC_ = partB_ + (size_t)cap_ * nch_;
     dev_alloc(&coef_, 2 * (size_t)cap_ * sizeof(double));
     dev_alloc(&sums_, 2 * (size_t)cap_ * sizeof(double));
-    dev_alloc(&zero_status_, sizeof(int));
-    QOP_CHECK_HIP(hipMemset(zero_status_, 0, sizeof(int)));
     memset(slot_h_, 0, cap_ * sizeof(MsSlot));
     memset(active_h_, 0, cap_ * sizeof(int));
     QOP_CHECK_HIP(hipMemset(active_, 0, 2 * cap_ * sizeof(int)));
@@ -82,7 +80,6 @@ void MultiShiftBatch::release() {
   dev_free(partA_);
   dev_free(coef_);
   dev_free(sums_);
-  dev_free(zero_status_);
 }
 
 void MultiShiftBatch::load(int slot, const DevVec &src, double ms_tol, int max_iter) {

@@ -95,7 +95,6 @@ class MultiShiftBatch {
   int *sel_ = nullptr;
   double *partA_ = nullptr, *partB_ = nullptr, *partC_ = nullptr;
   double *coef_ = nullptr, *sums_ = nullptr;
-  int *zero_status_ = nullptr;
   LaunchGraph graph_;
   HopShape shape_, shape2_;
 };
