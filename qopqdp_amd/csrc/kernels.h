@@ -12,7 +12,7 @@ namespace qop {
 // FP64 hops over flagged slots (launch_hop_flagged):
 // RED_SADD: src is src + src_add (FP32 increments), formed as it is read.
 // RED_RU32 / RED_RU16: the end of a reliable update in the epilogue, with the
-// sloppy vectors in FP32 / FP16 (RuArgs): x += xs, xs = 0; out = A x is not
+// sloppy vectors in FP32 / FP16 (HopFlagArgs): x += xs, xs = 0; out = A x is not
 // stored; r = b - A x goes into the sloppy rs; |r|^2 and <rs, ps>.
 enum { RED_NONE = 0, RED_OUT2 = 1, RED_X2 = 2, RED_CG = 3, RED_R = 4, RED_SADD = 5, RED_RU32 = 6, RED_RU16 = 7 };
 int hop_partial_blocks(const Lattice *lat);
@@ -32,10 +32,6 @@ struct HopArgs {
   double alpha = 1.0, beta = 0.0;
   double *partial = nullptr;     // [n][nchunk]
   const int *active = nullptr;   // device [n] or null
-  const int *slots = nullptr;    // device [1 + n] or null: count k, then the slots that launch RHS
-                                 // 0..k-1 work on.  No caller passes one, but the test for it stays:
-                                 // without it the compiler schedules the one-RHS FP64 hop 1.6 times
-                                 // slower (28 against 45 us at 16^3x32)
   const int *status = nullptr;   // device flag: kernel is a no-op when nonzero
   int remap = 1;
   int nt = 0;                    // non-temporal link loads

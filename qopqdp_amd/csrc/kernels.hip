@@ -545,15 +545,12 @@ __device__ __forceinline__ void hop_group(const A &a, int b0_in, int sb_in) {
   bool any = false;
 #pragma unroll
   for (int b = 0; b < NB; b++) {
-    // the launch's RHS j = b0 + b is slot j, or the j-th flagged or listed one
+    // the launch's RHS j = b0 + b is slot j, or the j-th flagged one
     const int j = b0 + b;
     if constexpr (GL) {
       sl[b] = nth_flag(a.flags, a.n, j);
       act[b] = sl[b] >= 0;
       if (!act[b]) sl[b] = j;
-    } else if (P == P64 && a.slots) {
-      act[b] = j < a.slots[0];
-      sl[b] = act[b] ? a.slots[1 + j] : j;
     } else {
       act[b] = (j < a.n) && (!a.active || a.active[j]);
       sl[b] = j;
@@ -739,6 +736,14 @@ __device__ __forceinline__ void hop_group(const A &a, int b0_in, int sb_in) {
           }
           if constexpr (P != P16) link_words_cvt<LP>(lw, w);
         }
+        // FP64: all words of a link and its neighbour are in flight before the
+        // first product, and the next link's loads stay behind the products
+        // (80 VGPRs, 6 waves per SIMD).  Left to itself the compiler keeps two
+        // to four loads in flight between the products: one RHS at 16^3x32
+        // 45 against 28 us.  Without the second barrier two links are in
+        // flight with 128 VGPRs: within 1% either way (24^3x48 171 / 173 us,
+        // 20^3x40 solve 21.1 / 20.9 ms).
+        if constexpr (P == P64 && !GL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int b = 0; b < NB; b++) {
           if (!act[b]) continue;
@@ -792,6 +797,7 @@ __device__ __forceinline__ void hop_group(const A &a, int b0_in, int sb_in) {
             }
           }
         }
+        if constexpr (P == P64 && !GL) __builtin_amdgcn_sched_barrier(0);
       }
     }
     hop_epilogue<P, NB, RED, HASX, NT>(a, h, Vh, sl, act, acc, red, ru);
@@ -1008,7 +1014,7 @@ void launch_hop_args(HopArgs a, int prec, int nl, int nb, int block, int red,
   QOP_REQUIRE(red != RED_CG || (a.cg_alpha && a.xs.data && prec != P64), "hop: RED_CG needs alpha and xs");
   QOP_REQUIRE(red != RED_R || a.cg_alpha, "hop: RED_R needs alpha");
   QOP_REQUIRE(a.n >= 1, "hop: n >= 1");
-  QOP_REQUIRE(!a.slots && red < RED_SADD, "hop: slot subsets go through launch_hop_flagged");
+  QOP_REQUIRE(red < RED_SADD, "hop: slot subsets go through launch_hop_flagged");
   check_hop_order(a, prec, nl, nb, block);
   // otherwise (or when a.plain asks for it) one RHS per thread with plain loads
   a.buf = hop_buf_fits(a, prec, nb);
@@ -1249,7 +1255,7 @@ static void launch_hop_pair(const HopArgs &a0, const HopArgs &b0, int prec, int 
 
 void launch_hop_one(const HopArgs &a, const HopArgs *b, int prec, int nl, int red, bool hasx, hipStream_t st) {
   QOP_REQUIRE(prec == P64 || prec == P32, "hop: the reference path has FP64 or FP32 vectors");
-  QOP_REQUIRE(a.n == 1 && !a.coef && !a.active && !a.slots && red < RED_SADD && red != RED_CG, "hop: one unmasked RHS");
+  QOP_REQUIRE(a.n == 1 && !a.coef && !a.active && red < RED_SADD && red != RED_CG, "hop: one unmasked RHS");
   // Solves, one thread per site / four waves (ms): FP64 8^3x16 4.2 / 3.2,
   // 12^3x24 6.0 / 5.4, 16^3x24 8.3 / 8.4, 16^3x32 13.0 / 13.3; FP32 8^3x16
   // 2.5 / 1.9, 16^3x32 4.5 / 4.2, 16^2x20x32 5.1 / 5.1, 20^3x32 5.9 / 6.3
