@@ -1,7 +1,9 @@
 """The block cache behind device allocations: results do not depend on what a
 reused block held, a link object reloaded on another lattice gets an array of
-that lattice, several threads may allocate and free, and QOP_finalize gives
-the kept memory back."""
+that lattice, several threads may allocate and free (their calls here wait for
+their own work; blocks freed with work in flight are the host checks' and
+test_gpu_beside_server's), freed blocks are kept, and QOP_finalize gives them
+back."""
 import ctypes as C
 import threading
 
@@ -89,3 +91,22 @@ def test_threads_and_finalize():
     assert not errors
     s.close()
     assert free_bytes() >= before - (16 << 20)  # reduction scratch may stay
+
+
+def test_freed_blocks_are_kept_until_finalize():
+    L = [16, 16, 16, 32]  # a vector is 6.3 MB
+    s = q.Session(L)
+    s.free(s.zeros())
+    before = free_bytes()
+    vs = [s.zeros() for _ in range(60)]
+    held = free_bytes()
+    assert held <= before - (350 << 20)
+    for v in vs:
+        s.free(v)
+    assert free_bytes() <= held + (16 << 20)
+    vs = [s.zeros() for _ in range(60)]  # from the kept blocks
+    assert free_bytes() >= held - (16 << 20)
+    for v in vs:
+        s.free(v)
+    s.close()
+    assert free_bytes() >= before - (16 << 20)
