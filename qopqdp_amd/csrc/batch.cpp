@@ -318,9 +318,11 @@ void BatchSolver::apply_A64(const int *mask, bool update) {
   a.flags = mask;
   // x + xs: formed in the first hop's gathers, which read the FP32 increments
   // 16 times per site instead of once, or in a pass of its own, a launch more.
-  // Masked first hop and pass per iteration: 16^3x32, 24 slots 34 against
-  // 39 us; 24^3x48, 16 slots 67 against 60 us
-  const bool sadd = update && lat_->Vh <= 131072;
+  // FP16 batches of 16 / 4 slots, in the gathers against in a pass (ms):
+  // 16^3x32 25.6 / 13.3 against 25.4 / 13.0, 16^2x20x32 31.2 / 14.4 against
+  // 30.9 / 14.8, 16^2x20x40 48.0 / 19.0 against 46.7 / 19.3, 20^3x40 66.2 /
+  // 23.2 against 64.0 / 23.3, 24^3x48 137.5 / 51.5 against 131.8 / 51.9.
+  const bool sadd = update && lat_->Vh <= 90112;
   if (update && !sadd) bs_launch_ru_x(mask, cap_, (int)lat_->Vh, x64_.slot(0), xs_.slot(0), 3 * lat_->Vh, st);
   a.src_add = xs_.data;
   ru_shape_.apply(a);
