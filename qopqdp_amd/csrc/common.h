@@ -218,7 +218,7 @@ struct LinkSet {
   int nl = 0;            // 16 with Naik, 8 without
   void *data = nullptr;  // [2][nl][9][Vh] complex
   float *scale = nullptr;  // FP16: [2][nl][Vh]
-  long sites = 0;          // Vh of the array, set by build_links64
+  long sites = 0;          // Vh of the FP64 array, set by links64_alloc
   const void *parity_data(const Lattice *lat, int p) const {
     return (const char *)data + (size_t)p * nl * 9 * lat->Vh * prec_cbytes(prec);
   }

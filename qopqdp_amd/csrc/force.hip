@@ -608,10 +608,14 @@ __global__ __launch_bounds__(TPB) void force_kernel(long V, double2 *F, const do
 // (the reference builds the outermost staple last, one path at a time): 15
 // staples per direction instead of 18, and three launches, each a pass over
 // the fields it needs once, instead of 18 that read and write the fat link.
-// Bytes per site and direction: (4 + 3) + (7 + 3) + (7 + 1) fields of 144 B
-// against 96; HBM-bound (3 flops per byte).
-// Measured per direction at 24^3x48: inner 209, middle 407, outer 198 us (L2 misses
-// at 6 TB/s), against nine staple passes of 117 us and nine of 99 us.
+// Fields of 144 B per site read + written per direction: (4 + 3) + (7 + 3) +
+// (7 + 1), where they were 96: 506 us at 24^3x48 at the rate of a copy, and the
+// FP64 products 145 us.  Measured per direction there: inner 208, middle 403,
+// outer 196 us, against nine staple passes of 117 us and nine of 99 us.  What
+// bounds them is the gathers that miss L2: 2.6, 3.7 and 1.4 times the fields are
+// read (0.98, 2.46, 0.97 GB), at 6.1, 6.8 and 5.4 TB/s with the stores.  The
+// links differ from a 64-bit restatement of the smearing by 2.2e-16 of their
+// norm, 1.6e-16 when the paths were added one at a time.
 template <bool HASE>
 __global__ __launch_bounds__(TPB, 1) void fat_inner_kernel(Geom g, Sched q, long V, Ptr4 U, MidPtr T, double c5, double c7,
                                                         int mu) {

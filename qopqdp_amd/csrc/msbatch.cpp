@@ -58,6 +58,9 @@ MultiShiftBatch::MultiShiftBatch(Links &L, int eo, int capacity, int sloppy_prec
     // while no slot is loaded)
     shape_ = tune_hop(L_, hp_, cap_, ps_, ts_, 1 - eo_, RED_OUT2);
     shape2_ = tune_hop(L_, hp_, cap_, ts_, rs_, eo_, RED_CG, &ps_, &xm_);
+    // the FP64 hop over flagged slots takes the shape of the plain FP64 hop on
+    // all slots (of it RHS per thread, block, remap, tile and staging apply); a
+    // sweep of its own with few flagged slots is not made
     ru_shape_ = tune_hop(L_, P64, cap_, x64_, t64_, 1 - eo_);
     sync();
   } catch (const DeviceOutOfMemory &) {

@@ -323,10 +323,10 @@ void invert_cgms(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg **r
 
 // ---------------------------------------------------------------------------
 // regular CG (lib/invert_cg_p.c:1-128), linop = ddagd.  The host runs the
-// (re)starts, where the residual is recomputed; the iterations between them run
-// on the device with the multi-shift CG's kernels at one shift, where they
-// took twelve launches and three host synchronisations each.  <p, A p> is
-// |D p|^2 + m^2 |p|^2, the value linop returns.
+// (re)starts, where the residual is recomputed.  The iterations between them run
+// on the device, as a multi-shift CG with one shift: five launches each, against
+// twelve and three host synchronisations when the host drove them.  <p, A p>
+// is |D p|^2 + m^2 |p|^2, the value linop returns.
 void invert_cg(Links &L, int prec, double mass, int eo, InvArg *ia, ResArg *ra,
                DevVec &out, const DevVec &in) {
   Lattice *lat = L.lat;
