@@ -234,24 +234,31 @@ struct Scratch {
   bool host = false;
   void *get(size_t bytes) {
     if (bytes <= n) return p;
-    if (p) {
-      QOP_CHECK_HIP(hipStreamSynchronize(stream()));
-      if (host) QOP_CHECK_HIP(hipHostFree(p)); else dev_free(p);
-    }
-    p = nullptr;
-    n = 0;
+    release();
     const size_t want = bytes < (1u << 20) ? (1u << 20) : bytes * 2;
     if (host) QOP_CHECK_HIP(hipHostMalloc(&p, want, hipHostMallocDefault));
     else dev_alloc(&p, want);
     n = want;
     return p;
   }
+  void release() {
+    if (!p) return;
+    QOP_CHECK_HIP(hipStreamSynchronize(stream()));
+    if (host) QOP_CHECK_HIP(hipHostFree(p)); else dev_free(p);
+    p = nullptr;
+    n = 0;
+  }
 };
-Scratch s_partial, s_result, s_host{nullptr, 0, true};
+// One per thread: a server's worker solves with the reference algorithm beside
+// the program's calls, and partials of one solve are summed by a later launch.
+thread_local Scratch s_partial, s_result, s_host{nullptr, 0, true};
 }  // namespace
 
 double *red_partial(size_t nd) { return (double *)s_partial.get(nd * sizeof(double)); }
 double *red_result(size_t nd) { return (double *)s_result.get(nd * sizeof(double)); }
 double *red_host(size_t nd) { return (double *)s_host.get(nd * sizeof(double)); }
+void red_release() {
+  for (Scratch *s : {&s_partial, &s_result, &s_host}) s->release();
+}
 
 }  // namespace qop

@@ -107,7 +107,10 @@ class Server {
     fr += dev_cache_bytes();  // given back when an allocation needs it
     reserve_ = std::min<size_t>((size_t)2 << 30, tot / 32);
     if (!budget_) budget_ = fr > reserve_ ? fr - reserve_ : 0;
-    worker_ = std::thread([this] { run(); });
+    worker_ = std::thread([this] {
+      run();
+      red_release();
+    });
   }
 
   ~Server() {

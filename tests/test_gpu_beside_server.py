@@ -83,3 +83,52 @@ def test_solves_beside_a_server_that_rebuilds_its_batches():
         s.lib.QOP_D3_destroy_G(g)
         s.close()
     assert not errors and asked[0] >= 4
+
+
+def test_solves_beside_a_server_of_the_reference_algorithm():
+    """A server of precision 64 solves on the library stream too: each thread's
+    reductions are its own."""
+    U = [q.gen_gauge(L, 7300 + k, 0.3) for k in range(2)]
+    src = q.gen_source(L, 7400, EVEN)
+    srv = q.Server(capacity=1, prec=64)
+    srv.add_gauge(L, U[0], MILC)
+
+    def ask():
+        out, st, res, _ = srv.wait(srv.submit(0, src, 0.1, 1e-9, EVEN))
+        assert st == 0
+        return out
+
+    want_srv = ask()
+    s = q.Session(L)
+    g = s.gauge(U[1])
+    fla, _ = s.links_from_gauge(g)
+    full = q.gen_source(L, 7500, EVENODD)
+    want = {eo: solve(s, fla, full, eo) for eo in (EVEN, EVENODD)}
+    errors, asked = [], [0]
+    stop = threading.Event()
+
+    def feed():
+        try:
+            while not stop.is_set():
+                if not np.array_equal(ask(), want_srv):
+                    errors.append(asked[0])
+                asked[0] += 1
+        except Exception as e:  # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    t = threading.Thread(target=feed)
+    t.start()
+    try:
+        for k in range(100):
+            eo = EVENODD if k % 2 else EVEN
+            assert np.array_equal(solve(s, fla, full, eo), want[eo]), k
+            if errors or (k >= 40 and asked[0] >= 20):
+                break
+    finally:
+        stop.set()
+        t.join()
+        srv.close()
+        s.lib.QOP_D3_asqtad_destroy_L(fla)
+        s.lib.QOP_D3_destroy_G(g)
+        s.close()
+    assert not errors and asked[0] >= 4
