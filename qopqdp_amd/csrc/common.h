@@ -250,12 +250,13 @@ struct Links {
 hipStream_t stream();  // library stream (default priority)
 void sync();
 
-// Reduction scratch of the calling thread: partial sums per 64-site chunk,
-// results in doubles.
+// Reduction scratch: partial sums per 64-site chunk, results in doubles.
 double *red_partial(size_t ndoubles);  // device, grows on demand
 double *red_result(size_t ndoubles);   // device
 double *red_host(size_t ndoubles);     // pinned host
-void red_release();                    // before a thread that used it ends
+// From begin to end the calling thread has reduction scratch of its own.
+void red_own_begin();
+void red_own_end();
 
 // Link preparation (links.hip)
 // the FP64 array of nl links per site for L.lat (kept when it already fits)

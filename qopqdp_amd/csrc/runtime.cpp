@@ -249,16 +249,25 @@ struct Scratch {
     n = 0;
   }
 };
-// One per thread: a server's worker solves with the reference algorithm beside
-// the program's calls, and partials of one solve are summed by a later launch.
-thread_local Scratch s_partial, s_result, s_host{nullptr, 0, true};
+struct ScratchSet {
+  Scratch partial, result, host{nullptr, 0, true};
+};
+// The program's calls share one set (they do not overlap); a server's worker,
+// which solves with the reference algorithm beside them, has one of its own:
+// partials of a solve are summed by a later launch.
+ScratchSet g_scratch;
+thread_local ScratchSet *t_scratch = &g_scratch;
 }  // namespace
 
-double *red_partial(size_t nd) { return (double *)s_partial.get(nd * sizeof(double)); }
-double *red_result(size_t nd) { return (double *)s_result.get(nd * sizeof(double)); }
-double *red_host(size_t nd) { return (double *)s_host.get(nd * sizeof(double)); }
-void red_release() {
-  for (Scratch *s : {&s_partial, &s_result, &s_host}) s->release();
+double *red_partial(size_t nd) { return (double *)t_scratch->partial.get(nd * sizeof(double)); }
+double *red_result(size_t nd) { return (double *)t_scratch->result.get(nd * sizeof(double)); }
+double *red_host(size_t nd) { return (double *)t_scratch->host.get(nd * sizeof(double)); }
+
+void red_own_begin() { t_scratch = new ScratchSet; }
+void red_own_end() {
+  for (Scratch *s : {&t_scratch->partial, &t_scratch->result, &t_scratch->host}) s->release();
+  delete t_scratch;
+  t_scratch = &g_scratch;
 }
 
 }  // namespace qop

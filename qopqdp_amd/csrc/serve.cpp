@@ -108,8 +108,9 @@ class Server {
     reserve_ = std::min<size_t>((size_t)2 << 30, tot / 32);
     if (!budget_) budget_ = fr > reserve_ ? fr - reserve_ : 0;
     worker_ = std::thread([this] {
+      red_own_begin();
       run();
-      red_release();
+      red_own_end();
     });
   }
 

@@ -86,7 +86,7 @@ def test_solves_beside_a_server_that_rebuilds_its_batches():
 
 
 def test_solves_beside_a_server_of_the_reference_algorithm():
-    """A server of precision 64 solves on the library stream too: each thread's
+    """A server of precision 64 solves on the library stream too: its worker's
     reductions are its own."""
     U = [q.gen_gauge(L, 7300 + k, 0.3) for k in range(2)]
     src = q.gen_source(L, 7400, EVEN)
