@@ -113,15 +113,11 @@ class BlockCache {
     for (Kept *k : {&ready, &pending})
       for (auto &b : *k) api_.free(b.second.p);
   }
-  // What an allocation of `bytes` takes: up to `block` whole units of 512
-  // bytes or of a power of two that is at most 1/16 of the size, above 16 MB
-  // at least whole 2 MB pages.  So nearby sizes share blocks, and none is more
-  // than 1/16 (1/8 from 16 to 32 MB), or 512 bytes, larger than asked for.
+  // What an allocation of `bytes` takes: whole units of 512 bytes.  Calls come
+  // back with the same sizes, so blocks need not serve nearby ones, and a
+  // caller's count of what it allocates holds.
   size_t size_of(size_t bytes) const {
-    size_t unit = 512;
-    while (unit * 32 <= bytes) unit *= 2;
-    if (bytes > ((size_t)16 << 20) && unit < ((size_t)2 << 20)) unit = (size_t)2 << 20;
-    const size_t n = bytes ? (bytes + unit - 1) / unit * unit : unit;
+    const size_t n = bytes ? (bytes + 511) / 512 * 512 : 512;
     return n <= block_ ? n : bytes;
   }
   size_t kept() {

@@ -68,8 +68,7 @@ inline void host_alloc(T **p, size_t bytes) {
 void host_free(void *p);
 void cache_trim();         // kept blocks go back to the driver
 size_t dev_cache_bytes();  // device memory held in kept blocks
-size_t dev_block_bytes(size_t bytes);  // what dev_alloc takes for a request
-bool dev_block_kept(size_t bytes);     // is it a size the cache keeps
+bool dev_block_kept(size_t bytes);  // is it a size the cache keeps
 // Owning device buffer for temporaries: freed when it goes out of scope,
 // also while a DeviceOutOfMemory unwinds.
 template <class T>

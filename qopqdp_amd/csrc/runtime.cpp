@@ -78,8 +78,7 @@ void cache_trim() {
   host_cache().trim();
 }
 size_t dev_cache_bytes() { return dev_cache().kept(); }
-size_t dev_block_bytes(size_t bytes) { return dev_cache().size_of(bytes); }
-bool dev_block_kept(size_t bytes) { return dev_block_bytes(bytes) <= CACHE_BLOCK; }
+bool dev_block_kept(size_t bytes) { return dev_cache().size_of(bytes) <= CACHE_BLOCK; }
 
 static std::mutex g_mu;
 

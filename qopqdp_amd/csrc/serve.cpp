@@ -76,24 +76,21 @@ struct Engine {
   double last_used = 0;
 };
 
-// Device memory of a link set and of an engine, block by block as they are
-// allocated.
 size_t link_bytes(const Lattice *lat, int prec) {
   const size_t n = (size_t)2 * 16 * 9 * lat->Vh;
-  const size_t scale = prec == P16 ? dev_block_bytes((size_t)2 * 16 * lat->Vh * sizeof(float)) : 0;
-  return dev_block_bytes(n * prec_cbytes(prec)) + scale;
+  if (prec == P64) return n * 16;
+  if (prec == P32) return n * 8;
+  return n * 4 + (size_t)2 * 16 * lat->Vh * sizeof(float);
 }
 
 size_t engine_bytes(const Lattice *lat, int cap, int prec) {
-  const size_t vh = lat->Vh, nch = (vh + 63) / 64, n = cap;
-  auto vectors = [&](size_t count, int p) { return dev_block_bytes(count * 3 * vh * prec_cbytes(p)); };
-  size_t bytes = 2 * vectors(2, P64);  // stage, raw
-  if (prec != P64) {  // the vectors of BatchSolver, norms, reduction partials
-    bytes += 5 * vectors(n, P64) + 3 * vectors(n, prec) + vectors(n, P32);
-    if (prec == P16) bytes += 3 * dev_block_bytes(n * vh * sizeof(float));
-    bytes += dev_block_bytes(3 * n * nch * sizeof(double));
-  }
-  return bytes + (1u << 20);  // masks, scalars
+  const size_t vh = lat->Vh;
+  const size_t fp64 = 48 * vh;                                  // one parity, FP64
+  const size_t sl = prec == P16 ? 12 * vh + 4 * vh : 24 * vh;   // one parity, sloppy
+  const size_t nch = (vh + 63) / 64;
+  size_t per_slot = 5 * fp64 + 3 * sl + 24 * vh + 3 * nch * sizeof(double) + 256;
+  if (prec == P64) per_slot = 0;
+  return (size_t)cap * per_slot + 2 * fp64 /* stage */ + 2 * fp64 /* raw */ + (1u << 20);
 }
 
 }  // namespace

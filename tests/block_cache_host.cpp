@@ -145,26 +145,27 @@ static void nobody_waits_behind_a_free() {
   }
 }
 
-// A block is at most 1/16, 512 bytes or, above 16 MB, 2 MB larger than asked
-// for; a kept block serves only requests of its size.
+// A block is less than 512 bytes larger than asked for; a kept block serves
+// only requests of its size.
 static void blocks_are_little_larger_than_asked() {
   Device d;
   Cache c(Memory{&d}, 384 << 20, (size_t)8 << 30);
-  for (size_t n = 0; n < ((size_t)300 << 20); n = n * 9 / 8 + 37)
-    for (size_t m : {n, n + 1, (n & (n - 1)) ? n : n + 3}) {
+  for (size_t n = 0; n < ((size_t)500 << 20); n = n * 9 / 8 + 37)
+    for (size_t m : {n, n + 1, n / 512 * 512}) {
       const size_t s = c.size_of(m);
-      const size_t least = m > ((size_t)16 << 20) ? (size_t)2 << 20 : 512;
-      CHECK(s >= m && s > 0 && s % 512 == 0 && s - m <= (m / 16 > least ? m / 16 : least));
+      CHECK(s >= m && s > 0 && (s < m + 512 || m == 0));
+      CHECK(m > ((size_t)384 << 20) ? s == m : s % 512 == 0);
       CHECK(c.size_of(s) == s);
     }
-  CHECK(c.size_of((size_t)257 << 20) <= (size_t)273 << 20);
-  CHECK(c.size_of((size_t)400 << 20) == (size_t)400 << 20);
   void *a = c.alloc(64 << 10);
   c.free(a);
   CHECK(c.kept() == 64 << 10);
-  void *b = c.alloc(60 << 10);  // a size class below
+  void *b = c.alloc(60 << 10);
   CHECK(b != a);
+  void *e = c.alloc((64 << 10) - 100);
+  CHECK(e == a);
   c.free(b);
+  c.free(e);
   c.trim();
 }
 
